@@ -317,6 +317,72 @@ int32_t prh_etd2_steps_noalloc(const prh_operator* op, const prh_schedule* sch, 
 int32_t prh_etd2_stage(const prh_operator* op, const prh_schedule* sch, const prh_state* st,
                        int32_t step, int32_t stage, void* stream);
 
+/* Plan of a team march (prh_team_march): nteam teams of `size` workgroups of 16
+ * waves.  Team t marches the right-hand sides of its share of [0, K) (K / nteam,
+ * the first K % nteam teams one more) through every step.  Ranks 0 .. ndwg - 1 of
+ * a team sum the dense rows over heavy mothers, the next nfwg finish the tail
+ * rows one stage behind, the others own the heavy rows; no heavy row may read a
+ * tail row.
+ *   lds_ptr  [size + 1]: range of lds_voff that belongs to a rank; lds_voff:
+ *            value offset (inside a window) of each 64-double LDS slot.
+ *   wave_ptr [size * 16 + 1]: tasks of each wave (pair_rows: the two waves 2 i and
+ *            2 i + 1 of a rank list the same tasks and share their columns);
+ *            rows [ntasks][10] = {row a, row b or -1, entries of both rows, of row
+ *            a, of row b (<= 64 in all), slots of the two rows' diagonals of M,
+ *            partials of the two rows or -1, first entry}; mothers [][2] =
+ *            {mother species, slot of its block (both rows: row a's, row b's in
+ *            the next slot)}, all blocks diagonal.  A partial >= 0 marks a tail
+ *            row's sum over heavy mothers, stored as that partial instead of a
+ *            finished row.  Without pair_rows every task is one row, with at
+ *            most 2 right-hand sides per team.
+ *   dense_ptr [ndwg * dgroups + 1]: entries of each mother group (at most 64);
+ *            dense_ent [][5] = {mother, slot, o_lo | nslot << 8} with slot and
+ *            band repeated for the second dense row (nslot 0: no block; 0 <=
+ *            o_lo, nslot <= 8, second row nslot <= 1).  The 16 waves form dgroups mother groups x 16 /
+ *            dgroups column groups of kd pairs; rank g's sum of dense
+ *            row r is partial 2 g + r.
+ *   fin      [nfin][8] = {row, diagonal's slot, first partial, stride, partials,
+ *            first block, blocks, 0}; fin_blk [][4] = {mother, slot, o_lo, nslot},
+ *            blocks from tail mothers.
+ * Device memory of the caller: sync, PRH_TEAM_SYNC_BYTES; dpart,
+ * [2][nparts][K][64] doubles. */
+#define PRH_TEAM_SYNC_BYTES 18688
+typedef struct prh_team {
+  int32_t nteam;
+  int32_t size;
+  int32_t kp;        /* pairs of right-hand sides per pass of a wave: 1 or 2 */
+  int32_t kd;        /* pairs of right-hand sides per dense-row wave: 1 or 2 */
+  int32_t dgroups;   /* mother groups per dense-row workgroup */
+  int32_t ndwg;
+  int32_t nfwg;
+  int32_t nfin;
+  int32_t nparts;
+  int32_t lds_slots; /* slots of the largest rank, finishing ranks counted twice */
+  int32_t red_slots; /* LDS rows of the mother groups' partial sums */
+  int32_t pair_rows; /* tasks hold row pairs */
+  const int32_t* lds_ptr;
+  const int32_t* lds_voff;
+  const int32_t* wave_ptr;
+  const int32_t* rows;
+  const int32_t* mothers;
+  const int32_t* dense_ptr;
+  const int32_t* dense_ent;
+  const int32_t* fin;
+  const int32_t* fin_blk;
+  double* dpart;
+  uint32_t* sync;
+} prh_team;
+
+/* ETD2 steps k_begin <= k < k_end in one cooperative launch: the steps of
+ * prh_etd2_steps (d = 64, no EM sector; recording as there) for operators whose
+ * rows are diagonal blocks except at most two dense rows.  op->tasks and
+ * op->blocks are not used.  The launch needs nteam * size CUs with
+ * 8 * 64 * (11 + red_slots + lds_slots) bytes of LDS each (two fields: 13 and
+ * twice lds_slots).  Returns 2 (nothing launched) when the device cannot hold
+ * that grid or the stream is capturing. */
+int32_t prh_team_march(const prh_operator* op, const prh_schedule* sch, const prh_state* st,
+                       const prh_team* tm, int32_t k_begin, int32_t k_end, void* stream);
+
 /* Adjoint of ETD2 step `step` (two transposed stage kernels).  opT is the
  * operator in transposed block layout with the transposed FD stencil.  No
  * counterpart in the reference (which has no adjoint); it is the reverse of

@@ -36,11 +36,15 @@ EXPORTED = (
     "prh_toeplitz_rows",
     "prh_em_transfer_stack",
     "prh_em_step_transfer",
+    "prh_team_march",
 )
 
 WG_WAVES = 16
 #: size of the static device scratch of prh_etd2_steps_noalloc (PRH_SCRATCH_BYTES)
 SCRATCH_BYTES = 64 << 20
+
+#: prh_team_march status: this launch cannot run here (the stage kernels can)
+NOT_LAUNCHABLE = 2
 
 PRH_F_PARTIAL_DIFF = 1
 PRH_F_INJECTION = 2
@@ -238,6 +242,34 @@ class PrhCascade(ctypes.Structure):
     ]
 
 
+class PrhTeam(ctypes.Structure):
+    _fields_ = [
+        ("nteam", _i32),
+        ("size", _i32),
+        ("kp", _i32),
+        ("kd", _i32),
+        ("dgroups", _i32),
+        ("ndwg", _i32),
+        ("nfwg", _i32),
+        ("nfin", _i32),
+        ("nparts", _i32),
+        ("lds_slots", _i32),
+        ("red_slots", _i32),
+        ("pair_rows", _i32),
+        ("lds_ptr", _p),
+        ("lds_voff", _p),
+        ("wave_ptr", _p),
+        ("rows", _p),
+        ("mothers", _p),
+        ("dense_ptr", _p),
+        ("dense_ent", _p),
+        ("fin", _p),
+        ("fin_blk", _p),
+        ("dpart", _p),
+        ("sync", _p),
+    ]
+
+
 def load():
     """Load (once) and return the ctypes library handle."""
     global _LIB
@@ -265,6 +297,16 @@ def load():
         ctypes.POINTER(PrhOperator),
         ctypes.POINTER(PrhSchedule),
         ctypes.POINTER(PrhState),
+        _i32,
+        _i32,
+        _p,
+    ]
+    lib.prh_team_march.restype = _i32
+    lib.prh_team_march.argtypes = [
+        ctypes.POINTER(PrhOperator),
+        ctypes.POINTER(PrhSchedule),
+        ctypes.POINTER(PrhState),
+        ctypes.POINTER(PrhTeam),
         _i32,
         _i32,
         _p,

@@ -10,10 +10,12 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
-SRC = os.path.join(HERE, "csrc", "prince_hip.hip")
+CSRC = os.path.join(HERE, "csrc")
+SOURCES = [os.path.join(CSRC, f) for f in ("prince_hip.hip", "team_march.hip")]
 OUT = os.path.join(HERE, "libprince_hip.so")
 
 HIPCC_FLAGS = [
@@ -21,13 +23,16 @@ HIPCC_FLAGS = [
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     "-Xclang",
     "-target-feature",
     "-Xclang",
     "-packed-fp32-ops",
     "-I" + os.path.join(ROOT, "include"),
 ]
+
+# the march holds its state in 128 registers: constants of exp() and the like
+# hoisted out of its step loop would spill (26 registers of scratch per wave)
+SOURCE_FLAGS = {"team_march.hip": ["-mllvm", "-disable-machine-licm"]}
 
 
 def hipcc():
@@ -38,15 +43,28 @@ def hipcc():
 
 
 def build(verbose=False):
-    tmp = OUT + ".tmp"
-    cmd = [hipcc(), *HIPCC_FLAGS, "-o", tmp, SRC]
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        sys.stderr.write(res.stdout + res.stderr)
-        raise RuntimeError("hipcc failed building libprince_hip.so")
-    if verbose:
-        sys.stdout.write(res.stdout)
-    os.replace(tmp, OUT)
+    """Compile every source (in parallel) and link the shared library."""
+    cc = hipcc()
+    with tempfile.TemporaryDirectory() as tmpdir:
+        objs = [os.path.join(tmpdir, os.path.basename(s) + ".o") for s in SOURCES]
+        procs = [subprocess.Popen([cc, *HIPCC_FLAGS,
+                                   *SOURCE_FLAGS.get(os.path.basename(s), []), "-c", "-o", o, s], stdout=subprocess.PIPE,
+                                  stderr=subprocess.STDOUT, text=True)
+                 for s, o in zip(SOURCES, objs)]
+        outs = [p.communicate()[0] for p in procs]
+        tmp = OUT + ".tmp"
+        ok = all(p.returncode == 0 for p in procs)
+        if ok:
+            res = subprocess.run([cc, "--offload-arch=gfx950", "-shared", "-o", tmp, *objs],
+                                 capture_output=True, text=True)
+            outs.append(res.stdout + res.stderr)
+            ok = res.returncode == 0
+        if not ok:
+            sys.stderr.write("".join(outs))
+            raise RuntimeError("hipcc failed building libprince_hip.so")
+        if verbose:
+            sys.stdout.write("".join(outs))
+        os.replace(tmp, OUT)
     return OUT
 
 

@@ -1,0 +1,1236 @@
+// team_march.hip -- the whole redshift march of a shared-schedule batch in one
+// cooperative launch (gfx950).
+//
+// What bounds the march when every stage is its own kernel: a stage moves
+// 3 MB of coupling values and the state, about 1 us of traffic for one
+// right-hand side, but costs two launches and their dependency gaps (11.9 us
+// per stage at K = 1, 33 us at K = 64), and it reads the same coupling values
+// again in each of the ~20 stages of a refresh window.  Here the chip is cut
+// into teams of workgroups, one workgroup per CU; a team owns a share of the
+// right-hand sides for the whole march (columns never exchange data), and a
+// workgroup of it owns species rows whose coupling values of the current
+// window stay in its LDS (93 KB per CU for the A <= 56 run on a 32-CU team).
+// Between stages only the state crosses workgroups: x and a are stored and
+// loaded with agent-scope cache policy (sc1), so no cache write-back or
+// invalidation is needed, and a team barrier costs 1.5 us (32 workgroups of
+// one XCD) to 2.6 us (256).  A full agent-scope release / acquire pair instead
+// measured 37 us per stage: it writes back and invalidates the whole L2.
+// Measured per stage of the A <= 56 run, stage kernels -> march: K = 1 11.6 ->
+// 6.3 us, K = 7 19.9 -> 6.6, K = 64 33 -> 17, K = 300 129 -> 45, K = 512 92 -> 82;
+// two fields, K = 48: 48 -> 21.
+//
+// Teams are workgroups blockIdx % nteam, which the dispatcher places on one
+// XCD (nteam = 8) or on a pair of XCDs (nteam = 4); only speed depends on that
+// placement, the sc1 accesses are coherent over the whole device.
+//
+// Dense rows (protons: one band block from almost every species; He-4: one
+// diagonal block from almost every species) would be one workgroup's serial
+// chain.  No nucleus feeds a heavier one, so the heavy rows never read the
+// dense rows or the few light rows that read those ("tail" rows), and the tail
+// runs one phase behind: in the phase of stage p the heavy rows do stage p,
+// `ndwg` workgroups sum the dense rows' blocks over the heavy mothers (shared
+// out by mothers, a mother panel loaded once for both rows), and `nfwg`
+// workgroups finish the tail rows of stage p - 1 from the partials of the
+// phase before.  One barrier per stage then orders everything; finishing the
+// dense rows inside the stage behind a second barrier measured 7.0 us per stage
+// at K = 1.
+//
+// Lanes: a wave holds two right-hand sides, 32 lanes each, two energy bins per
+// lane, so every state and value access is 16 bytes per lane.  8-byte loads of
+// the same panels stop at 18.8 TB/s over the chip (half of a CU's load path),
+// 16-byte ones reach 32 TB/s, with or without sc1; a shift by one bin also
+// moves half as many registers.
+//
+// Every wait is bounded: a workgroup that polls SPIN_LIMIT times without
+// progress raises the abort word, all workgroups leave, and the state is
+// filled with NaN.
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <mutex>
+#include <string>
+#include <type_traits>
+
+#include "../../include/prince_hip.h"
+#include "internal.h"
+
+namespace {
+
+#include "stage_math.h"
+
+constexpr int TWAVES = 16;  // waves per workgroup (128 registers each)
+constexpr int TTHREADS = TWAVES * WAVE;
+constexpr int TDENSE = 2;   // dense rows per operator
+constexpr int TCONST = 9;   // LDS rows: 7 FD coefficients, energy grid, FD diagonal
+constexpr int SC1 = 16;     // buffer cache policy: agent scope
+constexpr int SPIN_LIMIT = 1 << 25;
+// sync words (32-bit) of prh_team::sync: per team, 64 words apart
+constexpr int SY_SUB = 0;       // [8 teams][8 sub-groups] arrival counters
+constexpr int SY_ROOT = 4096;   // [8 teams] arrivals of complete sub-groups
+constexpr int SY_ABORT = 4608;
+constexpr int SY_WORDS = 4672;
+
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef double d2 __attribute__((ext_vector_type(2)));  // bins 2 l, 2 l + 1 of lane l of a half
+
+// state access: agent scope for x, a and the partials, plain for F(x) (read back
+// by the wave that wrote it)
+template <int POLICY>
+__device__ __forceinline__ d2 pload(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  return __builtin_bit_cast(d2, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, POLICY));
+}
+template <int POLICY>
+__device__ __forceinline__ void pstore(d2 v, __amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, voff, soff, POLICY);
+}
+
+// The arguments stay in the kernel's argument segment and are read from there,
+// phase by phase, through the scalar cache: as ordinary by-value arguments the
+// compiler keeps some 60 pointers in registers over the whole march and spills
+// (300 register moves to and from lanes of vector registers per phase).
+struct TeamArgs {
+  prh_operator op;
+  prh_schedule sch;
+  prh_state st;
+  prh_team tm;
+  int k_begin, k_end;
+};
+#define CONST_SPACE const __attribute__((address_space(4)))
+typedef CONST_SPACE TeamArgs CArgs;
+typedef CONST_SPACE prh_operator COp;
+typedef CONST_SPACE prh_schedule CSch;
+typedef CONST_SPACE prh_state CSt;
+typedef CONST_SPACE prh_team CTm;
+// the same pointer, as far as the compiler knows another one: what was read
+// through it before is read again
+__device__ __forceinline__ CArgs* reread(CArgs* a) {
+  asm volatile("" : "+s"(a));
+  return a;
+}
+
+// Read-only tables at wave-uniform indices: constant-space loads go through the
+// scalar cache, where a plain load becomes a vector load (the compiler cannot
+// rule out that the march's stores change them) and a 0.3 us wait in a chain.
+template <typename V>
+__device__ __forceinline__ V cload(const V* p) {
+  return *reinterpret_cast<CONST_SPACE V*>(reinterpret_cast<uintptr_t>(p));
+}
+
+// This lane's place in the wave.
+struct Lane {
+  int id;           // 0 .. 63
+  int half;         // right-hand side of the pair
+  int bin;          // first of its two bins
+  int off;          // byte offset of its bins in the pair's [2][64] panel
+  bool first, last; // bins 0, 1 / 62, 63
+  bool edge0, edge1;  // bins below 4 / above 59
+};
+__device__ __forceinline__ Lane lane_of() {
+  Lane n;
+  n.id = threadIdx.x & (WAVE - 1);
+  n.half = n.id >> 5;
+  n.bin = 2 * (n.id & 31);
+  n.off = n.id * 16;
+  n.first = n.bin == 0;
+  n.last = n.bin == 62;
+  n.edge0 = n.bin < 4;
+  n.edge1 = n.bin > 59;
+  return n;
+}
+
+// Lane shifts inside a half: the neighbour lane's value, zero past the ends (the
+// other half is another right-hand side).
+__device__ __forceinline__ double prev1(const Lane& n, double v) {
+  const double r = lane_prev(v);
+  return n.first ? 0.0 : r;
+}
+__device__ __forceinline__ double next1(const Lane& n, double v) {
+  const double r = lane_next(v);
+  return n.last ? 0.0 : r;
+}
+// the panel moved down by one bin: bin i receives bin i + 1
+__device__ __forceinline__ d2 shift_bin(const Lane& n, d2 v) {
+  const double t = next1(n, v.x);
+  return d2{v.y, t};
+}
+
+struct TeamLds {
+  double* cst;  // [9][64]
+  double* rp;   // [2][fields][64] pair-production rate of the window
+  double* red;  // [16 waves][2][64 lanes][2] partial sums of the dense rows' mother groups
+  double* val;  // [fields][slots][64] coupling values of the window (finishing
+                // workgroups: two such sets, they also need the window before)
+  int slots;
+};
+__device__ __forceinline__ d2 lds2(const double* base, int slot, int bin) {
+  return *reinterpret_cast<const d2*>(base + slot * WAVE + bin);
+}
+
+struct StepIn {
+  int step, ridx;  // ridx: slot of the record arrays, -1 when not recorded
+  double dl, h, hadia, finj;
+};
+// Per row: pair-production scale and source slot (-1: none).
+struct RowConst {
+  double pscale;
+  int sslot;
+};
+__device__ __forceinline__ RowConst row_const(COp& op, int da) {
+  return RowConst{cload(op.pscale + da),
+                  (op.flags & PRH_F_INJECTION) ? cload(op.src_slot + da) : -1};
+}
+
+// The state arrays as buffers over their whole [nspec][K][64] extent (one
+// descriptor each): row, column and panel offsets are scalar byte offsets.
+struct TeamState {
+  __amdgpu_buffer_rsrc_t x, a, f;
+  __amdgpu_buffer_rsrc_t part;  // [2 stages][nparts][K][64] partial sums of the tail rows
+  int pb;                       // bytes of one species' [K][64] panel
+  int phalf;                    // bytes of one stage's partials
+};
+
+// Source sums sum_j norm evolution(z) g_j of source slot sslot for the pairs from k0.
+template <int KP>
+__device__ __forceinline__ void team_source(COp& op, CSch& sch,
+                                            int step, int sslot, int k0, int kend, const Lane& n,
+                                            d2 (&src)[KP]) {
+  if (sslot < 0) return;
+  const int J = op.nsrc, K = op.K;
+  for (int j = 0; j < J; ++j) {
+    d2 g[KP];
+    double c[KP];
+#pragma unroll
+    for (int p = 0; p < KP; ++p) {
+      const int kk = k0 + 2 * p + n.half;
+      const int k = kk < kend ? kk : kend - 1;
+      g[p] = *reinterpret_cast<const d2*>(op.src_grid +
+                                          (((int64_t)sslot * J + j) * K + k) * WAVE + n.bin);
+      c[p] = sch.src_coef[((int64_t)step * J + j) * K + k];
+    }
+#pragma unroll
+    for (int p = 0; p < KP; ++p) src[p] = (j == 0) ? c[p] * g[p] : src[p] + c[p] * g[p];
+  }
+}
+
+// Diagonal factors of one bin in stage s2 (propagation.py:1389-1422,
+// etd2.py:329-390).
+__device__ __forceinline__ void bin_factors(int s2, double kadia, double pscale, double rate,
+                                            double mdiag, double ddiag, double dl, double h,
+                                            bool pdiff, double& kap, double& e, double& phi) {
+  kap = kadia + pscale * rate;
+  double dval = mdiag * dl;
+  if (pdiff) {
+    double kxd = kap * ddiag;
+    kxd = kxd * dl;
+    dval = dval + kxd;
+  }
+  const double hd = dval * h;
+  e = exp(hd);
+  phi = s2 ? phi2_of(hd, e) : phi1_of(hd, e);
+}
+
+// Factors of a row for one pair of right-hand sides.  One-field operators have the
+// same for every pair: computed once, each half of the wave one of the two bins
+// (half the exponentials), then exchanged.
+struct RowFactors {
+  d2 kap, e, phi;
+};
+__device__ __forceinline__ d2 from_halves(const Lane& n, double v) {
+  const double o = __shfl_xor(v, 32, WAVE);
+  return n.half ? d2{o, v} : d2{v, o};
+}
+template <bool TWO>
+__device__ __forceinline__ RowFactors row_factors(COp& op, const TeamLds& L,
+                                                  const StepIn& si, int s2, double pscale, int slot,
+                                                  int k, const Lane& n) {
+  const bool pdiff = (op.flags & PRH_F_PARTIAL_DIFF) != 0;
+  RowFactors f;
+  if constexpr (!TWO) {
+    const int bin = n.bin + n.half;
+    double kap, e, phi;
+    bin_factors(s2, si.hadia * L.cst[7 * WAVE + bin], pscale, L.rp[bin], L.val[slot * WAVE + bin],
+                L.cst[8 * WAVE + bin], si.dl, si.h, pdiff, kap, e, phi);
+    f.kap = from_halves(n, kap);
+    f.e = from_halves(n, e);
+    f.phi = from_halves(n, phi);
+  } else {
+    const double s = op.escale[k];
+#pragma unroll 1
+    for (int i = 0; i < 2; ++i) {
+      const int bin = n.bin + i;
+      double kap, e, phi;
+      bin_factors(s2, si.hadia * L.cst[7 * WAVE + bin], pscale, L.rp[bin] + s * L.rp[WAVE + bin],
+                  L.val[slot * WAVE + bin] + s * L.val[(L.slots + slot) * WAVE + bin],
+                  L.cst[8 * WAVE + bin], si.dl, si.h, pdiff, kap, e, phi);
+      if (i == 0) {
+        f.kap.x = kap;
+        f.e.x = e;
+        f.phi.x = phi;
+      } else {
+        f.kap.y = kap;
+        f.e.y = e;
+        f.phi.y = phi;
+      }
+    }
+  }
+  return f;
+}
+
+// Epilogue of row da for the pairs of right-hand sides from k0 (below kend): the
+// same expressions per bin as the per-stage kernels' epilogue.
+template <int KP, bool TWO, bool REC>
+__device__ __forceinline__ void team_epilogue(COp& op, CSt& st,
+                                              const TeamState& T, const TeamLds& L,
+                                              const StepIn& si, int s2, const RowFactors& f0,
+                                              const RowConst& rc, int da, int slot, int k0,
+                                              int kend, const Lane& n, const d2 (&acc)[KP],
+                                              const d2 (&xo)[KP], const d2 (&fo)[KP],
+                                              const d2 (&src)[KP]) {
+  const bool pdiff = (op.flags & PRH_F_PARTIAL_DIFF) != 0;
+#pragma unroll
+  for (int p = 0; p < KP; ++p) {
+    const int kp = k0 + 2 * p;
+    if (kp >= kend) break;  // uniform over the wave
+    const int k = kp + n.half;
+    RowFactors f = f0;
+    if (TWO) f = row_factors<true>(op, L, si, s2, rc.pscale, slot, k < kend ? k : kend - 1, n);
+    d2 out = acc[p];
+    if (pdiff) {
+      const d2 kx = f.kap * xo[p];
+      // stencil neighbours of bins 2 l and 2 l + 1, added in the order -3 .. 3
+      const double m1 = prev1(n, kx.y);  // bin 2 l - 1
+      const double m2 = prev1(n, kx.x);  // bin 2 l - 2
+      const double m3 = prev1(n, m1);    // bin 2 l - 3
+      const double q2 = next1(n, kx.x);  // bin 2 l + 2
+      const double q3 = next1(n, kx.y);  // bin 2 l + 3
+      const double q4 = next1(n, q2);    // bin 2 l + 4
+      d2 dx = {0.0, 0.0};
+      dx += lds2(L.cst, 0, n.bin) * d2{m3, m2};
+      dx += lds2(L.cst, 1, n.bin) * d2{m2, m1};
+      dx += lds2(L.cst, 2, n.bin) * d2{m1, kx.x};
+      dx += lds2(L.cst, 4, n.bin) * d2{kx.y, q2};
+      dx += lds2(L.cst, 5, n.bin) * d2{q2, q3};
+      dx += lds2(L.cst, 6, n.bin) * d2{q3, q4};
+      out = out + dx;
+    }
+    out = out * si.dl;
+    if (rc.sslot >= 0) out = out + si.finj * src[p];
+    if (k >= kend) continue;  // the odd last right-hand side's idle half
+    const int co = da * T.pb + kp * (WAVE * 8);
+    const int64_t nk = (int64_t)op.nspec * op.K * WAVE;
+    const int64_t rec = REC ? si.ridx * nk + ((int64_t)da * op.K + k) * WAVE + n.bin : 0;
+    if (s2 == 0) {
+      d2 a = f.e * xo[p];
+      d2 sc = f.phi * out;
+      sc = sc * si.h;
+      a = a + sc;
+      pstore<SC1>(a, T.a, n.off, co);
+      pstore<0>(out, T.f, n.off, co);
+      if (REC && si.ridx >= 0) {
+        *reinterpret_cast<d2*>(st.rec_x + rec) = xo[p];
+        *reinterpret_cast<d2*>(st.rec_a + rec) = a;
+        *reinterpret_cast<d2*>(st.rec_fx + rec) = out;
+      }
+    } else {
+      d2 sc = out - fo[p];
+      sc = sc * si.h;
+      sc = sc * f.phi;
+      pstore<SC1>(xo[p] + sc, T.x, n.off, co);
+      if (REC && si.ridx >= 0) *reinterpret_cast<d2*>(st.rec_fa + rec) = out;
+    }
+  }
+}
+
+// A wave's rows: row a, or two rows a and b (b < 0: none) read with one walk over
+// their mothers, so that a panel both rows read is loaded once (1.4 blocks per
+// panel on the A <= 56 run).  Lane e holds entry e (mother, LDS slot of the block):
+// first the n2 mothers of both rows (slot: row a's block, slot + 1 row b's), then
+// na of row a alone, then nb of row b alone.  part >= 0: a tail row whose coupling
+// sum over the heavy mothers goes to the partial buffer at that byte offset.
+struct RowTask {
+  int a, b, n2, na, nb, diag_a, diag_b, part_a, part_b;
+  RowConst ca, cb;
+  int mo, sl;  // lane entries
+};
+
+// Own state (and, in stage 2, F(x)) of row da for the pairs from k0.
+template <int KP>
+__device__ __forceinline__ void own_loads(const TeamState& T, int s2, int da, int k0, const Lane& n,
+                                          d2 (&xo)[KP], d2 (&fo)[KP]) {
+  const auto y = s2 ? T.a : T.x;
+#pragma unroll
+  for (int p = 0; p < KP; ++p) {
+    const int so = da * T.pb + (k0 + 2 * p) * (WAVE * 8);
+    xo[p] = pload<SC1>(y, n.off, so);
+    fo[p] = pload<0>(T.f, n.off, so);  // stage 1 does not use it
+  }
+}
+
+// Coupling of U entries from e on: both rows' blocks (BOTH) or those of one row.
+// Straight-line: U x KP panel loads, the values from LDS, then the products.
+template <int U, int KP, bool TWO, bool BOTH>
+__device__ __forceinline__ void couple_chunk(const TeamState& T, const TeamLds& L,
+                                             __amdgpu_buffer_rsrc_t y, const RowTask& rt, int e,
+                                             int cb, const Lane& n, d2 (&accA)[KP], d2 (&accB)[KP],
+                                             d2 (&accAE)[KP], d2 (&accBE)[KP]) {
+  d2 xv[U][KP], ma[U], mb[U], mae[U], mbe[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int po = __builtin_amdgcn_readlane(rt.mo, e + u) * T.pb + cb;
+#pragma unroll
+    for (int p = 0; p < KP; ++p) xv[u][p] = pload<SC1>(y, n.off, po + p * (2 * WAVE * 8));
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int sl = __builtin_amdgcn_readlane(rt.sl, e + u);
+    ma[u] = lds2(L.val, sl, n.bin);
+    if (BOTH) mb[u] = lds2(L.val, sl + 1, n.bin);
+    if (TWO) {
+      mae[u] = lds2(L.val, L.slots + sl, n.bin);
+      if (BOTH) mbe[u] = lds2(L.val, L.slots + sl + 1, n.bin);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+#pragma unroll
+    for (int p = 0; p < KP; ++p) {
+      accA[p] += ma[u] * xv[u][p];
+      if (BOTH) accB[p] += mb[u] * xv[u][p];
+      if (TWO) {
+        accAE[p] += mae[u] * xv[u][p];
+        if (BOTH) accBE[p] += mbe[u] * xv[u][p];
+      }
+    }
+  }
+}
+// Entries [e, e + m): chunks of U, then what is left in powers of two.
+template <int U, int KP, bool TWO, bool BOTH>
+__device__ __forceinline__ void couple_run(const TeamState& T, const TeamLds& L,
+                                           __amdgpu_buffer_rsrc_t y, const RowTask& rt, int e, int m,
+                                           int cb, const Lane& n, d2 (&accA)[KP], d2 (&accB)[KP],
+                                           d2 (&accAE)[KP], d2 (&accBE)[KP]) {
+#pragma unroll 1
+  for (; m >= U; m -= U, e += U)
+    couple_chunk<U, KP, TWO, BOTH>(T, L, y, rt, e, cb, n, accA, accB, accAE, accBE);
+  if (U > 2 && (m & 2)) {
+    couple_chunk<2, KP, TWO, BOTH>(T, L, y, rt, e, cb, n, accA, accB, accAE, accBE);
+    e += 2;
+  }
+  if (m & 1) couple_chunk<1, KP, TWO, BOTH>(T, L, y, rt, e, cb, n, accA, accB, accAE, accBE);
+}
+
+// One stage of a row task for the KP pairs of right-hand sides from k0.  Pairs
+// past kend read other panels (or zeros past the array) and are not stored.
+template <int KP, bool TWO, bool REC>
+__device__ __forceinline__ void team_rows(COp& op, CSch& sch,
+                                          CSt& st, const TeamState& T,
+                                          const TeamLds& L, const StepIn& si, int s2,
+                                          const RowTask& rt, const RowFactors& fa,
+                                          const RowFactors& fb, int k0, int kend, const Lane& n) {
+  constexpr int U = 4;
+  const auto y = s2 ? T.a : T.x;
+  d2 acc[2][KP], accE[2][KP], xo[KP], fo[KP];
+#pragma unroll
+  for (int p = 0; p < KP; ++p)
+    acc[0][p] = acc[1][p] = accE[0][p] = accE[1][p] = d2{0.0, 0.0};
+  const int cb = k0 * (WAVE * 8);
+  couple_run<U, KP, TWO, true>(T, L, y, rt, 0, rt.n2, cb, n, acc[0], acc[1], accE[0], accE[1]);
+  couple_run<U, KP, TWO, false>(T, L, y, rt, rt.n2, rt.na, cb, n, acc[0], acc[0], accE[0], accE[0]);
+  couple_run<U, KP, TWO, false>(T, L, y, rt, rt.n2 + rt.na, rt.nb, cb, n, acc[1], acc[1], accE[1],
+                                accE[1]);
+  if (TWO) {
+#pragma unroll
+    for (int p = 0; p < KP; ++p) {
+      const int k = k0 + 2 * p + n.half;
+      const double s = op.escale[k < kend ? k : kend - 1];
+      acc[0][p] = acc[0][p] + s * accE[0][p];
+      acc[1][p] = acc[1][p] + s * accE[1][p];
+    }
+  }
+  // the two rows' ends as a loop: half the code in the instruction cache
+  RowFactors f0 = fa;
+  RowConst rc = rt.ca;
+  int da = rt.a, diag = rt.diag_a, part = rt.part_a;
+#pragma unroll 1
+  for (int r = 0;;) {
+    if (part >= 0) {
+#pragma unroll
+      for (int p = 0; p < KP; ++p)
+        if (k0 + 2 * p + n.half < kend)
+          pstore<SC1>(acc[0][p], T.part, n.off,
+                      part + (s2 ? T.phalf : 0) + (k0 + 2 * p) * (WAVE * 8));
+    } else {
+      own_loads<KP>(T, s2, da, k0, n, xo, fo);
+      d2 src[KP];
+#pragma unroll
+      for (int p = 0; p < KP; ++p) src[p] = d2{0.0, 0.0};
+      team_source<KP>(op, sch, si.step, rc.sslot, k0, kend, n, src);
+      team_epilogue<KP, TWO, REC>(op, st, T, L, si, s2, f0, rc, da, diag, k0, kend, n, acc[0], xo,
+                                  fo, src);
+    }
+    if (++r == 2 || rt.b < 0) break;
+    f0 = fb;
+    rc = rt.cb;
+    da = rt.b;
+    diag = rt.diag_b;
+    part = rt.part_b;
+#pragma unroll
+    for (int p = 0; p < KP; ++p) acc[0][p] = acc[1][p];
+  }
+}
+
+// The same for one row and one pair of right-hand sides (teams of one or two
+// columns), ordered for latency: every load is issued first, the diagonal
+// factors are computed while they travel.  SPLIT (one right-hand side): the
+// upper half of the wave takes every second mother instead of a second column.
+template <bool TWO, bool REC, bool SPLIT>
+__device__ __forceinline__ void team_row1(COp& op, CSch& sch,
+                                          CSt& st, const TeamState& T,
+                                          const TeamLds& L, const StepIn& si, int s2,
+                                          const RowTask& rt, int k0, int kend, const Lane& n) {
+  constexpr int U = SPLIT ? 8 : 12;
+  constexpr int NB = SPLIT ? 2 : 1;  // mothers per load
+  const auto y = s2 ? T.a : T.x;
+  const int cb = k0 * (WAVE * 8);
+  const d2 z = {0.0, 0.0};
+  d2 acc[1] = {z}, xo[1] = {z}, fo[1] = {z}, src[1] = {z}, accE = z;
+  RowFactors f0{};
+  // offset of entry e's panel for this lane (SPLIT: e or e + 1 by half)
+  auto panel = [&](int e, int& slot, bool& has) {
+    int po = __builtin_amdgcn_readlane(rt.mo, e) * T.pb;
+    slot = __builtin_amdgcn_readlane(rt.sl, e);
+    has = true;
+    if (SPLIT) {
+      const int e1 = e + 1 < rt.na ? e + 1 : e;
+      const int p1 = __builtin_amdgcn_readlane(rt.mo, e1) * T.pb;
+      const int s1 = __builtin_amdgcn_readlane(rt.sl, e1);
+      po = n.half ? p1 : po;
+      slot = n.half ? s1 : slot;
+      has = e + n.half < rt.na;
+    }
+    return po;
+  };
+  for (int e = 0;; e += U * NB) {
+    d2 xv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (e + u * NB < rt.na) {
+        int slot;
+        bool has;
+        const int po = panel(e + u * NB, slot, has);
+        xv[u] = SPLIT ? pload<SC1>(y, n.bin * 8 + po, cb) : pload<SC1>(y, n.off, po + cb);
+      }
+    }
+    if (e == 0 && rt.part_a < 0) {
+      own_loads<1>(T, s2, rt.a, k0, n, xo, fo);
+      team_source<1>(op, sch, si.step, rt.ca.sslot, k0, kend, n, src);
+      if (!TWO) f0 = row_factors<false>(op, L, si, s2, rt.ca.pscale, rt.diag_a, k0, n);
+    }
+#pragma unroll
+    for (int u0 = 0; u0 < U; u0 += 4) {
+      d2 mc[4], me[4];
+      bool has[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        int slot;
+        const int ee = e + (u0 + u) * NB;
+        panel(ee < rt.na ? ee : rt.na - 1 < 0 ? 0 : rt.na - 1, slot, has[u]);
+        mc[u] = lds2(L.val, slot, n.bin);
+        if (TWO) me[u] = lds2(L.val, L.slots + slot, n.bin);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (e + (u0 + u) * NB < rt.na) {
+          // a half without a block adds 0 * 0, whatever the panel holds
+          const d2 x = has[u] ? xv[u0 + u] : z;
+          acc[0] += mc[u] * x;
+          if (TWO) accE += me[u] * x;
+        }
+      }
+    }
+    if (e + U * NB >= rt.na) break;
+  }
+  if (TWO) {
+    const int k = k0 + (SPLIT ? 0 : n.half);
+    acc[0] = acc[0] + op.escale[k < kend ? k : kend - 1] * accE;
+  }
+  if (SPLIT) {
+    acc[0].x += __shfl_xor(acc[0].x, 32, WAVE);
+    acc[0].y += __shfl_xor(acc[0].y, 32, WAVE);
+  }
+  if (rt.part_a >= 0) {
+    if (k0 + n.half < kend)
+      pstore<SC1>(acc[0], T.part, n.off, rt.part_a + (s2 ? T.phalf : 0) + cb);
+    return;
+  }
+  team_epilogue<1, TWO, REC>(op, st, T, L, si, s2, f0, rt.ca, rt.a, rt.diag_a, k0, kend, n, acc, xo,
+                             fo, src);
+}
+
+// A tail row to finish; its blocks from tail mothers sit one per lane.
+struct FinTask {
+  int da, slot, p0, pstep, pn, nb;
+  RowConst rc;
+  int mo, sl, band;  // lane entries: mother, LDS slot, first diagonal | diagonals << 8
+};
+__device__ __forceinline__ FinTask fin_task(COp& op, CTm& tm, int f,
+                                            int lane) {
+  const int* fr = tm.fin + 8 * f;
+  FinTask r;
+  r.da = cload(fr);
+  r.slot = cload(fr + 1);
+  r.p0 = cload(fr + 2);
+  r.pstep = cload(fr + 3);
+  r.pn = cload(fr + 4);
+  r.nb = cload(fr + 6);
+  r.rc = row_const(op, r.da);
+  r.mo = r.sl = r.band = 0;
+  if (lane < r.nb) {
+    const int* q = tm.fin_blk + 4 * (cload(fr + 5) + lane);
+    r.mo = q[0];
+    r.sl = q[1];
+    r.band = q[2] | q[3] << 8;
+  }
+  return r;
+}
+
+// One stage of a tail row for the pair of right-hand sides from k0: the partial
+// sums of its heavy mothers (of this stage) in their order, then its blocks from
+// tail mothers.  Every load is issued before the first use.
+template <bool TWO, bool REC>
+__device__ __forceinline__ void team_finish(COp& op, CSch& sch,
+                                            CSt& st, const TeamState& T,
+                                            const TeamLds& L, const StepIn& si, int stage,
+                                            const FinTask& ft, int k0, int kend, const Lane& n) {
+  constexpr int U = 6, UB = 5;
+  const auto y = stage ? T.a : T.x;
+  const int pbase = stage ? T.phalf : 0;
+  const int cb = k0 * (WAVE * 8);
+  const d2 z = {0.0, 0.0};
+  d2 acc[1] = {z}, xo[1], fo[1], src[1] = {z};
+  d2 accB = z, accE = z, xv[UB], pv[U];
+#pragma unroll
+  for (int u = 0; u < UB; ++u)
+    if (u < ft.nb) xv[u] = pload<SC1>(y, n.off, __builtin_amdgcn_readlane(ft.mo, u) * T.pb + cb);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (u < ft.pn) pv[u] = pload<SC1>(T.part, n.off, pbase + (ft.p0 + u * ft.pstep) * T.pb + cb);
+  own_loads<1>(T, stage, ft.da, k0, n, xo, fo);
+  team_source<1>(op, sch, si.step, ft.rc.sslot, k0, kend, n, src);
+  // one part after the other: all of them in flight at once would spill
+  __builtin_amdgcn_sched_barrier(0);
+  for (int g = 0;;) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (g + u < ft.pn) acc[0] += pv[u];
+    g += U;
+    if (g >= ft.pn) break;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (g + u < ft.pn)
+        pv[u] = pload<SC1>(T.part, n.off, pbase + (ft.p0 + (g + u) * ft.pstep) * T.pb + cb);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  RowFactors f0{};
+  if (!TWO) f0 = row_factors<false>(op, L, si, stage, ft.rc.pscale, ft.slot, k0, n);
+  __builtin_amdgcn_sched_barrier(0);
+  for (int b = 0;;) {
+#pragma unroll 1
+    for (int u = 0; u < UB && b + u < ft.nb; ++u) {
+      const int band = __builtin_amdgcn_readlane(ft.band, b + u);
+      const int sl = __builtin_amdgcn_readlane(ft.sl, b + u);
+      const int ns = band >> 8, ol = band & 255;
+      d2 mc[8], me[TWO ? 8 : 1];
+#pragma unroll
+      for (int s2 = 0; s2 < 8; ++s2) {
+        const int s = sl + (s2 < ns ? s2 : ns - 1);
+        mc[s2] = lds2(L.val, s, n.bin);
+        if (TWO) me[TWO ? s2 : 0] = lds2(L.val, L.slots + s, n.bin);
+      }
+      for (int o = 0; o < ol; ++o) xv[0] = shift_bin(n, xv[0]);
+#pragma unroll
+      for (int s2 = 0; s2 < 8; ++s2) {
+        if (s2 < ns) {
+          accB += mc[s2] * xv[0];
+          if (TWO) accE += me[TWO ? s2 : 0] * xv[0];
+          xv[0] = shift_bin(n, xv[0]);
+        }
+      }
+#pragma unroll
+      for (int v = 0; v + 1 < UB; ++v) xv[v] = xv[v + 1];  // the next block's panel
+    }
+    b += UB;
+    if (b >= ft.nb) break;
+#pragma unroll
+    for (int u = 0; u < UB; ++u)
+      if (b + u < ft.nb)
+        xv[u] = pload<SC1>(y, n.off, __builtin_amdgcn_readlane(ft.mo, b + u) * T.pb + cb);
+  }
+  if (TWO) accB += op.escale[k0 + n.half < kend ? k0 + n.half : kend - 1] * accE;
+  acc[0] = acc[0] + accB;
+  team_epilogue<1, TWO, REC>(op, st, T, L, si, stage, f0, ft.rc, ft.da, ft.slot, k0, kend, n, acc,
+                             xo, fo, src);
+}
+
+// Per-lane descriptor of a dense-row wave: entry lane = one mother.
+struct DenseDesc {
+  // LDS slot and (first diagonal | diagonals << 8) per dense row; the second row
+  // has single diagonals only
+  int mo, s0, b0, s1, b1;
+};
+
+// Partial sums of the dense rows over this wave's mothers (entries 0 .. ne-1 of
+// its descriptor lanes) for the KP pairs of right-hand sides from k0.
+template <int KP, bool TWO>
+__device__ __forceinline__ void dense_partial(COp& op, __amdgpu_buffer_rsrc_t y,
+                                              int pb, const TeamLds& L, const DenseDesc& dd, int ne,
+                                              int k0, int kend, const Lane& n,
+                                              d2 (&acc)[TDENSE][KP]) {
+  constexpr int U = 2;
+  d2 accE[TDENSE][KP];
+#pragma unroll
+  for (int p = 0; p < KP; ++p) acc[0][p] = acc[1][p] = accE[0][p] = accE[1][p] = d2{0.0, 0.0};
+  const int cb = k0 * (WAVE * 8);
+  for (int e = 0; e < ne; e += U) {
+    d2 xv[U][KP];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (e + u < ne) {
+        const int po = __builtin_amdgcn_readlane(dd.mo, e + u) * pb + cb;
+#pragma unroll
+        for (int p = 0; p < KP; ++p) xv[u][p] = pload<SC1>(y, n.off, po + p * (2 * WAVE * 8));
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (e + u < ne) {
+        // the second row (He-4: one diagonal) before the band moves the panel
+#pragma unroll
+        for (int r = TDENSE - 1; r >= 0; --r) {
+          const int ss = __builtin_amdgcn_readlane(r ? dd.s1 : dd.s0, e + u);
+          const int bd = __builtin_amdgcn_readlane(r ? dd.b1 : dd.b0, e + u);
+          const int ns = bd >> 8, ol = bd & 255;
+          if (ns == 0) continue;
+          d2 xs[KP], mc[8], me[TWO ? 8 : 1];
+          // the values first (no wait per diagonal), then products and shifts
+#pragma unroll
+          for (int s2 = 0; s2 < 8; ++s2) {
+            const int sl = ss + (s2 < ns ? s2 : ns - 1);
+            if (r == 0 || s2 == 0) mc[s2] = lds2(L.val, sl, n.bin);
+            if (TWO && (r == 0 || s2 == 0)) me[TWO ? s2 : 0] = lds2(L.val, L.slots + sl, n.bin);
+          }
+#pragma unroll
+          for (int p = 0; p < KP; ++p) xs[p] = xv[u][p];
+          for (int o = 0; o < ol; ++o) {
+#pragma unroll
+            for (int p = 0; p < KP; ++p) xs[p] = shift_bin(n, xs[p]);
+          }
+#pragma unroll
+          for (int s2 = 0; s2 < (r == 0 ? 8 : 1); ++s2) {
+            if (s2 < ns) {
+#pragma unroll
+              for (int p = 0; p < KP; ++p) {
+                acc[r][p] += mc[s2] * xs[p];
+                if (TWO) accE[r][p] += me[TWO ? s2 : 0] * xs[p];
+              }
+              if (s2 + 1 < ns) {
+#pragma unroll
+                for (int p = 0; p < KP; ++p) xs[p] = shift_bin(n, xs[p]);
+              }
+            }
+          }
+        }
+      }
+    }
+  }
+  if (TWO) {
+#pragma unroll
+    for (int p = 0; p < KP; ++p) {
+      const int k = k0 + 2 * p + n.half;
+      const double s = op.escale[k < kend ? k : kend - 1];
+      acc[0][p] += s * accE[0][p];
+      acc[1][p] += s * accE[1][p];
+    }
+  }
+}
+
+// Arrive at and wait for a team barrier.  Stores of every wave have reached the
+// coherence point before the arrival (vmcnt(0) of sc1 stores).  Returns false
+// when the march is aborted.
+__device__ __forceinline__ bool wait_count(const uint32_t* c, uint32_t target, uint32_t* abort_w) {
+  int spins = 0;
+  while (__hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
+    if ((++spins & 1023) == 0 &&
+        (spins >= SPIN_LIMIT ||
+         __hip_atomic_load(abort_w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+      __hip_atomic_store(abort_w, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return false;
+    }
+  }
+  return true;
+}
+__device__ __forceinline__ bool team_barrier(uint32_t* sub, uint32_t nsubwg, uint32_t* root,
+                                             uint32_t nsub, uint32_t epoch, uint32_t* abort_w,
+                                             int* bad) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (nsubwg * nsub == 1) return true;
+  if (threadIdx.x == 0) {
+    bool ok;
+    if (nsub > 1) {
+      const uint32_t old =
+          __hip_atomic_fetch_add(sub, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (old + 1 == epoch * nsubwg)
+        __hip_atomic_fetch_add(root, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      ok = wait_count(root, epoch * nsub, abort_w);
+    } else {
+      __hip_atomic_fetch_add(sub, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      ok = wait_count(sub, epoch * nsubwg, abort_w);
+    }
+    if (!ok) *bad = 1;
+  }
+  __syncthreads();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  return *bad == 0;
+}
+
+__global__ void team_reset(uint32_t* sync) {
+  for (int i = threadIdx.x; i < SY_WORDS; i += blockDim.x) sync[i] = 0;
+}
+
+// Where a workgroup stands in its team, and the team's sync words.
+struct TeamPos {
+  int rank, c0, cend;  // right-hand sides [c0, cend) of the team
+  int wv;
+  Lane n;
+  uint32_t *sub, *root, *abort_w;
+  uint32_t nsub, nsubwg;
+  int* bad;
+};
+
+__device__ __forceinline__ bool next_phase(const TeamPos& P, uint32_t& epoch) {
+  return team_barrier(P.sub, P.nsubwg, P.root, P.nsub, ++epoch, P.abort_w, P.bad);
+}
+
+template <bool REC>
+__device__ __forceinline__ StepIn step_in(CSch& sch, CSt& st, int step) {
+  StepIn si;
+  si.step = step;
+  si.dl = cload(sch.dldz + step);
+  si.h = cload(sch.h + step);
+  si.hadia = cload(sch.hadia + step);
+  si.finj = cload(sch.finj + step);
+  si.ridx = REC && step - st.rec_first < st.rec_count ? step - st.rec_first : -1;
+  return si;
+}
+
+// This workgroup's coupling values and the pair rate of window w into LDS (the
+// caller puts barriers around it).
+template <bool TWO>
+__device__ __forceinline__ void load_window(COp& op, CTm& tm,
+                                            const TeamLds& L, const TeamPos& P, int w) {
+  const double* mv = op.mvals + (int64_t)w * op.mvals_stride;
+  const double* me = TWO ? op.mvals_e + (int64_t)w * op.mvals_stride : nullptr;
+  const int* vo = tm.lds_voff + tm.lds_ptr[P.rank];
+  const int lane = P.n.id;
+#pragma unroll 4
+  for (int s = P.wv; s < L.slots; s += TWAVES) {
+    const int v = cload(vo + s) + lane;
+    L.val[s * WAVE + lane] = mv[v];
+    if (TWO) L.val[(L.slots + s) * WAVE + lane] = me[v];
+  }
+  if (P.wv == 0) {
+    L.rp[lane] = op.rpair[(int64_t)w * WAVE + lane];
+    if (TWO) L.rp[WAVE + lane] = op.rpair_e[(int64_t)w * WAVE + lane];
+  }
+}
+
+__device__ __forceinline__ RowTask row_task(COp& op, CTm& tm, int t,
+                                            int lane, int pb) {
+  const int* tk = tm.rows + 10 * t;
+  RowTask r;
+  r.a = cload(tk);
+  r.b = cload(tk + 1);
+  r.n2 = cload(tk + 2);
+  r.na = cload(tk + 3);
+  r.nb = cload(tk + 4);
+  r.diag_a = cload(tk + 5);
+  r.diag_b = cload(tk + 6);
+  const int pa = cload(tk + 7), pq = cload(tk + 8), first = cload(tk + 9);
+  r.part_a = pa < 0 ? -1 : pa * pb;
+  r.part_b = pq < 0 ? -1 : pq * pb;
+  r.ca = row_const(op, r.a);
+  r.cb = row_const(op, r.b < 0 ? r.a : r.b);
+  r.mo = r.sl = 0;
+  if (lane < r.n2 + r.na + r.nb) {
+    const int* q = tm.mothers + 2 * (first + lane);
+    r.mo = q[0];
+    r.sl = q[1];
+  }
+  return r;
+}
+
+// The state descriptors of this phase.
+__device__ __forceinline__ TeamState team_state(CArgs* a) {
+  TeamState T;
+  T.pb = a->op.K * WAVE * 8;
+  T.x = tile_rsrc(a->st.x, a->op.nspec * T.pb);
+  T.a = tile_rsrc(a->st.a, a->op.nspec * T.pb);
+  T.f = tile_rsrc(a->st.fphi, a->op.nspec * T.pb);
+  T.phalf = a->tm.nparts * T.pb;
+  T.part = tile_rsrc(a->tm.dpart, 2 * T.phalf);
+  return T;
+}
+
+// March of a workgroup of rows: wave wv's tasks.  R = 2: row pairs, KP pairs of
+// right-hand sides a pass, two waves per task (each every second pass).
+template <int R, int KP, bool TWO, bool REC, bool SPLIT>
+__device__ __forceinline__ void march_rows(CArgs* A, const TeamLds& L, const TeamPos& P) {
+  const int k_begin = A->k_begin, k_end = A->k_end;
+  const int* wt = A->tm.wave_ptr + P.rank * TWAVES + P.wv;
+  const int t0 = cload(wt), t1 = cload(wt + 1);
+  RowTask first{};  // most waves have one task: it stays in registers
+  if (t0 < t1) first = row_task(A->op, A->tm, t0, P.n.id, A->op.K * WAVE * 8);
+  uint32_t epoch = 0;
+  int wcur = -1;
+#pragma unroll 1
+  for (int p = 2 * k_begin; p < 2 * k_end; ++p) {
+    CArgs* a = reread(A);
+    const int s2 = p & 1, step = p >> 1;
+    if (s2 == 0) {
+      const int w = cload(a->sch.win + step);
+      if (w != wcur) {
+        __syncthreads();
+        load_window<TWO>(a->op, a->tm, L, P, w);
+        wcur = w;
+        __syncthreads();
+      }
+    }
+    const StepIn si = step_in<REC>(a->sch, a->st, step);
+    const TeamState T = team_state(a);
+#pragma unroll 1
+    for (int t = t0; t < t1; ++t) {
+      RowTask rt = first;
+      if (t != t0) rt = row_task(a->op, a->tm, t, P.n.id, T.pb);
+      if constexpr (R == 1) {
+        team_row1<TWO, REC, SPLIT>(a->op, a->sch, a->st, T, L, si, s2, rt, P.c0, P.cend, P.n);
+      } else {
+        RowFactors fa{}, fb{};
+        if (!TWO) {
+          if (rt.part_a < 0)
+            fa = row_factors<false>(a->op, L, si, s2, rt.ca.pscale, rt.diag_a, P.c0, P.n);
+          if (rt.b >= 0 && rt.part_b < 0)
+            fb = row_factors<false>(a->op, L, si, s2, rt.cb.pscale, rt.diag_b, P.c0, P.n);
+        }
+#pragma unroll 1
+        for (int k0 = P.c0 + 2 * KP * (P.wv & 1); k0 < P.cend; k0 += 4 * KP)
+          team_rows<KP, TWO, REC>(a->op, a->sch, a->st, T, L, si, s2, rt, fa, fb, k0, P.cend, P.n);
+      }
+    }
+    if (!next_phase(P, epoch)) return;
+  }
+}
+
+// One stage's partial sums of a dense-row workgroup, KP pairs of right-hand
+// sides per wave: mother group dg, column group dc.
+template <int KP, bool TWO>
+__device__ __forceinline__ void dense_stage_partials(COp& op, CTm& tm,
+                                                     const TeamState& T, const TeamLds& L,
+                                                     const TeamPos& P, __amdgpu_buffer_rsrc_t y,
+                                                     int pbase, const DenseDesc& dd, int ne, int dg,
+                                                     int dc) {
+  const int dG = tm.dgroups, dC = TWAVES / dG;
+  const int po = pbase + P.rank * TDENSE * T.pb;
+  d2* const red = reinterpret_cast<d2*>(L.red);
+  for (int k0 = P.c0 + dc * 2 * KP; k0 < P.cend; k0 += dC * 2 * KP) {
+    d2 acc[TDENSE][KP];
+    dense_partial<KP, TWO>(op, y, T.pb, L, dd, ne, k0, P.cend, P.n, acc);
+#pragma unroll
+    for (int r = 0; r < TDENSE; ++r)
+#pragma unroll
+      for (int p = 0; p < KP; ++p) {
+        if (KP == 1 && dG > 1)
+          red[(P.wv * TDENSE + r) * WAVE + P.n.id] = acc[r][p];
+        else if (k0 + 2 * p + P.n.half < P.cend)
+          pstore<SC1>(acc[r][p], T.part, P.n.off, po + r * T.pb + (k0 + 2 * p) * (WAVE * 8));
+      }
+  }
+  if (KP == 1 && dG > 1) {  // one column pass (2 dC covers the columns): add the mother groups in order
+    __syncthreads();
+    const int k0 = P.c0 + dc * 2;
+    if (dg < TDENSE && k0 < P.cend) {
+      d2 s = {0.0, 0.0};
+      for (int g = 0; g < dG; ++g) s += red[((g * dC + dc) * TDENSE + dg) * WAVE + P.n.id];
+      if (k0 + P.n.half < P.cend)
+        pstore<SC1>(s, T.part, P.n.off, po + dg * T.pb + k0 * (WAVE * 8));
+    }
+  }
+}
+
+// March of a dense-row workgroup: partial sums over its mothers.
+template <int KD, bool TWO>
+__device__ __forceinline__ void march_dense(CArgs* A, const TeamLds& L, const TeamPos& P) {
+  const int k_begin = A->k_begin, k_end = A->k_end;
+  const int dG = A->tm.dgroups, dC = TWAVES / dG;
+  const int dg = P.wv / dC, dc = P.wv % dC;
+  const int* ep = A->tm.dense_ptr + P.rank * dG + dg;
+  const int e0 = cload(ep), ne = cload(ep + 1) - e0;
+  DenseDesc dd{0, 0, 0, 0, 0};
+  if (P.n.id < ne) {
+    const int* q = A->tm.dense_ent + 5 * (e0 + P.n.id);
+    dd = DenseDesc{q[0], q[1], q[2], q[3], q[4]};
+  }
+  uint32_t epoch = 0;
+  int wcur = -1;
+#pragma unroll 1
+  for (int p = 2 * k_begin; p < 2 * k_end; ++p) {
+    CArgs* a = reread(A);
+    const int s2 = p & 1;
+    if (s2 == 0) {
+      const int w = cload(a->sch.win + (p >> 1));
+      if (w != wcur) {
+        __syncthreads();
+        load_window<TWO>(a->op, a->tm, L, P, w);
+        wcur = w;
+        __syncthreads();
+      }
+    }
+    const TeamState T = team_state(a);
+    dense_stage_partials<KD, TWO>(a->op, a->tm, T, L, P, s2 ? T.a : T.x, s2 ? T.phalf : 0, dd, ne,
+                                  dg, dc);
+    if (!next_phase(P, epoch)) return;
+  }
+}
+
+// March of a finishing workgroup: the tail rows, one stage behind the others.
+template <bool TWO, bool REC>
+__device__ __forceinline__ void march_finish(CArgs* A, const TeamLds& L, const TeamPos& P) {
+  constexpr int NF = TWO ? 2 : 1;
+  const int k_begin = A->k_begin, k_end = A->k_end;
+  const int groups = (P.cend - P.c0 + 1) / 2;
+  const int items = A->tm.nfin * groups;
+  const int it0 = (P.rank - A->tm.ndwg) * TWAVES + P.wv;
+  const int stride = A->tm.nfwg * TWAVES;
+  uint32_t epoch = 0;
+  int wcur = -1, buf = 0;
+  auto set = [&](int b) {  // LDS of value set b
+    TeamLds Q = L;
+    Q.val = L.val + b * NF * L.slots * WAVE;
+    Q.rp = L.rp + b * NF * WAVE;
+    return Q;
+  };
+  FinTask first{};
+  if (it0 < items) first = fin_task(A->op, A->tm, it0 / groups, P.n.id);
+  // phase p finishes stage p - 1: stage 2 of the step before, or stage 1 of its
+  // own; sbuf: the value set of that stage
+  int sbuf = 0;
+#pragma unroll 1
+  for (int p = 2 * k_begin; p <= 2 * k_end; ++p) {
+    CArgs* a = reread(A);
+    const int s2 = (p & 1) ^ 1;
+    sbuf = buf;
+    if (s2 && p < 2 * k_end) {
+      const int w = cload(a->sch.win + (p >> 1));
+      if (w != wcur) {
+        // into the other set: the last one is still read for the step before; the
+        // phase's workgroup barriers complete it
+        buf ^= 1;
+        load_window<TWO>(a->op, a->tm, set(buf), P, w);
+        wcur = w;
+      }
+    }
+    if (p > 2 * k_begin) {
+      const TeamLds Q = set(sbuf);
+      const StepIn si = step_in<REC>(a->sch, a->st, (p - 1) >> 1);
+      const TeamState T = team_state(a);
+#pragma unroll 1
+      for (int it = it0; it < items; it += stride) {
+        const int f = it / groups;
+        FinTask ft = first;
+        if (it != it0) ft = fin_task(a->op, a->tm, f, P.n.id);
+        team_finish<TWO, REC>(a->op, a->sch, a->st, T, Q, si, s2, ft, P.c0 + (it - f * groups) * 2,
+                              P.cend, P.n);
+      }
+    }
+    if (p < 2 * k_end && !next_phase(P, epoch)) return;
+  }
+}
+
+template <int R, int KP, int KD, bool TWO, bool REC, bool SPLIT>
+__global__ void __launch_bounds__(TTHREADS) team_march(TeamArgs) {
+  extern __shared__ __attribute__((aligned(16))) double lds[];  // 16-byte reads
+  __shared__ int bad;
+  CArgs* const A = reinterpret_cast<CArgs*>(
+      reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr()));
+  const int K = A->op.K, nteam = A->tm.nteam, size = A->tm.size;
+  const int team = (int)blockIdx.x % nteam;
+  TeamPos P;
+  P.rank = (int)blockIdx.x / nteam;
+  P.n = lane_of();
+  P.wv = wave_id();
+  const int per = K / nteam, rem = K % nteam;
+  P.c0 = team * per + (team < rem ? team : rem);
+  P.cend = P.c0 + per + (team < rem ? 1 : 0);
+  if (P.c0 == P.cend) return;  // uniform over the team: none of its workgroups waits
+
+  TeamLds L;
+  L.cst = lds;
+  L.rp = L.cst + TCONST * WAVE;
+  L.red = L.rp + (TWO ? 4 : 2) * WAVE;
+  L.val = L.red + A->tm.red_slots * WAVE;
+  L.slots = cload(A->tm.lds_ptr + P.rank + 1) - cload(A->tm.lds_ptr + P.rank);
+  for (int i = threadIdx.x; i < WAVE; i += TTHREADS) {
+    for (int o = 0; o < 7; ++o)
+      L.cst[o * WAVE + i] = (A->op.flags & PRH_F_PARTIAL_DIFF) ? A->op.dcoef[i * 7 + o] : 0.0;
+    L.cst[7 * WAVE + i] = A->op.egrid[i];
+    L.cst[8 * WAVE + i] = A->op.ddiag[i];
+  }
+  if (threadIdx.x == 0) bad = 0;
+  P.bad = &bad;
+
+  P.nsub = size > 32 ? size / 32 : 1;
+  P.nsubwg = (uint32_t)size / P.nsub;
+  P.sub = A->tm.sync + SY_SUB + (team * 8 + P.rank % P.nsub) * 64;
+  P.root = A->tm.sync + SY_ROOT + team * 64;
+  P.abort_w = A->tm.sync + SY_ABORT;
+  __syncthreads();
+
+  const int ndwg = A->tm.ndwg, nfwg = A->tm.nfwg;
+  if (P.rank < ndwg)
+    march_dense<KD, TWO>(A, L, P);
+  else if (P.rank < ndwg + nfwg)
+    march_finish<TWO, REC>(A, L, P);
+  else
+    march_rows<R, KP, TWO, REC, SPLIT>(A, L, P);
+  if (bad) {  // aborted: no silent result
+    for (int i = P.rank * TWAVES + P.wv; i < A->op.nspec; i += size * TWAVES)
+      for (int k = P.c0; k < P.cend; ++k)
+        A->st.x[((int64_t)i * K + k) * WAVE + P.n.id] = __builtin_nan("");
+  }
+}
+
+// Marches of one process on one device run one after the other, whatever streams
+// they are on: each waits for the event of the one before.  Two of them on the
+// chip together could each hold CUs the other's barriers need.
+constexpr int MAX_DEVICES = 64;
+std::mutex g_order_mu;
+hipEvent_t g_last_march[MAX_DEVICES] = {};
+
+template <int R, int KP, int KD, bool TWO, bool REC, bool SPLIT>
+int32_t launch_team_rec(const prh_operator& op, const prh_schedule& sch, const prh_state& st,
+                        const prh_team& tm, int k_begin, int k_end, hipStream_t s) {
+  const void* fn = reinterpret_cast<const void*>(&team_march<R, KP, KD, TWO, REC, SPLIT>);
+  const size_t lds =
+      8 * WAVE * (size_t)(TCONST + (TWO ? 4 : 2) + tm.red_slots + tm.lds_slots * (TWO ? 2 : 1));
+  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return prh_internal::check(e, "prh_team_march: dynamic LDS");
+  TeamArgs ta{op, sch, st, tm, k_begin, k_end};
+  void* args[] = {&ta};
+  int dev = -1;
+  e = hipGetDevice(&dev);
+  if (e != hipSuccess || dev < 0 || dev >= MAX_DEVICES)
+    return prh_internal::error("prh_team_march: no current device in [0, 64)");
+  std::lock_guard<std::mutex> lock(g_order_mu);
+  hipEvent_t& last = g_last_march[dev];
+  if (!last) {
+    e = hipEventCreateWithFlags(&last, hipEventDisableTiming);
+  } else {
+    e = hipStreamWaitEvent(s, last, 0);
+  }
+  if (e != hipSuccess) return prh_internal::check(e, "prh_team_march: march order");
+  hipLaunchKernelGGL(team_reset, dim3(1), dim3(1024), 0, s, tm.sync);
+  e = hipGetLastError();
+  if (e == hipSuccess)
+    e = hipLaunchCooperativeKernel(fn, dim3((unsigned)(tm.nteam * tm.size)), dim3(TTHREADS), args,
+                                   (unsigned)lds, s);
+  if (e == hipSuccess) e = hipEventRecord(last, s);
+  const int32_t rc = prh_internal::check(e, "prh_team_march launch");
+  // the device cannot hold the whole grid at once (or not cooperatively)
+  return e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported ? 2 : rc;
+}
+
+template <int R, int KP, int KD, bool TWO, bool SPLIT>
+int32_t launch_team(const prh_operator& op, const prh_schedule& sch, const prh_state& st,
+                    const prh_team& tm, int k_begin, int k_end, hipStream_t s) {
+  return st.rec_x ? launch_team_rec<R, KP, KD, TWO, true, SPLIT>(op, sch, st, tm, k_begin, k_end, s)
+                  : launch_team_rec<R, KP, KD, TWO, false, SPLIT>(op, sch, st, tm, k_begin, k_end, s);
+}
+
+}  // namespace
+
+extern "C" int32_t prh_team_march(const prh_operator* op, const prh_schedule* sch,
+                                  const prh_state* st, const prh_team* tm, int32_t k_begin,
+                                  int32_t k_end, void* stream) {
+  using prh_internal::error;
+  if (!op || !sch || !st || !tm) return error("prh_team_march: null argument");
+  if (op->d != WAVE) return error("prh_team_march: 64 energy bins only");
+  if (op->K <= 0 || op->nspec <= 0) return error("prh_team_march: empty operator");
+  // byte offsets of the state and of the partials are 32-bit
+  if ((int64_t)op->nspec * op->K * WAVE * 8 > 0x7fffffff ||
+      2 * (int64_t)tm->nparts * op->K * WAVE * 8 > 0x7fffffff)
+    return error("prh_team_march: a state array exceeds 2 GiB");
+  if ((op->mvals_e == nullptr) != (op->escale == nullptr) ||
+      (op->mvals_e != nullptr && op->rpair_e == nullptr))
+    return error("prh_team_march: mvals_e, rpair_e and escale go together");
+  if (st->em) return error("prh_team_march: no EM sector");
+  if (!st->x || !st->a || !st->fphi) return error("prh_team_march: null state");
+  if (st->rec_x && (!st->rec_a || !st->rec_fx || !st->rec_fa))
+    return error("prh_team_march: recording needs all four record arrays");
+  if (k_begin < 0 || k_end > sch->nsteps || k_begin > k_end)
+    return error("prh_team_march: step range outside the schedule");
+  if (tm->nteam < 1 || tm->nteam > 8 || tm->size < 1 || tm->size > 256 ||
+      (tm->size > 32 && tm->size % 32 != 0))
+    return error("prh_team_march: 1 to 8 teams of up to 32 workgroups, or a multiple of 32");
+  if (tm->ndwg < 0 || tm->nfwg < 0 || tm->nfin < 0 || tm->nparts < TDENSE * tm->ndwg ||
+      tm->ndwg + tm->nfwg > tm->size || (tm->nfin > 0) != (tm->nfwg > 0))
+    return error("prh_team_march: tail rows need finishing workgroups, all within the team");
+  if (!tm->sync || !tm->rows || !tm->wave_ptr || !tm->mothers || !tm->lds_ptr || !tm->lds_voff)
+    return error("prh_team_march: null table");
+  if ((tm->ndwg > 0 && (!tm->dense_ptr || !tm->dense_ent)) ||
+      (tm->nfin > 0 && (!tm->fin || !tm->fin_blk)) || (tm->nparts > 0 && !tm->dpart))
+    return error("prh_team_march: tail rows need their tables and partials");
+  if (!(tm->kd == 1 || tm->kd == 2) || tm->dgroups < 1 || tm->dgroups > TWAVES ||
+      TWAVES % tm->dgroups != 0)
+    return error("prh_team_march: bad dense-row tiling");
+  const int ncmax = (op->K + tm->nteam - 1) / tm->nteam;
+  if (tm->ndwg > 0 && tm->dgroups > 1 &&
+      (tm->dgroups < TDENSE || tm->kd != 1 || (TWAVES / tm->dgroups) * 2 < ncmax ||
+       tm->red_slots < TWAVES * TDENSE * 2))
+    return error("prh_team_march: mother groups need one column pass and their LDS rows");
+  if (k_begin == k_end) return 0;
+  hipStream_t s = (hipStream_t)stream;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (int32_t e = prh_internal::check(hipStreamIsCapturing(s, &cs), "prh_team_march: capture status"))
+    return e;
+  if (cs != hipStreamCaptureStatusNone) {
+    error("prh_team_march: a cooperative launch cannot be captured; use prh_etd2_steps");
+    return 2;
+  }
+  if (tm->pair_rows == 0 && ncmax > 2)
+    return error("prh_team_march: single-row tasks take at most 2 right-hand sides per team");
+  // one right-hand side per team: the halves of a wave share it
+  const int key = tm->pair_rows == 0 ? ncmax : 10 * tm->kp + tm->kd;
+#define TEAM(R, KP, KD, TWO, SPLIT) \
+  return launch_team<R, KP, KD, TWO, SPLIT>(*op, *sch, *st, *tm, k_begin, k_end, s)
+  if (op->mvals_e) {
+    switch (key) {
+      case 1: TEAM(1, 1, 1, true, true);
+      case 2: TEAM(1, 1, 1, true, false);
+      case 11: TEAM(2, 1, 1, true, false);
+      case 21: TEAM(2, 2, 1, true, false);
+      case 22: TEAM(2, 2, 2, true, false);
+    }
+  } else {
+    switch (key) {
+      case 1: TEAM(1, 1, 1, false, true);
+      case 2: TEAM(1, 1, 1, false, false);
+      case 11: TEAM(2, 1, 1, false, false);
+      case 21: TEAM(2, 2, 1, false, false);
+      case 22: TEAM(2, 2, 2, false, false);
+    }
+  }
+#undef TEAM
+  return error("prh_team_march: no kernel for this kp, kd");
+}

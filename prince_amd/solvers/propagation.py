@@ -42,6 +42,7 @@ from .layout import (
     transposed_layout,
 )
 from .result import UHECRPropagationResult
+from . import team as team_plan
 from .run_inputs import (
     em_cascade_grid,
     em_slices,
@@ -400,6 +401,13 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
             if kt <= K:
                 return kt
         return 1
+
+    def team_march_for(self, K):
+        """Whether the march may run as one cooperative launch (``prh_team_march``):
+        unless a stage configuration was forced or tuned for K."""
+        tuned = getattr(self, "_tuned", {})
+        on = tuned.get(("team", K))
+        return bool(on) if on is not None else not any(key[1] == K for key in tuned)
 
     def __init__(self, *args, **kwargs):
         super().__init__(*args, **kwargs)
@@ -823,11 +831,72 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
             "dense_mode": "pass" if dense is not None else "chunks" if chunked is not None else None,
             "em": em_struct, "em_bufs": em_bufs,
         }
-        if getattr(self.backend, "use_hip_graphs", True) and len(h) >= self.graph_chunk:
-            self._plan["graph"] = _lib.StepGraph(op, sch, st, self.graph_chunk)
+        self._plan["team"] = None
+        if self.team_march_for(K) and em_struct is None:
+            self._plan["team"] = self._team_setup(lay, dv, K, 2 if two else 1)
+        if self._plan["team"] is None:
+            self._capture_steps(self._plan)
         self.refresh_zs = zs
         self.timings["setup_host_s"] = t1 - t0
         return self._plan
+
+    def _capture_steps(self, plan):
+        """The step graph of the stage kernels (solves of at least one chunk)."""
+        if getattr(self.backend, "use_hip_graphs", True) and plan["nsteps"] >= self.graph_chunk:
+            plan["graph"] = _lib.StepGraph(plan["op"], plan["sch"], plan["st"], self.graph_chunk)
+
+    #: team plans (host tables on the device, read only) kept per layout
+    TEAM_PLANS_KEPT = 8
+
+    def _team_setup(self, lay, dv, K, fields):
+        """Team march of this plan (``prh_team``): the layout's tables for K
+        columns, and the plan's own partials and sync words.  None when the
+        operator or the device does not fit it."""
+        torch = _torch()
+        wl = lay["layout"]
+        args = getattr(self, "_tuned", {}).get(("team_args", K), {})
+        key = (K, fields, tuple(sorted(args.items())))
+        plans = lay.setdefault("team", {})
+        if key not in plans:
+            tp = team_plan.build_team(wl.blocks, wl.fwd.brow_ptr, wl.nspec, wl.d, wl.diag_off, K,
+                                      fields, **args)
+            names = ("lds_ptr", "lds_voff", "wave_ptr", "rows", "mothers", "dense_ptr",
+                     "dense_ent", "fin", "fin_blk")
+            tables = None if tp is None else {
+                n: dv(np.append(getattr(tp, n).ravel(), 0), np.int32) for n in names}
+            while len(plans) >= self.TEAM_PLANS_KEPT:
+                plans.pop(next(iter(plans)))
+            plans[key] = (tp, tables)
+        tp, tables = plans[key]
+        props = torch.cuda.get_device_properties(self.device)
+        if tp is None or props.multi_processor_count < tp.nteam * tp.size:
+            return None
+        b = dict(tables)
+        b["sync"] = torch.zeros(team_plan.SYNC_BYTES // 4, dtype=torch.int32, device=self.device)
+        b["dpart"] = torch.empty((2, max(1, tp.nparts), K, wl.d), dtype=torch.float64,
+                                 device=self.device)
+        tm = _lib.PrhTeam(
+            nteam=tp.nteam, size=tp.size, kp=tp.kp, kd=tp.kd, dgroups=tp.dgroups, ndwg=tp.ndwg,
+            nfwg=tp.nfwg, nfin=tp.fin.shape[0], nparts=tp.nparts,
+            lds_slots=tp.lds_slots, red_slots=tp.red_slots,
+            pair_rows=int(tp.pair_rows),
+            **{n: t.data_ptr() for n, t in b.items()})
+        return {"struct": tm, "bufs": b, "plan": tp}
+
+    def _team_run(self, plan, st, k_begin, k_end):
+        """Steps [k_begin, k_end) as one cooperative launch; False when it cannot
+        run here (then the stage kernels take over for this plan)."""
+        team = plan.get("team")
+        if team is None or _torch().cuda.is_current_stream_capturing():
+            return False
+        rc = self._lib.prh_team_march(
+            ctypes.byref(plan["op"]), ctypes.byref(plan["sch"]), ctypes.byref(st),
+            ctypes.byref(team["struct"]), k_begin, k_end, plan["stream"])
+        if rc == _lib.NOT_LAUNCHABLE:
+            plan["team"] = None
+            return False
+        _lib.check(rc, "team march")
+        return True
 
     def _em_setup(self, zs, K, dv):
         """Device buffers of the EM sector: per-window cascade transfers T(z) and
@@ -1005,6 +1074,8 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
 
     def _launch_steps(self, plan, k_begin, k_end, use_graph=True):
         plan["steps_run"] = k_end  # the EM photons' buffer after the last step
+        if self._team_run(plan, plan["st"], k_begin, k_end):
+            return
         if use_graph and plan["graph"] is not None:
             plan["graph"].run(k_begin, k_end, plan["stream"])
             return
@@ -1076,7 +1147,8 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
             lnz1=ab["lnz1"].data_ptr(),
             gdot=ab["gdot"].data_ptr() if plan["two"] else None,
         )
-        if getattr(self.backend, "use_hip_graphs", True) and C == self.graph_chunk:
+        if (plan["team"] is None and getattr(self.backend, "use_hip_graphs", True)
+                and C == self.graph_chunk):
             plan["rec_graph"] = _lib.StepGraph(plan["op"], plan["sch"], plan["st_rec"], C)
         else:
             plan["rec_graph"] = None
@@ -1114,11 +1186,13 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
         for c in range((nsteps + C - 1) // C - 1, -1, -1):
             k0, k1 = c * C, min((c + 1) * C, nsteps)
             plan["x"].copy_(ck[c])
-            if plan["rec_graph"] is not None:
+            st = plan["st_rec"]
+            st.rec_first = k0
+            if self._team_run(plan, st, k0, k1):
+                pass
+            elif plan["rec_graph"] is not None:
                 plan["rec_graph"].run(k0, k1, stream)
             else:
-                st = plan["st_rec"]
-                st.rec_first = k0
                 _lib.check(lib.prh_etd2_steps(ctypes.byref(plan["op"]), ctypes.byref(sch),
                                               ctypes.byref(st), k0, k1, stream), "recompute")
             adj.rec_first = k0

@@ -1,0 +1,280 @@
+"""Plan of the team march (``prh_team_march``): which workgroup of a team owns
+which species rows, and where their coupling values sit in its LDS.
+
+A team is ``size`` workgroups of 16 waves (one per CU), ``nteam`` teams fill the
+chip and each marches its own share of the right-hand sides.  Heavy rows
+(diagonal blocks only) go one per wave, or from 3 right-hand sides per team on as
+pairs of consecutive rows, read with one walk over their mothers by two waves that
+share the right-hand sides.  The tail rows -- the dense rows (at most
+two: band blocks or more than ``ROW_MAX`` blocks) and every row that reads a tail
+row -- run one stage behind them: ``ndwg`` workgroups sum the dense rows over the
+heavy mothers, each taking a contiguous range of mothers for both rows, the other
+tail rows' sums over heavy mothers run among the heavy rows, and ``nfwg``
+workgroups finish the tail rows.  Pure numpy.
+"""
+
+from __future__ import annotations
+
+from dataclasses import dataclass
+
+import numpy as np
+
+WAVES = 16
+CUS = 256
+#: LDS bytes a workgroup may use (160 KB per CU less the kernel's static words)
+LDS_BYTES = 160 * 1024 - 64
+CONST_SLOTS = 9
+ROW_MAX = 32
+DENSE_MAX = 2
+BAND_MAX = 8
+TAIL_MAX = 32
+SYNC_BYTES = 18688
+
+
+@dataclass
+class TeamPlan:
+    nteam: int
+    size: int
+    kp: int
+    kd: int
+    dgroups: int
+    ndwg: int
+    nfwg: int
+    pair_rows: bool
+    nparts: int
+    dense_rows: list
+    lds_slots: int
+    red_slots: int
+    lds_ptr: np.ndarray
+    lds_voff: np.ndarray
+    wave_ptr: np.ndarray
+    rows: np.ndarray
+    mothers: np.ndarray
+    dense_ptr: np.ndarray
+    dense_ent: np.ndarray
+    fin: np.ndarray
+    fin_blk: np.ndarray
+
+    def lds_bytes(self, fields):
+        return 512 * (CONST_SLOTS + 2 * fields + self.red_slots + fields * self.lds_slots)
+
+
+def dense_tiling(nc):
+    """(kd, dgroups) of the dense-row workgroups for ``nc`` columns per team: the
+    16 waves are column groups of ``kd`` pairs of columns times mother groups;
+    mother groups only while one pass of single pairs covers the columns."""
+    if nc <= 16:
+        pairs = 1
+        while 2 * pairs < nc:
+            pairs *= 2
+        return 1, WAVES // pairs
+    return (1 if nc <= 32 else 2), 1
+
+
+def row_tiling(nc):
+    """(row pairs or not, pairs of right-hand sides per pass of a wave)."""
+    return nc > 2, 1 if nc <= 4 else 2
+
+
+def _cut(cost, parts):
+    """Cut a cost list into ``parts`` contiguous ranges of similar cost (bounds)."""
+    c = np.concatenate([[0.0], np.cumsum(cost)])
+    at = np.searchsorted(c, c[-1] * np.arange(1, parts) / parts, side="left")
+    return np.concatenate([[0], np.minimum(at, len(cost)), [len(cost)]]).astype(np.int64)
+
+
+def tail_rows(blocks, ptr, nspec):
+    """(dense rows, tail rows): the tail is the smallest set that holds the dense
+    rows and every row that reads a row of the set."""
+    dense = []
+    for da in range(nspec):
+        b = blocks[ptr[da]:ptr[da + 1]]
+        if len(b) > ROW_MAX or not np.all((b[:, 1] == 0) & (b[:, 2] == 1)):
+            dense.append(da)
+    tail = set(dense)
+    grown = bool(tail)
+    while grown:
+        grown = False
+        for da in range(nspec):
+            if da not in tail and tail.intersection(blocks[ptr[da]:ptr[da + 1], 0].tolist()):
+                tail.add(da)
+                grown = True
+    return dense, sorted(tail)
+
+
+def build_team(blocks, brow_ptr, nspec, d, diag_off, K, fields=1, size=None, ndwg=None, nfwg=None):
+    """Team plan of an operator for K right-hand sides, or None when its rows do
+    not fit the march (d != 64, more than two dense rows, bands left of the
+    diagonal or wider than 8, a long tail, values beyond the LDS)."""
+    if d != 64 or nspec < 1 or nspec * K * 512 > 0x7FFFFFFF:
+        return None
+    blocks = np.asarray(blocks, dtype=np.int64).reshape(-1, 4)
+    ptr = np.asarray(brow_ptr, dtype=np.int64)
+    dense, tail = tail_rows(blocks, ptr, nspec)
+    if len(dense) > DENSE_MAX or len(tail) > TAIL_MAX:
+        return None
+    # the second dense row is the one of single diagonals
+    dense.sort(key=lambda da: -int(blocks[ptr[da]:ptr[da + 1], 2].max()))
+    if len(dense) == 2 and blocks[ptr[dense[1]]:ptr[dense[1] + 1], 2].max() > 1:
+        return None
+    for da in dense:
+        b = blocks[ptr[da]:ptr[da + 1]]
+        if np.any(b[:, 1] < 0) or np.any(b[:, 1] > 255) or np.any(b[:, 2] > BAND_MAX):
+            return None
+    sizes = [1] if len(tail) == nspec else [size] if size is not None else [32, 64, 128, 256]
+    for s in sizes:
+        plan = _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, s, ndwg, nfwg)
+        if plan is not None:
+            return plan
+    return None
+
+
+def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, size, ndwg, nfwg):
+    nteam = min(8, CUS // size)
+    nc = -(-K // nteam)
+    kd, dgroups = dense_tiling(nc)
+    pair_rows, kp = row_tiling(nc)
+    tset = set(tail)
+    # dense entries: one per heavy mother, both rows' blocks
+    ent = {}
+    for r, da in enumerate(dense):
+        for v in range(int(ptr[da]), int(ptr[da + 1])):
+            mo, ol, ns, vo = (int(q) for q in blocks[v])
+            if mo not in tset:
+                ent.setdefault(mo, [[0, 0, 0], [0, 0, 0]])[r] = [ol, ns, vo]
+    mothers = sorted(ent)
+    eslots = np.array([sum(q[1] for q in ent[m]) for m in mothers], dtype=np.int64)
+    red = WAVES * DENSE_MAX * 2 if (mothers and dgroups > 1) else 0
+    budget = (LDS_BYTES // 512 - CONST_SLOTS - 2 * fields - red) // fields
+    if not mothers:
+        ndwg = 0
+    elif ndwg is None:
+        # the least number of workgroups whose LDS holds the dense values
+        ndwg = max(1, -(-int(eslots.sum()) // max(1, budget)))
+        while ndwg < size and max(eslots[a:b].sum() for a, b in zip(*_bounds(eslots, ndwg))) > budget:
+            ndwg += 1
+    heavy = [da for da in range(nspec) if da not in tset]
+    # tail rows that are not dense sum their heavy mothers among the heavy rows
+    light = [da for da in tail if da not in dense]
+    nfwg = 0 if not tail else 1 if size == 1 or nfwg is None and len(tail) * nc <= WAVES else (nfwg or 2)
+    nrow_wg = size - ndwg - nfwg
+    if nrow_wg < (1 if heavy else 0):
+        return None
+    lds_ptr, lds_voff = [0], []
+    dptr, dent = [0], []
+    wave_ptr, rows, mlist = [0], [], []
+    if ndwg:
+        for a, b in zip(*_bounds(eslots, ndwg)):
+            voff = []
+            slot = {}
+            for e in range(a, b):
+                q = []
+                for ol, ns, vo in ent[mothers[e]]:
+                    q += [len(voff) if ns else 0, ol | ns << 8]
+                    voff += [vo + 64 * s for s in range(ns)]
+                slot[e] = q
+            for g in range(dgroups):  # mother groups: contiguous, similar counts
+                lo, hi = a + (b - a) * g // dgroups, a + (b - a) * (g + 1) // dgroups
+                if hi - lo > 64:
+                    return None
+                dent += [[mothers[e]] + slot[e] for e in range(lo, hi)]
+                dptr.append(len(dent))
+            lds_voff += voff
+            lds_ptr.append(len(lds_voff))
+            wave_ptr += [0] * WAVES
+    # finishing workgroups: every tail row's diagonal and its blocks from tail mothers
+    fin, fin_blk, fvoff = [], [], []
+    for da in tail:
+        first = len(fin_blk)
+        slot = len(fvoff)
+        fvoff.append(diag_off + da * 64)
+        for v in range(int(ptr[da]), int(ptr[da + 1])):
+            mo, ol, ns, vo = (int(q) for q in blocks[v])
+            if mo in tset:
+                fin_blk.append([mo, len(fvoff), ol, ns])
+                fvoff += [vo + 64 * s for s in range(ns)]
+        p0, pstep, pn = ((dense.index(da), DENSE_MAX, ndwg) if da in dense
+                         else (DENSE_MAX * ndwg + light.index(da), 1, 1))
+        fin.append([da, slot, p0, pstep, pn, first, len(fin_blk) - first, 0])
+    for _ in range(nfwg):
+        lds_voff += fvoff
+        lds_ptr.append(len(lds_voff))
+        wave_ptr += [0] * WAVES
+    # rows over heavy mothers in species order (neighbouring rows share mothers)
+    rowlist = []
+    for da in sorted(light + heavy):
+        b = blocks[ptr[da]:ptr[da + 1]]
+        b = b[[int(m) not in tset for m in b[:, 0]]] if da in tset else b
+        rowlist.append((da, b, DENSE_MAX * ndwg + light.index(da) if da in tset else -1))
+    per = 2 if pair_rows else 1
+    lanes = WAVES // per  # tasks that run at once in a workgroup
+    tasks = [rowlist[i:i + per] for i in range(0, len(rowlist), per)]
+    cost = np.array([sum(8.0 + len(b) for _, b, _ in t) for t in tasks])
+    if nrow_wg:
+        bounds = _cut(cost, nrow_wg) if tasks else np.zeros(nrow_wg + 1, dtype=np.int64)
+        if len(tasks) <= nrow_wg * lanes:  # one task at a time
+            for i in range(nrow_wg):
+                bounds[i + 1] = min(max(bounds[i + 1], len(tasks) - (nrow_wg - 1 - i) * lanes),
+                                    bounds[i] + lanes)
+        for i in range(nrow_wg):
+            voff = []
+            per_lane = [[] for _ in range(lanes)]
+            load = [0.0] * lanes
+            for t in sorted(range(bounds[i], bounds[i + 1]), key=lambda q: -cost[q]):
+                w = min(range(lanes), key=lambda q: load[q])
+                load[w] += cost[t]
+                per_lane[w].append(t)
+            for w in range(lanes):
+                mine = [_row_task(tasks[t], voff, mlist, diag_off) for t in per_lane[w]]
+                if any(m is None for m in mine):
+                    return None
+                for _ in range(per):
+                    rows += mine
+                    wave_ptr.append(len(rows))
+            lds_voff += voff
+            lds_ptr.append(len(lds_voff))
+    n = np.diff(lds_ptr)
+    n[ndwg:ndwg + nfwg] *= 2
+    plan = TeamPlan(
+        nteam=nteam, size=size, kp=kp, kd=kd, dgroups=dgroups, ndwg=ndwg,
+        nfwg=nfwg, pair_rows=pair_rows, nparts=DENSE_MAX * ndwg + len(light), dense_rows=list(dense),
+        lds_slots=int(n.max()), red_slots=red,
+        lds_ptr=np.asarray(lds_ptr, dtype=np.int32), lds_voff=np.asarray(lds_voff, dtype=np.int32),
+        wave_ptr=np.asarray(wave_ptr, dtype=np.int32),
+        rows=np.asarray(rows, dtype=np.int32).reshape(-1, 10),
+        mothers=np.asarray(mlist, dtype=np.int32).reshape(-1, 2),
+        dense_ptr=np.asarray(dptr, dtype=np.int32),
+        dense_ent=np.asarray(dent, dtype=np.int32).reshape(-1, 5),
+        fin=np.asarray(fin, dtype=np.int32).reshape(-1, 8),
+        fin_blk=np.asarray(fin_blk, dtype=np.int32).reshape(-1, 4))
+    return plan if plan.lds_bytes(fields) <= LDS_BYTES else None
+
+
+def _row_task(rows, voff, mlist, diag_off):
+    """Task of one or two rows: their values appended to ``voff``, their mothers to
+    ``mlist`` (those of both rows first)."""
+    head = []
+    for da, _, part in rows:
+        head.append((da, len(voff), part))
+        voff.append(diag_off + da * 64)
+    (a, ga, pa), (b, gb, pb) = (head + [(-1, 0, -1)])[:2]
+    vals = [{int(m): int(v) for m, _, _, v in q.tolist()} for _, q, _ in rows]
+    both = sorted(set(vals[0]) & set(vals[1])) if len(rows) == 2 else []
+    first = len(mlist)
+    for m in both:
+        mlist.append([m, len(voff)])
+        voff += [vals[0][m], vals[1][m]]
+    alone = [[m for m in sorted(v) if m not in both] for v in vals] + [[]]
+    for v, ms in zip(vals, alone):
+        for m in ms:
+            mlist.append([m, len(voff)])
+            voff.append(v[m])
+    if len(mlist) - first > 64:
+        return None
+    return [a, b, len(both), len(alone[0]), len(alone[1]), ga, gb, pa, pb, first]
+
+
+def _bounds(slots, parts):
+    """Contiguous ranges (starts, ends) of similar slot count."""
+    b = _cut(slots.astype(np.float64), parts)
+    return b[:-1], b[1:]
