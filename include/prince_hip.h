@@ -323,8 +323,9 @@ int32_t prh_etd2_stage(const prh_operator* op, const prh_schedule* sch, const pr
  * a team sum the dense rows over heavy mothers, the next nfwg finish the tail
  * rows one stage behind, the others own the heavy rows; no heavy row may read a
  * tail row.
- *   lds_ptr  [size + 1]: range of lds_voff that belongs to a rank; lds_voff:
- *            value offset (inside a window) of each 64-double LDS slot.
+ *   lds_ptr  [size + 1]: range of lds_voff that belongs to a rank; lds_voff
+ *            [][2]: value offset (inside a window) of each 64-double LDS slot, and
+ *            the bins it is shifted up by (the first dense row's diagonal o by o).
  *   wave_ptr [size * 16 + 1]: tasks of each wave (pair_rows: the two waves 2 i and
  *            2 i + 1 of a rank list the same tasks and share their columns);
  *            rows [ntasks][10] = {row a, row b or -1, entries of both rows, of row
@@ -338,7 +339,7 @@ int32_t prh_etd2_stage(const prh_operator* op, const prh_schedule* sch, const pr
  *   dense_ptr [ndwg * dgroups + 1]: entries of each mother group (at most 64);
  *            dense_ent [][5] = {mother, slot, o_lo | nslot << 8} with slot and
  *            band repeated for the second dense row (nslot 0: no block; 0 <=
- *            o_lo, nslot <= 8, second row nslot <= 1).  The 16 waves form dgroups mother groups x 16 /
+ *            o_lo, o_lo + nslot <= 8; second row o_lo 0, nslot <= 1).  The 16 waves form dgroups mother groups x 16 /
  *            dgroups column groups of kd pairs; rank g's sum of dense
  *            row r is partial 2 g + r.
  *   fin      [nfin][8] = {row, diagonal's slot, first partial, stride, partials,
@@ -360,6 +361,8 @@ typedef struct prh_team {
   int32_t lds_slots; /* slots of the largest rank, finishing ranks counted twice */
   int32_t red_slots; /* LDS rows of the mother groups' partial sums */
   int32_t pair_rows; /* tasks hold row pairs */
+  int32_t coef_slots; /* LDS rows of staged source coefficients: >= J x columns of a team / 64 */
+  int32_t pad_;
   const int32_t* lds_ptr;
   const int32_t* lds_voff;
   const int32_t* wave_ptr;
@@ -377,7 +380,7 @@ typedef struct prh_team {
  * prh_etd2_steps (d = 64, no EM sector; recording as there) for operators whose
  * rows are diagonal blocks except at most two dense rows.  op->tasks and
  * op->blocks are not used.  The launch needs nteam * size CUs with
- * 8 * 64 * (11 + red_slots + lds_slots) bytes of LDS each (two fields: 13 and
+ * 8 * 64 * (11 + 2 coef_slots + red_slots + lds_slots) bytes of LDS each (two fields: 13 and
  * twice lds_slots).  Returns 2 (nothing launched) when the device cannot hold
  * that grid or the stream is capturing. */
 int32_t prh_team_march(const prh_operator* op, const prh_schedule* sch, const prh_state* st,

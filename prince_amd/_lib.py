@@ -256,6 +256,8 @@ class PrhTeam(ctypes.Structure):
         ("lds_slots", _i32),
         ("red_slots", _i32),
         ("pair_rows", _i32),
+        ("coef_slots", _i32),
+        ("pad_", _i32),
         ("lds_ptr", _p),
         ("lds_voff", _p),
         ("wave_ptr", _p),

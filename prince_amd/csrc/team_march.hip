@@ -159,9 +159,11 @@ struct TeamLds {
   double* cst;  // [9][64]
   double* rp;   // [2][fields][64] pair-production rate of the window
   double* red;  // [16 waves][2][64 lanes][2] partial sums of the dense rows' mother groups
+  double* coef; // [2][coefs] source coefficients of the team's columns, this step's
+                // and the next one's
   double* val;  // [fields][slots][64] coupling values of the window (finishing
                 // workgroups: two such sets, they also need the window before)
-  int slots;
+  int slots, coefs;
 };
 __device__ __forceinline__ d2 lds2(const double* base, int slot, int bin) {
   return *reinterpret_cast<const d2*>(base + slot * WAVE + bin);
@@ -190,13 +192,28 @@ struct TeamState {
   int phalf;                    // bytes of one stage's partials
 };
 
+// Source coefficients norm evolution(z) of a step for the team's nc columns from c0:
+// read a step ahead into a register by coef_ahead, into LDS by coef_stage after
+// the step's work, so that no stage waits for memory it never touched before (about
+// 2 us; 5 us per stage on the rows with sources at K = 64).
+__device__ __forceinline__ double coef_ahead(COp& op, CSch& sch, int step, int c0, int nc) {
+  if (!(op.flags & PRH_F_INJECTION)) return 0.0;  // uniform
+  const int J = op.nsrc;
+  const int i = (int)threadIdx.x < J * nc ? threadIdx.x : J * nc - 1;
+  const int j = i / nc;
+  return sch.src_coef[((int64_t)step * J + j) * op.K + c0 + (i - j * nc)];
+}
+__device__ __forceinline__ void coef_stage(const TeamLds& L, int step, double c) {
+  if ((int)threadIdx.x < L.coefs) L.coef[(step & 1) * L.coefs + threadIdx.x] = c;
+}
+
 // Source sums sum_j norm evolution(z) g_j of source slot sslot for the pairs from k0.
 template <int KP>
-__device__ __forceinline__ void team_source(COp& op, CSch& sch,
-                                            int step, int sslot, int k0, int kend, const Lane& n,
+__device__ __forceinline__ void team_source(COp& op, const TeamLds& L, int step,
+                                            int sslot, int c0, int k0, int kend, const Lane& n,
                                             d2 (&src)[KP]) {
   if (sslot < 0) return;
-  const int J = op.nsrc, K = op.K;
+  const int J = op.nsrc, K = op.K, nc = kend - c0;
   for (int j = 0; j < J; ++j) {
     d2 g[KP];
     double c[KP];
@@ -206,7 +223,7 @@ __device__ __forceinline__ void team_source(COp& op, CSch& sch,
       const int k = kk < kend ? kk : kend - 1;
       g[p] = *reinterpret_cast<const d2*>(op.src_grid +
                                           (((int64_t)sslot * J + j) * K + k) * WAVE + n.bin);
-      c[p] = sch.src_coef[((int64_t)step * J + j) * K + k];
+      c[p] = L.coef[(step & 1) * L.coefs + j * nc + k - c0];
     }
 #pragma unroll
     for (int p = 0; p < KP; ++p) src[p] = (j == 0) ? c[p] * g[p] : src[p] + c[p] * g[p];
@@ -236,9 +253,13 @@ __device__ __forceinline__ void bin_factors(int s2, double kadia, double pscale,
 struct RowFactors {
   d2 kap, e, phi;
 };
-__device__ __forceinline__ d2 from_halves(const Lane& n, double v) {
-  const double o = __shfl_xor(v, 32, WAVE);
-  return n.half ? d2{o, v} : d2{v, o};
+// {lane l's value, lane l + 32's value} in both halves (v_permlane32_swap: no LDS)
+__device__ __forceinline__ d2 from_halves(double v) {
+  const u32x2 b = __builtin_bit_cast(u32x2, v);
+  const auto lo = __builtin_amdgcn_permlane32_swap(b.x, b.x, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(b.y, b.y, false, false);
+  return d2{__builtin_bit_cast(double, u32x2{lo[0], hi[0]}),
+            __builtin_bit_cast(double, u32x2{lo[1], hi[1]})};
 }
 template <bool TWO>
 __device__ __forceinline__ RowFactors row_factors(COp& op, const TeamLds& L,
@@ -251,9 +272,9 @@ __device__ __forceinline__ RowFactors row_factors(COp& op, const TeamLds& L,
     double kap, e, phi;
     bin_factors(s2, si.hadia * L.cst[7 * WAVE + bin], pscale, L.rp[bin], L.val[slot * WAVE + bin],
                 L.cst[8 * WAVE + bin], si.dl, si.h, pdiff, kap, e, phi);
-    f.kap = from_halves(n, kap);
-    f.e = from_halves(n, e);
-    f.phi = from_halves(n, phi);
+    f.kap = from_halves(kap);
+    f.e = from_halves(e);
+    f.phi = from_halves(phi);
   } else {
     const double s = op.escale[k];
 #pragma unroll 1
@@ -427,8 +448,9 @@ __device__ __forceinline__ void team_rows(COp& op, CSch& sch,
                                           CSt& st, const TeamState& T,
                                           const TeamLds& L, const StepIn& si, int s2,
                                           const RowTask& rt, const RowFactors& fa,
-                                          const RowFactors& fb, int k0, int kend, const Lane& n) {
-  constexpr int U = 4;
+                                          const RowFactors& fb, int c0, int k0, int kend,
+                                          const Lane& n) {
+  constexpr int U = TWO ? 2 : 4;
   const auto y = s2 ? T.a : T.x;
   d2 acc[2][KP], accE[2][KP], xo[KP], fo[KP];
 #pragma unroll
@@ -465,7 +487,7 @@ __device__ __forceinline__ void team_rows(COp& op, CSch& sch,
       d2 src[KP];
 #pragma unroll
       for (int p = 0; p < KP; ++p) src[p] = d2{0.0, 0.0};
-      team_source<KP>(op, sch, si.step, rc.sslot, k0, kend, n, src);
+      team_source<KP>(op, L, si.step, rc.sslot, c0, k0, kend, n, src);
       team_epilogue<KP, TWO, REC>(op, st, T, L, si, s2, f0, rc, da, diag, k0, kend, n, acc[0], xo,
                                   fo, src);
     }
@@ -524,7 +546,7 @@ __device__ __forceinline__ void team_row1(COp& op, CSch& sch,
     }
     if (e == 0 && rt.part_a < 0) {
       own_loads<1>(T, s2, rt.a, k0, n, xo, fo);
-      team_source<1>(op, sch, si.step, rt.ca.sslot, k0, kend, n, src);
+      team_source<1>(op, L, si.step, rt.ca.sslot, k0, k0, kend, n, src);
       if (!TWO) f0 = row_factors<false>(op, L, si, s2, rt.ca.pscale, rt.diag_a, k0, n);
     }
 #pragma unroll
@@ -556,8 +578,8 @@ __device__ __forceinline__ void team_row1(COp& op, CSch& sch,
     acc[0] = acc[0] + op.escale[k < kend ? k : kend - 1] * accE;
   }
   if (SPLIT) {
-    acc[0].x += __shfl_xor(acc[0].x, 32, WAVE);
-    acc[0].y += __shfl_xor(acc[0].y, 32, WAVE);
+    const d2 sx = from_halves(acc[0].x), sy = from_halves(acc[0].y);
+    acc[0] = d2{sx.x + sx.y, sy.x + sy.y};
   }
   if (rt.part_a >= 0) {
     if (k0 + n.half < kend)
@@ -602,7 +624,8 @@ template <bool TWO, bool REC>
 __device__ __forceinline__ void team_finish(COp& op, CSch& sch,
                                             CSt& st, const TeamState& T,
                                             const TeamLds& L, const StepIn& si, int stage,
-                                            const FinTask& ft, int k0, int kend, const Lane& n) {
+                                            const FinTask& ft, int c0, int k0, int kend,
+                                            const Lane& n) {
   constexpr int U = 6, UB = 5;
   const auto y = stage ? T.a : T.x;
   const int pbase = stage ? T.phalf : 0;
@@ -617,7 +640,7 @@ __device__ __forceinline__ void team_finish(COp& op, CSch& sch,
   for (int u = 0; u < U; ++u)
     if (u < ft.pn) pv[u] = pload<SC1>(T.part, n.off, pbase + (ft.p0 + u * ft.pstep) * T.pb + cb);
   own_loads<1>(T, stage, ft.da, k0, n, xo, fo);
-  team_source<1>(op, sch, si.step, ft.rc.sslot, k0, kend, n, src);
+  team_source<1>(op, L, si.step, ft.rc.sslot, c0, k0, kend, n, src);
   // one part after the other: all of them in flight at once would spill
   __builtin_amdgcn_sched_barrier(0);
   for (int g = 0;;) {
@@ -641,20 +664,23 @@ __device__ __forceinline__ void team_finish(COp& op, CSch& sch,
       const int band = __builtin_amdgcn_readlane(ft.band, b + u);
       const int sl = __builtin_amdgcn_readlane(ft.sl, b + u);
       const int ns = band >> 8, ol = band & 255;
-      d2 mc[8], me[TWO ? 8 : 1];
-#pragma unroll
-      for (int s2 = 0; s2 < 8; ++s2) {
-        const int s = sl + (s2 < ns ? s2 : ns - 1);
-        mc[s2] = lds2(L.val, s, n.bin);
-        if (TWO) me[TWO ? s2 : 0] = lds2(L.val, L.slots + s, n.bin);
-      }
       for (int o = 0; o < ol; ++o) xv[0] = shift_bin(n, xv[0]);
+#pragma unroll 1
+      for (int s0 = 0; s0 < ns; s0 += 4) {
+        d2 mc[4], me[TWO ? 4 : 1];
 #pragma unroll
-      for (int s2 = 0; s2 < 8; ++s2) {
-        if (s2 < ns) {
-          accB += mc[s2] * xv[0];
-          if (TWO) accE += me[TWO ? s2 : 0] * xv[0];
-          xv[0] = shift_bin(n, xv[0]);
+        for (int s2 = 0; s2 < 4; ++s2) {
+          const int s = sl + (s0 + s2 < ns ? s0 + s2 : ns - 1);
+          mc[s2] = lds2(L.val, s, n.bin);
+          if (TWO) me[TWO ? s2 : 0] = lds2(L.val, L.slots + s, n.bin);
+        }
+#pragma unroll
+        for (int s2 = 0; s2 < 4; ++s2) {
+          if (s0 + s2 < ns) {
+            accB += mc[s2] * xv[0];
+            if (TWO) accE += me[TWO ? s2 : 0] * xv[0];
+            xv[0] = shift_bin(n, xv[0]);
+          }
         }
       }
 #pragma unroll
@@ -681,77 +707,70 @@ struct DenseDesc {
 };
 
 // Partial sums of the dense rows over this wave's mothers (entries 0 .. ne-1 of
-// its descriptor lanes) for the KP pairs of right-hand sides from k0.
+// its descriptor lanes) for the KP pairs of right-hand sides from k0.  The band row
+// keeps one accumulator per diagonal, aligned with the mother's bins (its values
+// are stored shifted by their diagonal, load_window): z_o[j] += v_o[j - o] x[j], and
+// y[i] = sum_o z_o[i + o] once per stage -- 18 products per mother and pair
+// instead of 18 and 7 shifts of 4 instructions.
 template <int KP, bool TWO>
-__device__ __forceinline__ void dense_partial(COp& op, __amdgpu_buffer_rsrc_t y,
-                                              int pb, const TeamLds& L, const DenseDesc& dd, int ne,
-                                              int k0, int kend, const Lane& n,
-                                              d2 (&acc)[TDENSE][KP]) {
+__device__ __forceinline__ void dense_partial(COp& op, __amdgpu_buffer_rsrc_t y, int pb,
+                                              const TeamLds& L, const DenseDesc& dd, int ne, int k0,
+                                              int kend, const Lane& n, d2 (&acc)[TDENSE][KP]) {
   constexpr int U = 2;
-  d2 accE[TDENSE][KP];
+  d2 z[8][KP], w[KP];
+  double sc[KP];
 #pragma unroll
-  for (int p = 0; p < KP; ++p) acc[0][p] = acc[1][p] = accE[0][p] = accE[1][p] = d2{0.0, 0.0};
+  for (int p = 0; p < KP; ++p) {
+#pragma unroll
+    for (int o = 0; o < 8; ++o) z[o][p] = d2{0.0, 0.0};
+    w[p] = d2{0.0, 0.0};
+    const int k = k0 + 2 * p + n.half;
+    sc[p] = TWO ? op.escale[k < kend ? k : kend - 1] : 0.0;
+  }
   const int cb = k0 * (WAVE * 8);
   for (int e = 0; e < ne; e += U) {
     d2 xv[U][KP];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (e + u < ne) {
-        const int po = __builtin_amdgcn_readlane(dd.mo, e + u) * pb + cb;
+      const int po = __builtin_amdgcn_readlane(dd.mo, (e + u) & 63) * pb + cb;
+      const int vo = e + u < ne ? n.off : 0x7ffffff0;  // past the end: zeros
 #pragma unroll
-        for (int p = 0; p < KP; ++p) xv[u][p] = pload<SC1>(y, n.off, po + p * (2 * WAVE * 8));
-      }
+      for (int p = 0; p < KP; ++p) xv[u][p] = pload<SC1>(y, vo, po + p * (2 * WAVE * 8));
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (e + u < ne) {
-        // the second row (He-4: one diagonal) before the band moves the panel
+      if (e + u >= ne) break;
+      const int s0 = __builtin_amdgcn_readlane(dd.s0, e + u);
+      const int b0 = __builtin_amdgcn_readlane(dd.b0, e + u);
+      const int s1 = __builtin_amdgcn_readlane(dd.s1, e + u);
+      const int b1 = __builtin_amdgcn_readlane(dd.b1, e + u);
+      const int ns = b0 >> 8, ol = b0 & 255;
+      // the diagonals in order; a row with fewer or later ones skips the others
 #pragma unroll
-        for (int r = TDENSE - 1; r >= 0; --r) {
-          const int ss = __builtin_amdgcn_readlane(r ? dd.s1 : dd.s0, e + u);
-          const int bd = __builtin_amdgcn_readlane(r ? dd.b1 : dd.b0, e + u);
-          const int ns = bd >> 8, ol = bd & 255;
-          if (ns == 0) continue;
-          d2 xs[KP], mc[8], me[TWO ? 8 : 1];
-          // the values first (no wait per diagonal), then products and shifts
+      for (int o = 0; o < 8; ++o) {
+        if (o >= ol && o < ol + ns) {
+          const d2 mc = lds2(L.val, s0 + o - ol, n.bin);
+          const d2 me = TWO ? lds2(L.val, L.slots + s0 + o - ol, n.bin) : d2{0.0, 0.0};
 #pragma unroll
-          for (int s2 = 0; s2 < 8; ++s2) {
-            const int sl = ss + (s2 < ns ? s2 : ns - 1);
-            if (r == 0 || s2 == 0) mc[s2] = lds2(L.val, sl, n.bin);
-            if (TWO && (r == 0 || s2 == 0)) me[TWO ? s2 : 0] = lds2(L.val, L.slots + sl, n.bin);
-          }
-#pragma unroll
-          for (int p = 0; p < KP; ++p) xs[p] = xv[u][p];
-          for (int o = 0; o < ol; ++o) {
-#pragma unroll
-            for (int p = 0; p < KP; ++p) xs[p] = shift_bin(n, xs[p]);
-          }
-#pragma unroll
-          for (int s2 = 0; s2 < (r == 0 ? 8 : 1); ++s2) {
-            if (s2 < ns) {
-#pragma unroll
-              for (int p = 0; p < KP; ++p) {
-                acc[r][p] += mc[s2] * xs[p];
-                if (TWO) accE[r][p] += me[TWO ? s2 : 0] * xs[p];
-              }
-              if (s2 + 1 < ns) {
-#pragma unroll
-                for (int p = 0; p < KP; ++p) xs[p] = shift_bin(n, xs[p]);
-              }
-            }
-          }
+          for (int p = 0; p < KP; ++p) z[o][p] += (TWO ? mc + sc[p] * me : mc) * xv[u][p];
         }
+      }
+      if (b1 >> 8) {
+        const d2 mc = lds2(L.val, s1, n.bin);
+        const d2 me = TWO ? lds2(L.val, L.slots + s1, n.bin) : d2{0.0, 0.0};
+#pragma unroll
+        for (int p = 0; p < KP; ++p) w[p] += (TWO ? mc + sc[p] * me : mc) * xv[u][p];
       }
     }
   }
-  if (TWO) {
+  // y = z_0 + shift(z_1 + shift(z_2 + ...)): seven shifts
 #pragma unroll
-    for (int p = 0; p < KP; ++p) {
-      const int k = k0 + 2 * p + n.half;
-      const double s = op.escale[k < kend ? k : kend - 1];
-      acc[0][p] += s * accE[0][p];
-      acc[1][p] += s * accE[1][p];
-    }
+  for (int p = 0; p < KP; ++p) {
+    d2 t = z[7][p];
+#pragma unroll
+    for (int o = 6; o >= 0; --o) t = z[o][p] + shift_bin(n, t);
+    acc[0][p] = t;
+    acc[1][p] = w[p];
   }
 }
 
@@ -795,6 +814,8 @@ __device__ __forceinline__ bool team_barrier(uint32_t* sub, uint32_t nsubwg, uin
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
   return *bad == 0;
 }
+// (One arrival word per workgroup, polled with one vector load, measured the same at
+// K = 1 and slower with more traffic: the pollers and writers share the lines.)
 
 __global__ void team_reset(uint32_t* sync) {
   for (int i = threadIdx.x; i < SY_WORDS; i += blockDim.x) sync[i] = 0;
@@ -833,13 +854,15 @@ __device__ __forceinline__ void load_window(COp& op, CTm& tm,
                                             const TeamLds& L, const TeamPos& P, int w) {
   const double* mv = op.mvals + (int64_t)w * op.mvals_stride;
   const double* me = TWO ? op.mvals_e + (int64_t)w * op.mvals_stride : nullptr;
-  const int* vo = tm.lds_voff + tm.lds_ptr[P.rank];
+  const int* vo = tm.lds_voff + 2 * cload(tm.lds_ptr + P.rank);
   const int lane = P.n.id;
 #pragma unroll 4
   for (int s = P.wv; s < L.slots; s += TWAVES) {
-    const int v = cload(vo + s) + lane;
-    L.val[s * WAVE + lane] = mv[v];
-    if (TWO) L.val[(L.slots + s) * WAVE + lane] = me[v];
+    // value offset of the slot and by how many bins it is stored shifted
+    const int v = cload(vo + 2 * s) + lane, sh = cload(vo + 2 * s + 1);
+    const int at = lane + sh < WAVE ? lane + sh : lane + sh - WAVE;  // the wrapped bins: zeros
+    L.val[s * WAVE + at] = lane + sh < WAVE ? mv[v] : 0.0;
+    if (TWO) L.val[(L.slots + s) * WAVE + at] = lane + sh < WAVE ? me[v] : 0.0;
   }
   if (P.wv == 0) {
     L.rp[lane] = op.rpair[(int64_t)w * WAVE + lane];
@@ -895,10 +918,16 @@ __device__ __forceinline__ void march_rows(CArgs* A, const TeamLds& L, const Tea
   if (t0 < t1) first = row_task(A->op, A->tm, t0, P.n.id, A->op.K * WAVE * 8);
   uint32_t epoch = 0;
   int wcur = -1;
+  const int nc = P.cend - P.c0;
+  coef_stage(L, k_begin, coef_ahead(A->op, A->sch, k_begin, P.c0, nc));
+  __syncthreads();
 #pragma unroll 1
   for (int p = 2 * k_begin; p < 2 * k_end; ++p) {
     CArgs* a = reread(A);
     const int s2 = p & 1, step = p >> 1;
+    const int nx = step + 1 < k_end ? step + 1 : step;
+    const bool ahead = s2 && P.wv * WAVE < L.coefs;
+    const double cn = ahead ? coef_ahead(a->op, a->sch, nx, P.c0, nc) : 0.0;
     if (s2 == 0) {
       const int w = cload(a->sch.win + step);
       if (w != wcur) {
@@ -926,9 +955,11 @@ __device__ __forceinline__ void march_rows(CArgs* A, const TeamLds& L, const Tea
         }
 #pragma unroll 1
         for (int k0 = P.c0 + 2 * KP * (P.wv & 1); k0 < P.cend; k0 += 4 * KP)
-          team_rows<KP, TWO, REC>(a->op, a->sch, a->st, T, L, si, s2, rt, fa, fb, k0, P.cend, P.n);
+          team_rows<KP, TWO, REC>(a->op, a->sch, a->st, T, L, si, s2, rt, fa, fb, P.c0, k0, P.cend,
+                                  P.n);
       }
     }
+    if (s2 && nx != step) coef_stage(L, nx, cn);  // complete behind the phase's barriers
     if (!next_phase(P, epoch)) return;
   }
 }
@@ -1026,10 +1057,14 @@ __device__ __forceinline__ void march_finish(CArgs* A, const TeamLds& L, const T
   // phase p finishes stage p - 1: stage 2 of the step before, or stage 1 of its
   // own; sbuf: the value set of that stage
   int sbuf = 0;
+  const int nc = P.cend - P.c0;
 #pragma unroll 1
   for (int p = 2 * k_begin; p <= 2 * k_end; ++p) {
     CArgs* a = reread(A);
     const int s2 = (p & 1) ^ 1;
+    // the step that its next phase begins to finish
+    const bool ahead = s2 && p < 2 * k_end && P.wv * WAVE < L.coefs;
+    const double cn = ahead ? coef_ahead(a->op, a->sch, p >> 1, P.c0, nc) : 0.0;
     sbuf = buf;
     if (s2 && p < 2 * k_end) {
       const int w = cload(a->sch.win + (p >> 1));
@@ -1050,10 +1085,11 @@ __device__ __forceinline__ void march_finish(CArgs* A, const TeamLds& L, const T
         const int f = it / groups;
         FinTask ft = first;
         if (it != it0) ft = fin_task(a->op, a->tm, f, P.n.id);
-        team_finish<TWO, REC>(a->op, a->sch, a->st, T, Q, si, s2, ft, P.c0 + (it - f * groups) * 2,
-                              P.cend, P.n);
+        team_finish<TWO, REC>(a->op, a->sch, a->st, T, Q, si, s2, ft, P.c0,
+                              P.c0 + (it - f * groups) * 2, P.cend, P.n);
       }
     }
+    if (s2 && p < 2 * k_end) coef_stage(L, p >> 1, cn);
     if (p < 2 * k_end && !next_phase(P, epoch)) return;
   }
 }
@@ -1079,7 +1115,9 @@ __global__ void __launch_bounds__(TTHREADS) team_march(TeamArgs) {
   L.cst = lds;
   L.rp = L.cst + TCONST * WAVE;
   L.red = L.rp + (TWO ? 4 : 2) * WAVE;
-  L.val = L.red + A->tm.red_slots * WAVE;
+  L.coef = L.red + A->tm.red_slots * WAVE;
+  L.coefs = A->tm.coef_slots * WAVE;
+  L.val = L.coef + 2 * L.coefs;
   L.slots = cload(A->tm.lds_ptr + P.rank + 1) - cload(A->tm.lds_ptr + P.rank);
   for (int i = threadIdx.x; i < WAVE; i += TTHREADS) {
     for (int o = 0; o < 7; ++o)
@@ -1123,7 +1161,7 @@ int32_t launch_team_rec(const prh_operator& op, const prh_schedule& sch, const p
                         const prh_team& tm, int k_begin, int k_end, hipStream_t s) {
   const void* fn = reinterpret_cast<const void*>(&team_march<R, KP, KD, TWO, REC, SPLIT>);
   const size_t lds =
-      8 * WAVE * (size_t)(TCONST + (TWO ? 4 : 2) + tm.red_slots + tm.lds_slots * (TWO ? 2 : 1));
+      8 * WAVE * (size_t)(TCONST + (TWO ? 4 : 2) + 2 * tm.coef_slots + tm.red_slots + tm.lds_slots * (TWO ? 2 : 1));
   hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return prh_internal::check(e, "prh_team_march: dynamic LDS");
   TeamArgs ta{op, sch, st, tm, k_begin, k_end};
@@ -1199,6 +1237,8 @@ extern "C" int32_t prh_team_march(const prh_operator* op, const prh_schedule* sc
       (tm->dgroups < TDENSE || tm->kd != 1 || (TWAVES / tm->dgroups) * 2 < ncmax ||
        tm->red_slots < TWAVES * TDENSE * 2))
     return error("prh_team_march: mother groups need one column pass and their LDS rows");
+  if (op->nsrc * ncmax > TTHREADS || op->nsrc * ncmax > WAVE * tm->coef_slots)
+    return error("prh_team_march: more source coefficients per team than staged");
   if (k_begin == k_end) return 0;
   hipStream_t s = (hipStream_t)stream;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;

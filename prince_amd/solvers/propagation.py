@@ -833,7 +833,7 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
         }
         self._plan["team"] = None
         if self.team_march_for(K) and em_struct is None:
-            self._plan["team"] = self._team_setup(lay, dv, K, 2 if two else 1)
+            self._plan["team"] = self._team_setup(lay, dv, K, 2 if two else 1, J)
         if self._plan["team"] is None:
             self._capture_steps(self._plan)
         self.refresh_zs = zs
@@ -848,18 +848,18 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
     #: team plans (host tables on the device, read only) kept per layout
     TEAM_PLANS_KEPT = 8
 
-    def _team_setup(self, lay, dv, K, fields):
+    def _team_setup(self, lay, dv, K, fields, nsrc):
         """Team march of this plan (``prh_team``): the layout's tables for K
         columns, and the plan's own partials and sync words.  None when the
         operator or the device does not fit it."""
         torch = _torch()
         wl = lay["layout"]
         args = getattr(self, "_tuned", {}).get(("team_args", K), {})
-        key = (K, fields, tuple(sorted(args.items())))
+        key = (K, fields, nsrc, tuple(sorted(args.items())))
         plans = lay.setdefault("team", {})
         if key not in plans:
             tp = team_plan.build_team(wl.blocks, wl.fwd.brow_ptr, wl.nspec, wl.d, wl.diag_off, K,
-                                      fields, **args)
+                                      fields, nsrc, **args)
             names = ("lds_ptr", "lds_voff", "wave_ptr", "rows", "mothers", "dense_ptr",
                      "dense_ent", "fin", "fin_blk")
             tables = None if tp is None else {
@@ -879,7 +879,7 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
             nteam=tp.nteam, size=tp.size, kp=tp.kp, kd=tp.kd, dgroups=tp.dgroups, ndwg=tp.ndwg,
             nfwg=tp.nfwg, nfin=tp.fin.shape[0], nparts=tp.nparts,
             lds_slots=tp.lds_slots, red_slots=tp.red_slots,
-            pair_rows=int(tp.pair_rows),
+            pair_rows=int(tp.pair_rows), coef_slots=tp.coef_slots, pad_=0,
             **{n: t.data_ptr() for n, t in b.items()})
         return {"struct": tm, "bufs": b, "plan": tp}
 

@@ -45,6 +45,7 @@ class TeamPlan:
     dense_rows: list
     lds_slots: int
     red_slots: int
+    coef_slots: int
     lds_ptr: np.ndarray
     lds_voff: np.ndarray
     wave_ptr: np.ndarray
@@ -56,7 +57,7 @@ class TeamPlan:
     fin_blk: np.ndarray
 
     def lds_bytes(self, fields):
-        return 512 * (CONST_SLOTS + 2 * fields + self.red_slots + fields * self.lds_slots)
+        return 512 * (CONST_SLOTS + 2 * fields + 2 * self.coef_slots + self.red_slots + fields * self.lds_slots)
 
 
 def dense_tiling(nc):
@@ -102,10 +103,12 @@ def tail_rows(blocks, ptr, nspec):
     return dense, sorted(tail)
 
 
-def build_team(blocks, brow_ptr, nspec, d, diag_off, K, fields=1, size=None, ndwg=None, nfwg=None):
+def build_team(blocks, brow_ptr, nspec, d, diag_off, K, fields=1, nsrc=1, size=None, ndwg=None,
+               nfwg=None):
     """Team plan of an operator for K right-hand sides, or None when its rows do
     not fit the march (d != 64, more than two dense rows, bands left of the
-    diagonal or wider than 8, a long tail, values beyond the LDS)."""
+    diagonal or wider than 8, a long tail, values beyond the LDS, more source
+    coefficients per team than threads)."""
     if d != 64 or nspec < 1 or nspec * K * 512 > 0x7FFFFFFF:
         return None
     blocks = np.asarray(blocks, dtype=np.int64).reshape(-1, 4)
@@ -115,25 +118,30 @@ def build_team(blocks, brow_ptr, nspec, d, diag_off, K, fields=1, size=None, ndw
         return None
     # the second dense row is the one of single diagonals
     dense.sort(key=lambda da: -int(blocks[ptr[da]:ptr[da + 1], 2].max()))
-    if len(dense) == 2 and blocks[ptr[dense[1]]:ptr[dense[1] + 1], 2].max() > 1:
-        return None
+    if len(dense) == 2:
+        b = blocks[ptr[dense[1]]:ptr[dense[1] + 1]]
+        if np.any(b[:, 2] > 1) or np.any(b[:, 1] != 0):
+            return None
     for da in dense:
         b = blocks[ptr[da]:ptr[da + 1]]
-        if np.any(b[:, 1] < 0) or np.any(b[:, 1] > 255) or np.any(b[:, 2] > BAND_MAX):
+        if np.any(b[:, 1] < 0) or np.any(b[:, 1] + b[:, 2] > BAND_MAX):
             return None
     sizes = [1] if len(tail) == nspec else [size] if size is not None else [32, 64, 128, 256]
     for s in sizes:
-        plan = _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, s, ndwg, nfwg)
+        plan = _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, s, ndwg, nfwg)
         if plan is not None:
             return plan
     return None
 
 
-def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, size, ndwg, nfwg):
+def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, size, ndwg, nfwg):
     nteam = min(8, CUS // size)
     nc = -(-K // nteam)
     kd, dgroups = dense_tiling(nc)
     pair_rows, kp = row_tiling(nc)
+    if nsrc * nc > 64 * WAVES:
+        return None
+    coef = -(-nsrc * nc // 64)
     tset = set(tail)
     # dense entries: one per heavy mother, both rows' blocks
     ent = {}
@@ -145,7 +153,7 @@ def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, size, ndwg, nfw
     mothers = sorted(ent)
     eslots = np.array([sum(q[1] for q in ent[m]) for m in mothers], dtype=np.int64)
     red = WAVES * DENSE_MAX * 2 if (mothers and dgroups > 1) else 0
-    budget = (LDS_BYTES // 512 - CONST_SLOTS - 2 * fields - red) // fields
+    budget = (LDS_BYTES // 512 - CONST_SLOTS - 2 * fields - 2 * coef - red) // fields
     if not mothers:
         ndwg = 0
     elif ndwg is None:
@@ -171,7 +179,8 @@ def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, size, ndwg, nfw
                 q = []
                 for ol, ns, vo in ent[mothers[e]]:
                     q += [len(voff) if ns else 0, ol | ns << 8]
-                    voff += [vo + 64 * s for s in range(ns)]
+                    # diagonal o sits o bins up, in line with the mother's bins
+                    voff += [(vo + 64 * s, ol + s) for s in range(ns)]
                 slot[e] = q
             for g in range(dgroups):  # mother groups: contiguous, similar counts
                 lo, hi = a + (b - a) * g // dgroups, a + (b - a) * (g + 1) // dgroups
@@ -187,12 +196,12 @@ def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, size, ndwg, nfw
     for da in tail:
         first = len(fin_blk)
         slot = len(fvoff)
-        fvoff.append(diag_off + da * 64)
+        fvoff.append((diag_off + da * 64, 0))
         for v in range(int(ptr[da]), int(ptr[da + 1])):
             mo, ol, ns, vo = (int(q) for q in blocks[v])
             if mo in tset:
                 fin_blk.append([mo, len(fvoff), ol, ns])
-                fvoff += [vo + 64 * s for s in range(ns)]
+                fvoff += [(vo + 64 * s, 0) for s in range(ns)]
         p0, pstep, pn = ((dense.index(da), DENSE_MAX, ndwg) if da in dense
                          else (DENSE_MAX * ndwg + light.index(da), 1, 1))
         fin.append([da, slot, p0, pstep, pn, first, len(fin_blk) - first, 0])
@@ -209,7 +218,9 @@ def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, size, ndwg, nfw
     per = 2 if pair_rows else 1
     lanes = WAVES // per  # tasks that run at once in a workgroup
     tasks = [rowlist[i:i + per] for i in range(0, len(rowlist), per)]
-    cost = np.array([sum(8.0 + len(b) for _, b, _ in t) for t in tasks])
+    # a mother panel loaded costs 1, a row's own state, factors and epilogue about 5
+    cost = np.array([5.0 * len(t) + len(set(m for _, b, _ in t for m in b[:, 0].tolist()))
+                     for t in tasks])
     if nrow_wg:
         bounds = _cut(cost, nrow_wg) if tasks else np.zeros(nrow_wg + 1, dtype=np.int64)
         if len(tasks) <= nrow_wg * lanes:  # one task at a time
@@ -238,8 +249,8 @@ def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, size, ndwg, nfw
     plan = TeamPlan(
         nteam=nteam, size=size, kp=kp, kd=kd, dgroups=dgroups, ndwg=ndwg,
         nfwg=nfwg, pair_rows=pair_rows, nparts=DENSE_MAX * ndwg + len(light), dense_rows=list(dense),
-        lds_slots=int(n.max()), red_slots=red,
-        lds_ptr=np.asarray(lds_ptr, dtype=np.int32), lds_voff=np.asarray(lds_voff, dtype=np.int32),
+        lds_slots=int(n.max()), red_slots=red, coef_slots=coef,
+        lds_ptr=np.asarray(lds_ptr, dtype=np.int32), lds_voff=np.asarray(lds_voff, dtype=np.int32).reshape(-1, 2),
         wave_ptr=np.asarray(wave_ptr, dtype=np.int32),
         rows=np.asarray(rows, dtype=np.int32).reshape(-1, 10),
         mothers=np.asarray(mlist, dtype=np.int32).reshape(-1, 2),
@@ -256,19 +267,19 @@ def _row_task(rows, voff, mlist, diag_off):
     head = []
     for da, _, part in rows:
         head.append((da, len(voff), part))
-        voff.append(diag_off + da * 64)
+        voff.append((diag_off + da * 64, 0))
     (a, ga, pa), (b, gb, pb) = (head + [(-1, 0, -1)])[:2]
     vals = [{int(m): int(v) for m, _, _, v in q.tolist()} for _, q, _ in rows]
     both = sorted(set(vals[0]) & set(vals[1])) if len(rows) == 2 else []
     first = len(mlist)
     for m in both:
         mlist.append([m, len(voff)])
-        voff += [vals[0][m], vals[1][m]]
+        voff += [(vals[0][m], 0), (vals[1][m], 0)]
     alone = [[m for m in sorted(v) if m not in both] for v in vals] + [[]]
     for v, ms in zip(vals, alone):
         for m in ms:
             mlist.append([m, len(voff)])
-            voff.append(v[m])
+            voff.append((v[m], 0))
     if len(mlist) - first > 64:
         return None
     return [a, b, len(both), len(alone[0]), len(alone[1]), ga, gb, pa, pb, first]

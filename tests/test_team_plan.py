@@ -41,7 +41,7 @@ def test_plan_reproduces_the_operator(layouts, name, K, fields, size):
     assert p is not None and p.nteam * p.size <= team.CUS
     assert p.lds_bytes(fields) <= team.LDS_BYTES
     assert p.lds_ptr.size == p.size + 1 and p.wave_ptr.size == p.size * team.WAVES + 1
-    assert np.all((p.lds_voff >= 0) & (p.lds_voff + 64 <= vals.size))
+    assert np.all((p.lds_voff[:, 0] >= 0) & (p.lds_voff[:, 0] + 64 <= vals.size))
     x = np.random.default_rng(3).standard_normal((nspec, 64))
     got = np.full((nspec, 64), np.nan)
     diag = np.full((nspec, 64), np.nan)
@@ -49,7 +49,10 @@ def test_plan_reproduces_the_operator(layouts, name, K, fields, size):
     tail = set(p.fin[:, 0].tolist())
     assert p.fin.shape[0] == len(tail) and set(p.dense_rows) <= tail
     for rank in range(p.size):
-        lds = [vals[v:v + 64] for v in p.lds_voff[p.lds_ptr[rank]:p.lds_ptr[rank + 1]]]
+        lds = []
+        for v, sh in p.lds_voff[p.lds_ptr[rank]:p.lds_ptr[rank + 1]]:
+            assert sh == 0 or rank < p.ndwg
+            lds.append(np.concatenate([np.zeros(sh), vals[v:v + 64 - sh]]))
         mult = 2 if p.ndwg <= rank < p.ndwg + p.nfwg else 1
         assert mult * len(lds) <= p.lds_slots
         if rank < p.ndwg:
@@ -58,8 +61,8 @@ def test_plan_reproduces_the_operator(layouts, name, K, fields, size):
             for mo, s0, b0, s1, b1 in p.dense_ent[e0:e1]:
                 assert mo not in tail
                 for r, (s, b) in enumerate(((s0, b0), (s1, b1))):
-                    for i in range(b >> 8):
-                        part[2 * rank + r] += lds[s + i] * _shift(x[mo], (b & 255) + i)
+                    for i in range(b >> 8):  # the value in the mother's bins
+                        part[2 * rank + r] += _shift(lds[s + i] * x[mo], (b & 255) + i)
         if rank < p.ndwg + p.nfwg:
             assert p.wave_ptr[rank * team.WAVES] == p.wave_ptr[(rank + 1) * team.WAVES]
             continue
@@ -89,7 +92,7 @@ def test_plan_reproduces_the_operator(layouts, name, K, fields, size):
                     got[da], diag[da] = s, lds[dg]
     if p.nfwg:  # every finishing workgroup holds the same slots
         r = p.ndwg
-        fl = [vals[v:v + 64] for v in p.lds_voff[p.lds_ptr[r]:p.lds_ptr[r + 1]]]
+        fl = [vals[v:v + 64] for v, _ in p.lds_voff[p.lds_ptr[r]:p.lds_ptr[r + 1]]]
         for k in range(r, r + p.nfwg):
             assert np.array_equal(p.lds_voff[p.lds_ptr[k]:p.lds_ptr[k + 1]],
                                   p.lds_voff[p.lds_ptr[r]:p.lds_ptr[r + 1]])
@@ -131,3 +134,5 @@ def test_operators_outside_the_march_are_refused():
     chain = np.array([[1, 0, 8, 0]] + [[i - 1, 0, 1, 64 * i] for i in range(1, 40)])
     assert team.build_team(chain, np.arange(41), 40, 64, 0, 1) is None  # every row reads the tail
     assert team.build_team(diag, ptr, 1, 64, 0, 5_000_000) is None  # state beyond 2 GiB
+    assert team.build_team(diag, ptr, 1, 64, 0, 64, nsrc=128) is not None
+    assert team.build_team(diag, ptr, 1, 64, 0, 64, nsrc=129) is None  # coefficients per team
