@@ -374,6 +374,13 @@ typedef struct prh_team {
   const int32_t* fin_blk;
   double* dpart;
   uint32_t* sync;
+  /* EM sector (NULL: none): the march stores em_w[t - em_first][k][64] = sum_s
+   * cbh[s] x[s][k] of the state after each step t of the range.  The dense
+   * entries then cover every heavy row and rank g's sums are partials 3 g .. 3 g + 2. */
+  double* em_w;
+  const double* cbh;  /* [nspec] */
+  int32_t em_first;
+  int32_t pad2_;
 } prh_team;
 
 /* ETD2 steps k_begin <= k < k_end in one cooperative launch: the steps of
@@ -385,6 +392,15 @@ typedef struct prh_team {
  * that grid or the stream is capturing. */
 int32_t prh_team_march(const prh_operator* op, const prh_schedule* sch, const prh_state* st,
                        const prh_team* tm, int32_t k_begin, int32_t k_end, void* stream);
+
+/* Photon states of steps k_begin <= t < k_end from the Bethe-Heitler sums wsum
+ * ([t - w_first][K][64], prh_team.em_w of the marched steps): the EM part of
+ * prh_em_step for every step of the range in one launch (d = 64, d_em a multiple
+ * of 8).  Reads gam / gam2 by the parity of k_begin, leaves the photons where
+ * prh_em_step of step k_end - 1 would. */
+int32_t prh_em_photon_march(const prh_operator* op, const prh_schedule* sch, const prh_em* em,
+                            const double* wsum, int32_t w_first, int32_t k_begin, int32_t k_end,
+                            void* stream);
 
 /* Adjoint of ETD2 step `step` (two transposed stage kernels).  opT is the
  * operator in transposed block layout with the transposed FD stencil.  No

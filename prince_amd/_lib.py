@@ -37,6 +37,7 @@ EXPORTED = (
     "prh_em_transfer_stack",
     "prh_em_step_transfer",
     "prh_team_march",
+    "prh_em_photon_march",
 )
 
 WG_WAVES = 16
@@ -269,6 +270,10 @@ class PrhTeam(ctypes.Structure):
         ("fin_blk", _p),
         ("dpart", _p),
         ("sync", _p),
+        ("em_w", _p),
+        ("cbh", _p),
+        ("em_first", _i32),
+        ("pad2_", _i32),
     ]
 
 
@@ -303,6 +308,10 @@ def load():
         _i32,
         _p,
     ]
+    lib.prh_em_photon_march.restype = _i32
+    lib.prh_em_photon_march.argtypes = [
+        ctypes.POINTER(PrhOperator), ctypes.POINTER(PrhSchedule), ctypes.POINTER(PrhEm), _p, _i32,
+        _i32, _i32, _p]
     lib.prh_team_march.restype = _i32
     lib.prh_team_march.argtypes = [
         ctypes.POINTER(PrhOperator),

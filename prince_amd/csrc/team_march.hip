@@ -62,6 +62,7 @@ namespace {
 constexpr int TWAVES = 16;  // waves per workgroup (128 registers each)
 constexpr int TTHREADS = TWAVES * WAVE;
 constexpr int TDENSE = 2;   // dense rows per operator
+constexpr int TSUMS = 3;    // sums a dense-row workgroup may form: those rows, and the EM weights
 constexpr int TCONST = 9;   // LDS rows: 7 FD coefficients, energy grid, FD diagonal
 constexpr int SC1 = 16;     // buffer cache policy: agent scope
 constexpr int SPIN_LIMIT = 1 << 25;
@@ -704,6 +705,7 @@ struct DenseDesc {
   // LDS slot and (first diagonal | diagonals << 8) per dense row; the second row
   // has single diagonals only
   int mo, s0, b0, s1, b1;
+  double cw;  // Bethe-Heitler weight of the mother (EM sector)
 };
 
 // Partial sums of the dense rows over this wave's mothers (entries 0 .. ne-1 of
@@ -712,18 +714,19 @@ struct DenseDesc {
 // are stored shifted by their diagonal, load_window): z_o[j] += v_o[j - o] x[j], and
 // y[i] = sum_o z_o[i + o] once per stage -- 18 products per mother and pair
 // instead of 18 and 7 shifts of 4 instructions.
-template <int KP, bool TWO>
+// EM: also the Bethe-Heitler sum over the mothers, weight dd.cw each.
+template <int KP, bool TWO, bool EM>
 __device__ __forceinline__ void dense_partial(COp& op, __amdgpu_buffer_rsrc_t y, int pb,
                                               const TeamLds& L, const DenseDesc& dd, int ne, int k0,
-                                              int kend, const Lane& n, d2 (&acc)[TDENSE][KP]) {
+                                              int kend, const Lane& n, d2 (&acc)[TSUMS][KP]) {
   constexpr int U = 2;
-  d2 z[8][KP], w[KP];
+  d2 z[8][KP], w[KP], em[KP];
   double sc[KP];
 #pragma unroll
   for (int p = 0; p < KP; ++p) {
 #pragma unroll
     for (int o = 0; o < 8; ++o) z[o][p] = d2{0.0, 0.0};
-    w[p] = d2{0.0, 0.0};
+    w[p] = em[p] = d2{0.0, 0.0};
     const int k = k0 + 2 * p + n.half;
     sc[p] = TWO ? op.escale[k < kend ? k : kend - 1] : 0.0;
   }
@@ -740,6 +743,11 @@ __device__ __forceinline__ void dense_partial(COp& op, __amdgpu_buffer_rsrc_t y,
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (e + u >= ne) break;
+      if (EM) {
+        const double cw = readlane_f64(dd.cw, e + u);
+#pragma unroll
+        for (int p = 0; p < KP; ++p) em[p] += cw * xv[u][p];
+      }
       const int s0 = __builtin_amdgcn_readlane(dd.s0, e + u);
       const int b0 = __builtin_amdgcn_readlane(dd.b0, e + u);
       const int s1 = __builtin_amdgcn_readlane(dd.s1, e + u);
@@ -771,6 +779,7 @@ __device__ __forceinline__ void dense_partial(COp& op, __amdgpu_buffer_rsrc_t y,
     for (int o = 6; o >= 0; --o) t = z[o][p] + shift_bin(n, t);
     acc[0][p] = t;
     acc[1][p] = w[p];
+    acc[2][p] = em[p];
   }
 }
 
@@ -909,7 +918,7 @@ __device__ __forceinline__ TeamState team_state(CArgs* a) {
 
 // March of a workgroup of rows: wave wv's tasks.  R = 2: row pairs, KP pairs of
 // right-hand sides a pass, two waves per task (each every second pass).
-template <int R, int KP, bool TWO, bool REC, bool SPLIT>
+template <int R, int KP, bool TWO, bool REC, bool SPLIT, bool EM>
 __device__ __forceinline__ void march_rows(CArgs* A, const TeamLds& L, const TeamPos& P) {
   const int k_begin = A->k_begin, k_end = A->k_end;
   const int* wt = A->tm.wave_ptr + P.rank * TWAVES + P.wv;
@@ -962,28 +971,30 @@ __device__ __forceinline__ void march_rows(CArgs* A, const TeamLds& L, const Tea
     if (s2 && nx != step) coef_stage(L, nx, cn);  // complete behind the phase's barriers
     if (!next_phase(P, epoch)) return;
   }
+  if (EM) next_phase(P, epoch);
 }
 
 // One stage's partial sums of a dense-row workgroup, KP pairs of right-hand
-// sides per wave: mother group dg, column group dc.
-template <int KP, bool TWO>
-__device__ __forceinline__ void dense_stage_partials(COp& op, CTm& tm,
-                                                     const TeamState& T, const TeamLds& L,
-                                                     const TeamPos& P, __amdgpu_buffer_rsrc_t y,
-                                                     int pbase, const DenseDesc& dd, int ne, int dg,
-                                                     int dc) {
+// sides per wave: mother group dg, column group dc.  Sum r of rank g is partial
+// nsum g + r.
+template <int KP, bool TWO, bool EM>
+__device__ __forceinline__ void dense_stage_partials(COp& op, CTm& tm, const TeamState& T,
+                                                     const TeamLds& L, const TeamPos& P,
+                                                     __amdgpu_buffer_rsrc_t y, int pbase,
+                                                     const DenseDesc& dd, int ne, int dg, int dc) {
+  constexpr int NS = EM ? TSUMS : TDENSE;
   const int dG = tm.dgroups, dC = TWAVES / dG;
-  const int po = pbase + P.rank * TDENSE * T.pb;
+  const int po = pbase + P.rank * NS * T.pb;
   d2* const red = reinterpret_cast<d2*>(L.red);
   for (int k0 = P.c0 + dc * 2 * KP; k0 < P.cend; k0 += dC * 2 * KP) {
-    d2 acc[TDENSE][KP];
-    dense_partial<KP, TWO>(op, y, T.pb, L, dd, ne, k0, P.cend, P.n, acc);
+    d2 acc[TSUMS][KP];
+    dense_partial<KP, TWO, EM>(op, y, T.pb, L, dd, ne, k0, P.cend, P.n, acc);
 #pragma unroll
-    for (int r = 0; r < TDENSE; ++r)
+    for (int r = 0; r < NS; ++r)
 #pragma unroll
       for (int p = 0; p < KP; ++p) {
         if (KP == 1 && dG > 1)
-          red[(P.wv * TDENSE + r) * WAVE + P.n.id] = acc[r][p];
+          red[(P.wv * NS + r) * WAVE + P.n.id] = acc[r][p];
         else if (k0 + 2 * p + P.n.half < P.cend)
           pstore<SC1>(acc[r][p], T.part, P.n.off, po + r * T.pb + (k0 + 2 * p) * (WAVE * 8));
       }
@@ -991,35 +1002,37 @@ __device__ __forceinline__ void dense_stage_partials(COp& op, CTm& tm,
   if (KP == 1 && dG > 1) {  // one column pass (2 dC covers the columns): add the mother groups in order
     __syncthreads();
     const int k0 = P.c0 + dc * 2;
-    if (dg < TDENSE && k0 < P.cend) {
+    for (int r = dg; r < NS; r += dG) {
+      if (k0 >= P.cend) break;
       d2 s = {0.0, 0.0};
-      for (int g = 0; g < dG; ++g) s += red[((g * dC + dc) * TDENSE + dg) * WAVE + P.n.id];
+      for (int g = 0; g < dG; ++g) s += red[((g * dC + dc) * NS + r) * WAVE + P.n.id];
       if (k0 + P.n.half < P.cend)
-        pstore<SC1>(s, T.part, P.n.off, po + dg * T.pb + k0 * (WAVE * 8));
+        pstore<SC1>(s, T.part, P.n.off, po + r * T.pb + k0 * (WAVE * 8));
     }
   }
 }
 
 // March of a dense-row workgroup: partial sums over its mothers.
-template <int KD, bool TWO>
+template <int KD, bool TWO, bool EM>
 __device__ __forceinline__ void march_dense(CArgs* A, const TeamLds& L, const TeamPos& P) {
   const int k_begin = A->k_begin, k_end = A->k_end;
   const int dG = A->tm.dgroups, dC = TWAVES / dG;
   const int dg = P.wv / dC, dc = P.wv % dC;
   const int* ep = A->tm.dense_ptr + P.rank * dG + dg;
   const int e0 = cload(ep), ne = cload(ep + 1) - e0;
-  DenseDesc dd{0, 0, 0, 0, 0};
+  DenseDesc dd{0, 0, 0, 0, 0, 0.0};
   if (P.n.id < ne) {
     const int* q = A->tm.dense_ent + 5 * (e0 + P.n.id);
-    dd = DenseDesc{q[0], q[1], q[2], q[3], q[4]};
+    dd = DenseDesc{q[0], q[1], q[2], q[3], q[4], EM ? A->tm.cbh[q[0]] : 0.0};
   }
   uint32_t epoch = 0;
   int wcur = -1;
+  // with an EM sector one phase more: the weights of the last step's state
 #pragma unroll 1
-  for (int p = 2 * k_begin; p < 2 * k_end; ++p) {
+  for (int p = 2 * k_begin; p < 2 * k_end + (EM ? 1 : 0); ++p) {
     CArgs* a = reread(A);
     const int s2 = p & 1;
-    if (s2 == 0) {
+    if (s2 == 0 && p < 2 * k_end) {
       const int w = cload(a->sch.win + (p >> 1));
       if (w != wcur) {
         __syncthreads();
@@ -1029,14 +1042,32 @@ __device__ __forceinline__ void march_dense(CArgs* A, const TeamLds& L, const Te
       }
     }
     const TeamState T = team_state(a);
-    dense_stage_partials<KD, TWO>(a->op, a->tm, T, L, P, s2 ? T.a : T.x, s2 ? T.phalf : 0, dd, ne,
+    dense_stage_partials<KD, TWO, EM>(a->op, a->tm, T, L, P, s2 ? T.a : T.x, s2 ? T.phalf : 0, dd, ne,
                                   dg, dc);
     if (!next_phase(P, epoch)) return;
   }
 }
 
+// sum_s cbh[s] x[s] for the pair of right-hand sides from k0 into slot step of the
+// march's weights ([step - em_first][K][64]).
+__device__ __forceinline__ void em_weights(CTm& tm, const TeamState& T, int step, int K, int k0,
+                                           int kend, const Lane& n) {
+  const int cb = k0 * (WAVE * 8);
+  d2 s = {0.0, 0.0};
+#pragma unroll 4
+  for (int g = 0; g < tm.ndwg; ++g)
+    s += pload<SC1>(T.part, n.off, (g * TSUMS + TDENSE) * T.pb + cb);
+  for (int f = 0; f < tm.nfin; ++f) {
+    const int da = cload(tm.fin + 8 * f);
+    s += cload(tm.cbh + da) * pload<SC1>(T.x, n.off, da * T.pb + cb);
+  }
+  const int k = k0 + n.half;
+  if (k < kend)
+    *reinterpret_cast<d2*>(tm.em_w + ((int64_t)(step - tm.em_first) * K + k) * WAVE + n.bin) = s;
+}
+
 // March of a finishing workgroup: the tail rows, one stage behind the others.
-template <bool TWO, bool REC>
+template <bool TWO, bool REC, bool EM>
 __device__ __forceinline__ void march_finish(CArgs* A, const TeamLds& L, const TeamPos& P) {
   constexpr int NF = TWO ? 2 : 1;
   const int k_begin = A->k_begin, k_end = A->k_end;
@@ -1058,8 +1089,9 @@ __device__ __forceinline__ void march_finish(CArgs* A, const TeamLds& L, const T
   // own; sbuf: the value set of that stage
   int sbuf = 0;
   const int nc = P.cend - P.c0;
+  constexpr int X = EM ? 1 : 0;  // the EM weights of the last step take a phase more
 #pragma unroll 1
-  for (int p = 2 * k_begin; p <= 2 * k_end; ++p) {
+  for (int p = 2 * k_begin; p <= 2 * k_end + X; ++p) {
     CArgs* a = reread(A);
     const int s2 = (p & 1) ^ 1;
     // the step that its next phase begins to finish
@@ -1076,7 +1108,15 @@ __device__ __forceinline__ void march_finish(CArgs* A, const TeamLds& L, const T
         wcur = w;
       }
     }
-    if (p > 2 * k_begin) {
+    if (EM && !s2 && (p >> 1) > k_begin) {
+      // Bethe-Heitler sums of the state after step (p >> 1) - 1, which this phase
+      // has whole: the partials of the heavy mothers and the tail rows' x
+      const TeamState T = team_state(a);
+#pragma unroll 1
+      for (int g = it0; g < groups; g += stride)
+        em_weights(a->tm, T, (p >> 1) - 1, a->op.K, P.c0 + 2 * g, P.cend, P.n);
+    }
+    if (p > 2 * k_begin && p <= 2 * k_end) {
       const TeamLds Q = set(sbuf);
       const StepIn si = step_in<REC>(a->sch, a->st, (p - 1) >> 1);
       const TeamState T = team_state(a);
@@ -1090,11 +1130,11 @@ __device__ __forceinline__ void march_finish(CArgs* A, const TeamLds& L, const T
       }
     }
     if (s2 && p < 2 * k_end) coef_stage(L, p >> 1, cn);
-    if (p < 2 * k_end && !next_phase(P, epoch)) return;
+    if (p < 2 * k_end + X && !next_phase(P, epoch)) return;
   }
 }
 
-template <int R, int KP, int KD, bool TWO, bool REC, bool SPLIT>
+template <int R, int KP, int KD, bool TWO, bool REC, bool SPLIT, bool EM>
 __global__ void __launch_bounds__(TTHREADS) team_march(TeamArgs) {
   extern __shared__ __attribute__((aligned(16))) double lds[];  // 16-byte reads
   __shared__ int bad;
@@ -1137,11 +1177,11 @@ __global__ void __launch_bounds__(TTHREADS) team_march(TeamArgs) {
 
   const int ndwg = A->tm.ndwg, nfwg = A->tm.nfwg;
   if (P.rank < ndwg)
-    march_dense<KD, TWO>(A, L, P);
+    march_dense<KD, TWO, EM>(A, L, P);
   else if (P.rank < ndwg + nfwg)
-    march_finish<TWO, REC>(A, L, P);
+    march_finish<TWO, REC, EM>(A, L, P);
   else
-    march_rows<R, KP, TWO, REC, SPLIT>(A, L, P);
+    march_rows<R, KP, TWO, REC, SPLIT, EM>(A, L, P);
   if (bad) {  // aborted: no silent result
     for (int i = P.rank * TWAVES + P.wv; i < A->op.nspec; i += size * TWAVES)
       for (int k = P.c0; k < P.cend; ++k)
@@ -1156,10 +1196,103 @@ constexpr int MAX_DEVICES = 64;
 std::mutex g_order_mu;
 hipEvent_t g_last_march[MAX_DEVICES] = {};
 
-template <int R, int KP, int KD, bool TWO, bool REC, bool SPLIT>
+// ---------------------------------------------------------------------------
+// Photons of the co-evolved EM cascade over a range of steps.  The nuclei do not
+// see the photons, so the march leaves only the Bethe-Heitler sums of each step
+// and the photons follow here: per step out = [qstep | 2 T_e R_BH] [gam; bhw W]
+// for every column by itself.  One workgroup carries 16 columns through all steps
+// with the photons in LDS, one wave per 16 photon bins (FP64 MFMA); the
+// registers of the step's matrix fragment are refilled with the next step's as
+// each is used.  Bound by the FP64 MFMA rate of its CU, about 3 us a step
+// (136 x 200 x 16), against 18.8 us a step for two launches over the whole
+// batch at K = 512 and 8 us at K = 64.
+constexpr int EMW_TILES = PRH_EM_MAX / 16;    // waves: 16-row tiles of the photon grid
+constexpr int EMW_NQ = PRH_EM_MAX / 8;        // pairs of k-steps over the photons
+constexpr int EMW_NW = WAVE / 8;              // and over the nucleon bins
+constexpr int EMW_ROW = PRH_EM_MAX + WAVE + 2;  // LDS row of a column (padded)
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+__global__ void __launch_bounds__(EMW_TILES * WAVE)
+    em_photon_march(prh_schedule sch, prh_em em, const double* __restrict__ wsum, int w_first, int K,
+                    int k_begin, int k_end) {
+  __shared__ __attribute__((aligned(16))) double y[2][16][EMW_ROW];
+  const int de = em.d_em;
+  const int kd = de + WAVE;
+  const int nq = de / 8;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wv = wave_id();
+  const int col = lane & 15, kq = lane >> 4;
+  const int row = wv * 16 + col;                 // A operand: this lane's matrix row
+  const int rowc = row < de ? row : de - 1;
+  // columns' photons (rows past de stay zero) and the first step's weights
+  const double* g0 = (k_begin & 1) ? em.gam2 : em.gam;
+  for (int i = threadIdx.x; i < 16 * EMW_ROW; i += blockDim.x) {
+    const int c = i / EMW_ROW, r = i % EMW_ROW;
+    const int k = blockIdx.x * 16 + c;
+    y[0][c][r] = (r < de && k < K) ? g0[(int64_t)r * K + k] : 0.0;
+    y[1][c][r] = 0.0;
+  }
+  // weights of step t for this thread's (column, bin) pairs: 1024 over 576 threads
+  constexpr int NT = EMW_TILES * WAVE;
+  auto weight = [&](int t, int i) {
+    const int c = i / WAVE, j = i % WAVE;
+    const int k = blockIdx.x * 16 + c < K ? blockIdx.x * 16 + c : K - 1;
+    return em.bhw[(int64_t)sch.win[t] * WAVE + j] *
+           wsum[((int64_t)(t - w_first) * K + k) * WAVE + j];
+  };
+  auto fragment = [&](int t, int i) -> d2 {  // pair of k-steps i of step t
+    if (i < nq)
+      return *reinterpret_cast<const d2*>(em.qstep + ((int64_t)t * de + rowc) * de + 8 * i + 2 * kq);
+    return *reinterpret_cast<const d2*>(em.tstack + ((int64_t)sch.win[t] * de + rowc) * kd + 8 * i +
+                                        2 * kq);
+  };
+  d2 a[EMW_NQ + EMW_NW];
+  const int np = nq + EMW_NW;
+#pragma unroll
+  for (int i = 0; i < EMW_NQ + EMW_NW; ++i)
+    if (i < np) a[i] = fragment(k_begin, i);
+  __syncthreads();
+  for (int i = threadIdx.x; i < 16 * WAVE; i += NT) y[0][i / WAVE][de + i % WAVE] = weight(k_begin, i);
+  __syncthreads();
+#pragma unroll 1
+  for (int t = k_begin; t < k_end; ++t) {
+    const int b = (t - k_begin) & 1;
+    const int nx = t + 1 < k_end ? t + 1 : t;
+    const double w0 = weight(nx, threadIdx.x);
+    const double w1 = threadIdx.x + NT < 16 * WAVE ? weight(nx, threadIdx.x + NT) : 0.0;
+    d4 acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = acc0;
+#pragma unroll
+    for (int i = 0; i < EMW_NQ + EMW_NW; ++i) {
+      if (i < np) {
+        const d2 v = *reinterpret_cast<const d2*>(&y[b][col][8 * i + 2 * kq]);
+        acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, v.x, acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].y, v.y, acc1, 0, 0, 0);
+        a[i] = fragment(nx, i);
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int r = wv * 16 + kq + 4 * v;
+      if (r < de) y[b ^ 1][col][r] = acc0[v] + acc1[v];
+    }
+    y[b ^ 1][threadIdx.x / WAVE][de + threadIdx.x % WAVE] = w0;
+    if (threadIdx.x + NT < 16 * WAVE)
+      y[b ^ 1][(threadIdx.x + NT) / WAVE][de + threadIdx.x % WAVE] = w1;
+    __syncthreads();
+  }
+  const int b = (k_end - k_begin) & 1;
+  double* g1 = (k_end & 1) ? em.gam2 : em.gam;
+  for (int i = threadIdx.x; i < 16 * de; i += blockDim.x) {
+    const int r = i / 16, c = i % 16;
+    const int k = blockIdx.x * 16 + c;
+    if (k < K) g1[(int64_t)r * K + k] = y[b][c][r];
+  }
+}
+
+template <int R, int KP, int KD, bool TWO, bool REC, bool SPLIT, bool EM>
 int32_t launch_team_rec(const prh_operator& op, const prh_schedule& sch, const prh_state& st,
                         const prh_team& tm, int k_begin, int k_end, hipStream_t s) {
-  const void* fn = reinterpret_cast<const void*>(&team_march<R, KP, KD, TWO, REC, SPLIT>);
+  const void* fn = reinterpret_cast<const void*>(&team_march<R, KP, KD, TWO, REC, SPLIT, EM>);
   const size_t lds =
       8 * WAVE * (size_t)(TCONST + (TWO ? 4 : 2) + 2 * tm.coef_slots + tm.red_slots + tm.lds_slots * (TWO ? 2 : 1));
   hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -1192,8 +1325,15 @@ int32_t launch_team_rec(const prh_operator& op, const prh_schedule& sch, const p
 template <int R, int KP, int KD, bool TWO, bool SPLIT>
 int32_t launch_team(const prh_operator& op, const prh_schedule& sch, const prh_state& st,
                     const prh_team& tm, int k_begin, int k_end, hipStream_t s) {
-  return st.rec_x ? launch_team_rec<R, KP, KD, TWO, true, SPLIT>(op, sch, st, tm, k_begin, k_end, s)
-                  : launch_team_rec<R, KP, KD, TWO, false, SPLIT>(op, sch, st, tm, k_begin, k_end, s);
+  if constexpr (!TWO) {
+    if (tm.em_w)
+      return launch_team_rec<R, KP, KD, false, false, SPLIT, true>(op, sch, st, tm, k_begin, k_end,
+                                                                  s);
+  }
+  return st.rec_x ? launch_team_rec<R, KP, KD, TWO, true, SPLIT, false>(op, sch, st, tm, k_begin,
+                                                                       k_end, s)
+                  : launch_team_rec<R, KP, KD, TWO, false, SPLIT, false>(op, sch, st, tm, k_begin,
+                                                                        k_end, s);
 }
 
 }  // namespace
@@ -1221,7 +1361,7 @@ extern "C" int32_t prh_team_march(const prh_operator* op, const prh_schedule* sc
   if (tm->nteam < 1 || tm->nteam > 8 || tm->size < 1 || tm->size > 256 ||
       (tm->size > 32 && tm->size % 32 != 0))
     return error("prh_team_march: 1 to 8 teams of up to 32 workgroups, or a multiple of 32");
-  if (tm->ndwg < 0 || tm->nfwg < 0 || tm->nfin < 0 || tm->nparts < TDENSE * tm->ndwg ||
+  if (tm->ndwg < 0 || tm->nfwg < 0 || tm->nfin < 0 || tm->nparts < (tm->em_w ? TSUMS : TDENSE) * tm->ndwg ||
       tm->ndwg + tm->nfwg > tm->size || (tm->nfin > 0) != (tm->nfwg > 0))
     return error("prh_team_march: tail rows need finishing workgroups, all within the team");
   if (!tm->sync || !tm->rows || !tm->wave_ptr || !tm->mothers || !tm->lds_ptr || !tm->lds_voff)
@@ -1229,13 +1369,15 @@ extern "C" int32_t prh_team_march(const prh_operator* op, const prh_schedule* sc
   if ((tm->ndwg > 0 && (!tm->dense_ptr || !tm->dense_ent)) ||
       (tm->nfin > 0 && (!tm->fin || !tm->fin_blk)) || (tm->nparts > 0 && !tm->dpart))
     return error("prh_team_march: tail rows need their tables and partials");
+  if (tm->em_w && (!tm->cbh || tm->nfin < 1 || op->mvals_e || st->rec_x || k_begin < tm->em_first))
+    return error("prh_team_march: EM weights need cbh, a tail row, one field and no recording");
   if (!(tm->kd == 1 || tm->kd == 2) || tm->dgroups < 1 || tm->dgroups > TWAVES ||
       TWAVES % tm->dgroups != 0)
     return error("prh_team_march: bad dense-row tiling");
   const int ncmax = (op->K + tm->nteam - 1) / tm->nteam;
   if (tm->ndwg > 0 && tm->dgroups > 1 &&
       (tm->dgroups < TDENSE || tm->kd != 1 || (TWAVES / tm->dgroups) * 2 < ncmax ||
-       tm->red_slots < TWAVES * TDENSE * 2))
+       tm->red_slots < TWAVES * 2 * (tm->em_w ? TSUMS : TDENSE)))
     return error("prh_team_march: mother groups need one column pass and their LDS rows");
   if (op->nsrc * ncmax > TTHREADS || op->nsrc * ncmax > WAVE * tm->coef_slots)
     return error("prh_team_march: more source coefficients per team than staged");
@@ -1273,4 +1415,22 @@ extern "C" int32_t prh_team_march(const prh_operator* op, const prh_schedule* sc
   }
 #undef TEAM
   return error("prh_team_march: no kernel for this kp, kd");
+}
+
+extern "C" int32_t prh_em_photon_march(const prh_operator* op, const prh_schedule* sch,
+                                       const prh_em* em, const double* wsum, int32_t w_first,
+                                       int32_t k_begin, int32_t k_end, void* stream) {
+  using prh_internal::error;
+  if (!op || !sch || !em || !wsum) return error("prh_em_photon_march: null argument");
+  if (op->d != WAVE || em->d_em < 8 || em->d_em > PRH_EM_MAX || em->d_em % 8 != 0)
+    return error("prh_em_photon_march: 64 nucleon bins, EM bins a multiple of 8 up to 144");
+  if (!em->gam || !em->gam2 || !em->bhw || !em->tstack || !em->qstep || op->K < 1)
+    return error("prh_em_photon_march: EM sector with a null buffer");
+  if (k_begin < 0 || k_end > sch->nsteps || k_begin > k_end || w_first < 0 || w_first > k_begin)
+    return error("prh_em_photon_march: step range outside the schedule");
+  if (k_begin == k_end) return 0;
+  hipLaunchKernelGGL(em_photon_march, dim3((unsigned)((op->K + 15) / 16)), dim3(EMW_TILES * WAVE), 0,
+                     (hipStream_t)stream, *sch, *em, wsum, (int)w_first, (int)op->K, (int)k_begin,
+                     (int)k_end);
+  return prh_internal::check(hipGetLastError(), "prh_em_photon_march launch");
 }

@@ -832,8 +832,8 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
             "em": em_struct, "em_bufs": em_bufs,
         }
         self._plan["team"] = None
-        if self.team_march_for(K) and em_struct is None:
-            self._plan["team"] = self._team_setup(lay, dv, K, 2 if two else 1, J)
+        if self.team_march_for(K):
+            self._plan["team"] = self._team_setup(lay, dv, K, 2 if two else 1, J, self._plan)
         if self._plan["team"] is None:
             self._capture_steps(self._plan)
         self.refresh_zs = zs
@@ -845,21 +845,27 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
         if getattr(self.backend, "use_hip_graphs", True) and plan["nsteps"] >= self.graph_chunk:
             plan["graph"] = _lib.StepGraph(plan["op"], plan["sch"], plan["st"], self.graph_chunk)
 
+    #: steps per range of a march with the EM cascade (its Bethe-Heitler sums: 512
+    #: bytes per step and column)
+    EM_RANGE = 256
     #: team plans (host tables on the device, read only) kept per layout
     TEAM_PLANS_KEPT = 8
 
-    def _team_setup(self, lay, dv, K, fields, nsrc):
+    def _team_setup(self, lay, dv, K, fields, nsrc, plan):
         """Team march of this plan (``prh_team``): the layout's tables for K
         columns, and the plan's own partials and sync words.  None when the
         operator or the device does not fit it."""
         torch = _torch()
         wl = lay["layout"]
         args = getattr(self, "_tuned", {}).get(("team_args", K), {})
-        key = (K, fields, nsrc, tuple(sorted(args.items())))
+        em = plan["em"]
+        if em is not None and (em.d_em % 8 or not 8 <= em.d_em <= _lib.EM_MAX):
+            return None
+        key = (K, fields, nsrc, em is not None, tuple(sorted(args.items())))
         plans = lay.setdefault("team", {})
         if key not in plans:
             tp = team_plan.build_team(wl.blocks, wl.fwd.brow_ptr, wl.nspec, wl.d, wl.diag_off, K,
-                                      fields, nsrc, **args)
+                                      fields, nsrc, em is not None, **args)
             names = ("lds_ptr", "lds_voff", "wave_ptr", "rows", "mothers", "dense_ptr",
                      "dense_ent", "fin", "fin_blk")
             tables = None if tp is None else {
@@ -881,7 +887,16 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
             lds_slots=tp.lds_slots, red_slots=tp.red_slots,
             pair_rows=int(tp.pair_rows), coef_slots=tp.coef_slots, pad_=0,
             **{n: t.data_ptr() for n, t in b.items()})
-        return {"struct": tm, "bufs": b, "plan": tp}
+        team = {"struct": tm, "bufs": b, "plan": tp, "em_steps": 0}
+        if em is not None:
+            # the march leaves the Bethe-Heitler sums of a range of steps, the
+            # photons of that range follow in one launch
+            n = min(plan["nsteps"], self.EM_RANGE)
+            b["em_w"] = torch.empty((n, K, wl.d), dtype=torch.float64, device=self.device)
+            tm.em_w = b["em_w"].data_ptr()
+            tm.cbh = plan["em_bufs"]["cbh"].data_ptr()
+            team["em_steps"] = n
+        return team
 
     def _team_run(self, plan, st, k_begin, k_end):
         """Steps [k_begin, k_end) as one cooperative launch; False when it cannot
@@ -889,13 +904,26 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
         team = plan.get("team")
         if team is None or _torch().cuda.is_current_stream_capturing():
             return False
-        rc = self._lib.prh_team_march(
-            ctypes.byref(plan["op"]), ctypes.byref(plan["sch"]), ctypes.byref(st),
-            ctypes.byref(team["struct"]), k_begin, k_end, plan["stream"])
-        if rc == _lib.NOT_LAUNCHABLE:
-            plan["team"] = None
-            return False
-        _lib.check(rc, "team march")
+        em = plan["em"] if st.em else None
+        if em is not None:  # the photons are stepped apart
+            st = _lib.PrhState.from_buffer_copy(st)
+            st.em = None
+        n = team["em_steps"] if em is not None else max(1, k_end - k_begin)
+        for k0 in range(k_begin, k_end, n):
+            k1 = min(k0 + n, k_end)
+            team["struct"].em_first = k0
+            rc = self._lib.prh_team_march(
+                ctypes.byref(plan["op"]), ctypes.byref(plan["sch"]), ctypes.byref(st),
+                ctypes.byref(team["struct"]), k0, k1, plan["stream"])
+            if rc == _lib.NOT_LAUNCHABLE and k0 == k_begin:
+                plan["team"] = None
+                self._capture_steps(plan)
+                return False
+            _lib.check(rc, "team march")
+            if em is not None:
+                _lib.check(self._lib.prh_em_photon_march(
+                    ctypes.byref(plan["op"]), ctypes.byref(plan["sch"]), ctypes.byref(em),
+                    team["bufs"]["em_w"].data_ptr(), k0, k0, k1, plan["stream"]), "photon march")
         return True
 
     def _em_setup(self, zs, K, dv):

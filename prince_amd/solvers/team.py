@@ -103,18 +103,19 @@ def tail_rows(blocks, ptr, nspec):
     return dense, sorted(tail)
 
 
-def build_team(blocks, brow_ptr, nspec, d, diag_off, K, fields=1, nsrc=1, size=None, ndwg=None,
-               nfwg=None):
+def build_team(blocks, brow_ptr, nspec, d, diag_off, K, fields=1, nsrc=1, em=False, size=None,
+               ndwg=None, nfwg=None):
     """Team plan of an operator for K right-hand sides, or None when its rows do
     not fit the march (d != 64, more than two dense rows, bands left of the
     diagonal or wider than 8, a long tail, values beyond the LDS, more source
-    coefficients per team than threads)."""
+    coefficients per team than threads).  ``em``: the march also forms the
+    Bethe-Heitler sums (every heavy row gets a dense entry)."""
     if d != 64 or nspec < 1 or nspec * K * 512 > 0x7FFFFFFF:
         return None
     blocks = np.asarray(blocks, dtype=np.int64).reshape(-1, 4)
     ptr = np.asarray(brow_ptr, dtype=np.int64)
     dense, tail = tail_rows(blocks, ptr, nspec)
-    if len(dense) > DENSE_MAX or len(tail) > TAIL_MAX:
+    if len(dense) > DENSE_MAX or len(tail) > TAIL_MAX or (em and not tail):
         return None
     # the second dense row is the one of single diagonals
     dense.sort(key=lambda da: -int(blocks[ptr[da]:ptr[da + 1], 2].max()))
@@ -128,13 +129,13 @@ def build_team(blocks, brow_ptr, nspec, d, diag_off, K, fields=1, nsrc=1, size=N
             return None
     sizes = [1] if len(tail) == nspec else [size] if size is not None else [32, 64, 128, 256]
     for s in sizes:
-        plan = _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, s, ndwg, nfwg)
+        plan = _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, em, s, ndwg, nfwg)
         if plan is not None:
             return plan
     return None
 
 
-def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, size, ndwg, nfwg):
+def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, em, size, ndwg, nfwg):
     nteam = min(8, CUS // size)
     nc = -(-K // nteam)
     kd, dgroups = dense_tiling(nc)
@@ -150,9 +151,14 @@ def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, size, ndw
             mo, ol, ns, vo = (int(q) for q in blocks[v])
             if mo not in tset:
                 ent.setdefault(mo, [[0, 0, 0], [0, 0, 0]])[r] = [ol, ns, vo]
+    if em:
+        for da in range(nspec):
+            if da not in tset:
+                ent.setdefault(da, [[0, 0, 0], [0, 0, 0]])
     mothers = sorted(ent)
     eslots = np.array([sum(q[1] for q in ent[m]) for m in mothers], dtype=np.int64)
-    red = WAVES * DENSE_MAX * 2 if (mothers and dgroups > 1) else 0
+    nsum = DENSE_MAX + int(em)
+    red = WAVES * nsum * 2 if (mothers and dgroups > 1) else 0
     budget = (LDS_BYTES // 512 - CONST_SLOTS - 2 * fields - 2 * coef - red) // fields
     if not mothers:
         ndwg = 0
@@ -202,8 +208,8 @@ def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, size, ndw
             if mo in tset:
                 fin_blk.append([mo, len(fvoff), ol, ns])
                 fvoff += [(vo + 64 * s, 0) for s in range(ns)]
-        p0, pstep, pn = ((dense.index(da), DENSE_MAX, ndwg) if da in dense
-                         else (DENSE_MAX * ndwg + light.index(da), 1, 1))
+        p0, pstep, pn = ((dense.index(da), nsum, ndwg) if da in dense
+                         else (nsum * ndwg + light.index(da), 1, 1))
         fin.append([da, slot, p0, pstep, pn, first, len(fin_blk) - first, 0])
     for _ in range(nfwg):
         lds_voff += fvoff
@@ -214,7 +220,7 @@ def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, size, ndw
     for da in sorted(light + heavy):
         b = blocks[ptr[da]:ptr[da + 1]]
         b = b[[int(m) not in tset for m in b[:, 0]]] if da in tset else b
-        rowlist.append((da, b, DENSE_MAX * ndwg + light.index(da) if da in tset else -1))
+        rowlist.append((da, b, nsum * ndwg + light.index(da) if da in tset else -1))
     per = 2 if pair_rows else 1
     lanes = WAVES // per  # tasks that run at once in a workgroup
     tasks = [rowlist[i:i + per] for i in range(0, len(rowlist), per)]
@@ -248,7 +254,7 @@ def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, size, ndw
     n[ndwg:ndwg + nfwg] *= 2
     plan = TeamPlan(
         nteam=nteam, size=size, kp=kp, kd=kd, dgroups=dgroups, ndwg=ndwg,
-        nfwg=nfwg, pair_rows=pair_rows, nparts=DENSE_MAX * ndwg + len(light), dense_rows=list(dense),
+        nfwg=nfwg, pair_rows=pair_rows, nparts=nsum * ndwg + len(light), dense_rows=list(dense),
         lds_slots=int(n.max()), red_slots=red, coef_slots=coef,
         lds_ptr=np.asarray(lds_ptr, dtype=np.int32), lds_voff=np.asarray(lds_voff, dtype=np.int32).reshape(-1, 2),
         wave_ptr=np.asarray(wave_ptr, dtype=np.int32),

@@ -150,3 +150,30 @@ def test_a_capturing_stream_takes_the_stage_kernels():
             graph.replay()
             torch.cuda.synchronize()
             assert _norm_dev(p["x"], want) <= TOL
+
+
+@pytest.mark.parametrize("K,z", [(1, 0.03), (3, 0.021), (16, 0.02), (17, 0.02), (70, 0.3)])
+def test_em_march_equals_the_stage_kernels(K, z):
+    """Nuclei and photons of the march with the EM cascade against the per-step EM
+    kernels: odd step counts (the photon buffers alternate), ragged columns of the
+    16-column photon tiles, and more steps than one range."""
+    run = workloads.nuclear_em_run()
+    out = []
+    for team in (True, False):
+        g = _solver(run, z, K, 5, team)
+        p = g.prepare(1e-3)
+        assert (p["team"] is not None) == team
+        x = g.execute(p).clone()
+        gam = g.em_host_state(p).copy()
+        assert bool((g.execute(p) == x).all()) and np.array_equal(g.em_host_state(p), gam)
+        if team and z > 0.25:
+            assert p["nsteps"] > g.EM_RANGE
+            g.execute(p, 0, 111)
+            g.execute(p, 111, p["nsteps"])  # photons across a cut in mid range
+            assert np.array_equal(g.em_host_state(p), gam)
+        out.append((x, gam))
+        g.close()
+    dx = _norm_dev(out[0][0], out[1][0])
+    dg = np.linalg.norm(out[0][1] - out[1][1]) / np.linalg.norm(out[1][1])
+    print(f"K={K}: nuclei {dx:.2e}, photons {dg:.2e}")
+    assert dx <= TOL and dg <= TOL

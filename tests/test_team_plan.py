@@ -26,18 +26,19 @@ def _shift(x, o):
     return y
 
 
+@pytest.mark.parametrize("em", [False, True])
 @pytest.mark.parametrize("name,K,fields,size", [
     ("proton", 1, 1, None), ("proton", 9, 2, None), ("nuclear", 1, 1, None),
     ("nuclear", 7, 2, None), ("nuclear", 37, 1, 64), ("nuclear", 64, 1, None),
     ("nuclear", 64, 1, 256), ("nuclear", 300, 2, 128), ("nuclear", 512, 1, None)])
-def test_plan_reproduces_the_operator(layouts, name, K, fields, size):
+def test_plan_reproduces_the_operator(layouts, name, K, fields, size, em):
     lay, M, m0 = layouts[name]
     nspec, n = lay.nspec, lay.n
     blocks = lay.blocks.copy()
     blocks[:, 3] += n
     vals = np.concatenate([np.where(lay.sel < 0, 0.0, m0[np.maximum(lay.sel, 0)])[lay.zslots:],
                            np.where(lay.sel < 0, 0.0, m0[np.maximum(lay.sel, 0)])[: lay.zslots]])
-    p = team.build_team(blocks, lay.brow_ptr, nspec, 64, 0, K, fields, size=size)
+    p = team.build_team(blocks, lay.brow_ptr, nspec, 64, 0, K, fields, em=em, size=size)
     assert p is not None and p.nteam * p.size <= team.CUS
     assert p.lds_bytes(fields) <= team.LDS_BYTES
     assert p.lds_ptr.size == p.size + 1 and p.wave_ptr.size == p.size * team.WAVES + 1
@@ -62,7 +63,7 @@ def test_plan_reproduces_the_operator(layouts, name, K, fields, size):
                 assert mo not in tail
                 for r, (s, b) in enumerate(((s0, b0), (s1, b1))):
                     for i in range(b >> 8):  # the value in the mother's bins
-                        part[2 * rank + r] += _shift(lds[s + i] * x[mo], (b & 255) + i)
+                        part[(3 if em else 2) * rank + r] += _shift(lds[s + i] * x[mo], (b & 255) + i)
         if rank < p.ndwg + p.nfwg:
             assert p.wave_ptr[rank * team.WAVES] == p.wave_ptr[(rank + 1) * team.WAVES]
             continue
@@ -90,6 +91,9 @@ def test_plan_reproduces_the_operator(layouts, name, K, fields, size):
                     part[ps] = s
                 else:
                     got[da], diag[da] = s, lds[dg]
+    if em and p.ndwg:  # every heavy row has a weight in exactly one dense entry
+        heavy = sorted(set(range(nspec)) - tail)
+        assert sorted(p.dense_ent[:, 0].tolist()) == heavy
     if p.nfwg:  # every finishing workgroup holds the same slots
         r = p.ndwg
         fl = [vals[v:v + 64] for v, _ in p.lds_voff[p.lds_ptr[r]:p.lds_ptr[r + 1]]]
