@@ -393,6 +393,17 @@ typedef struct prh_team {
 int32_t prh_team_march(const prh_operator* op, const prh_schedule* sch, const prh_state* st,
                        const prh_team* tm, int32_t k_begin, int32_t k_end, void* stream);
 
+/* Adjoint steps k_end - 1 down to k_begin (prh_adjoint_steps) in one cooperative
+ * launch (d = 64).  opT as there (tasks and blocks not used); tm: every rank's rows
+ * [][10] = {row, diagonal blocks, band blocks, diagonal's slot, column group,
+ * column groups, first entry, 0, 0, 0}, mothers [][4] = {mother, slot, first
+ * diagonal (0, or negative), diagonals (<= 8, none right of the main one)}, the
+ * diagonal blocks first, at most 64 entries a row; a wave takes every
+ * `column groups`-th pair of its team's columns.  Dense and tail fields are not
+ * used.  Returns 2 (nothing launched) as prh_team_march. */
+int32_t prh_team_adjoint(const prh_operator* opT, const prh_schedule* sch, const prh_adjoint* adj,
+                         const prh_team* tm, int32_t k_begin, int32_t k_end, void* stream);
+
 /* Photon states of steps k_begin <= t < k_end from the Bethe-Heitler sums wsum
  * ([t - w_first][K][64], prh_team.em_w of the marched steps): the EM part of
  * prh_em_step for every step of the range in one launch (d = 64, d_em a multiple

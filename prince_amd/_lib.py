@@ -38,6 +38,7 @@ EXPORTED = (
     "prh_em_step_transfer",
     "prh_team_march",
     "prh_em_photon_march",
+    "prh_team_adjoint",
 )
 
 WG_WAVES = 16
@@ -308,6 +309,10 @@ def load():
         _i32,
         _p,
     ]
+    lib.prh_team_adjoint.restype = _i32
+    lib.prh_team_adjoint.argtypes = [
+        ctypes.POINTER(PrhOperator), ctypes.POINTER(PrhSchedule), ctypes.POINTER(PrhAdjoint),
+        ctypes.POINTER(PrhTeam), _i32, _i32, _p]
     lib.prh_em_photon_march.restype = _i32
     lib.prh_em_photon_march.argtypes = [
         ctypes.POINTER(PrhOperator), ctypes.POINTER(PrhSchedule), ctypes.POINTER(PrhEm), _p, _i32,

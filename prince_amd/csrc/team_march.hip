@@ -1189,6 +1189,341 @@ __global__ void __launch_bounds__(TTHREADS) team_march(TeamArgs) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Adjoint sweep of a range of steps (the transposed stages of prh_adjoint_step) as
+// one cooperative launch: teams, LDS values and barriers as above.  A transposed
+// row reads at most a dozen lighter species by diagonal blocks and the protons by
+// one band left of the diagonal, so there are no dense rows: a wave takes one row
+// and a share of the team's columns.  u and v cross workgroups (sc1); lam, lam_a,
+// the records and the accumulators belong to the row's wave.
+// Per (row, pair of columns) and stage the two fields' factors cost about 250 of
+// 400 vector instructions (two exponentials per bin in stage 2); the launches and
+// their gaps were 65 us a stage at K = 64.
+struct AdjArgs {
+  prh_operator op;
+  prh_schedule sch;
+  prh_adjoint adj;
+  prh_team tm;
+  int k_begin, k_end;
+};
+typedef CONST_SPACE AdjArgs CAdjArgs;
+__device__ __forceinline__ CAdjArgs* reread(CAdjArgs* a) {
+  asm volatile("" : "+s"(a));
+  return a;
+}
+
+__device__ __forceinline__ double dphi1_of(double z, double e, double p1) {
+  return (fabs(z) < 1e-2) ? 0.5 + z * (1.0 / 3.0 + z * (1.0 / 8.0 + z * (1.0 / 30.0)))
+                          : (e - p1) / z;
+}
+__device__ __forceinline__ double dphi2_of(double z, double p1, double p2) {
+  return (fabs(z) < 1e-2) ? 1.0 / 6.0 + z * (1.0 / 12.0 + z * (1.0 / 40.0 + z * (1.0 / 180.0)))
+                          : (p1 - 2.0 * p2) / z;
+}
+// the panel moved up by one bin: bin i receives bin i - 1
+__device__ __forceinline__ d2 shift_bin_up(const Lane& n, d2 v) { return d2{prev1(n, v.y), v.x}; }
+
+// kappa, h d of a row and column at one bin, and their field parts
+struct BinCoef {
+  double kap, kapE, hd, dE;
+};
+template <bool TWO>
+__device__ __forceinline__ BinCoef bin_coef(double kadia, double pscale, double rc, double re,
+                                            double mdc, double mde, double ddiag, double s,
+                                            double dl, double h, bool pdiff) {
+  BinCoef b;
+  b.kap = kadia + pscale * (TWO ? rc + s * re : rc);
+  b.kapE = TWO ? pscale * re : 0.0;
+  double dval = (TWO ? mdc + s * mde : mdc) * dl;
+  if (pdiff) {
+    double kxd = b.kap * ddiag;
+    kxd = kxd * dl;
+    dval = dval + kxd;
+  }
+  b.hd = dval * h;
+  b.dE = TWO ? (mde + b.kapE * ddiag) * dl : 0.0;
+  return b;
+}
+
+// A transposed row of a wave; lane e holds entry e: mother, LDS slot, and for a
+// band its first diagonal (negative) and number of diagonals.
+struct AdjRow {
+  int r, nd, nb, slot, cg, ncg;
+  double pscale;
+  int sslot;
+  int mo, sl, ol, ns;
+};
+
+template <bool TWO>
+__device__ __forceinline__ void adjoint_row(CAdjArgs* a, const TeamLds& L, const TeamState& T,
+                                            const AdjRow& ar, int s2, int step, int c0, int k0,
+                                            int kend, const Lane& n) {
+  constexpr int U = 6;
+  const auto y = s2 ? T.a : T.x;  // v or u
+  const int K = a->op.K;
+  const int cb = k0 * (WAVE * 8);
+  const int own = ar.r * T.pb + cb;
+  const int k = k0 + n.half;
+  const int kc = k < kend ? k : kend - 1;
+  const int64_t oi = ((int64_t)ar.r * K + kc) * WAVE + n.bin;
+  const bool pdiff = (a->op.flags & PRH_F_PARTIAL_DIFF) != 0;
+  d2 acc = {0.0, 0.0}, accE = acc;
+  const d2 yo = pload<SC1>(y, n.off, own);
+  const d2 lp = *reinterpret_cast<const d2*>((s2 ? a->adj.lam_a : a->adj.lam) + oi);
+  // diagonal blocks
+#pragma unroll 1
+  for (int e = 0; e < ar.nd; e += U) {
+    d2 xv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int po = __builtin_amdgcn_readlane(ar.mo, (e + u) & 63) * T.pb + cb;
+      xv[u] = pload<SC1>(y, e + u < ar.nd ? n.off : 0x7ffffff0, po);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (e + u < ar.nd) {
+        const int sl = __builtin_amdgcn_readlane(ar.sl, e + u);
+        acc += lds2(L.val, sl, n.bin) * xv[u];
+        if (TWO) accE += lds2(L.val, L.slots + sl, n.bin) * xv[u];
+      }
+    }
+  }
+  // bands: every diagonal at or left of the main one, walked from the last
+#pragma unroll 1
+  for (int e = ar.nd; e < ar.nd + ar.nb; ++e) {
+    const int sl = __builtin_amdgcn_readlane(ar.sl, e);
+    const int ol = __builtin_amdgcn_readlane(ar.ol, e), ns = __builtin_amdgcn_readlane(ar.ns, e);
+    d2 x = pload<SC1>(y, n.off, __builtin_amdgcn_readlane(ar.mo, e) * T.pb + cb);
+    for (int o = ol + ns - 1; o < 0; ++o) x = shift_bin_up(n, x);
+#pragma unroll 1
+    for (int q0 = ns - 1; q0 >= 0; q0 -= 4) {
+      d2 mc[4], me[TWO ? 4 : 1];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int sq = sl + (q0 - q >= 0 ? q0 - q : 0);
+        mc[q] = lds2(L.val, sq, n.bin);
+        if (TWO) me[TWO ? q : 0] = lds2(L.val, L.slots + sq, n.bin);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (q0 - q >= 0) {
+          acc += mc[q] * x;
+          if (TWO) accE += me[TWO ? q : 0] * x;
+          x = shift_bin_up(n, x);
+        }
+      }
+    }
+  }
+  const double s = TWO ? a->op.escale[kc] : 0.0;
+  const double dl = cload(a->sch.dldz + step), hh = cload(a->sch.h + step);
+  const double hadia = cload(a->sch.hadia + step);
+  // transposed FD stencil D^T y, neighbours -3 .. 3 in order
+  d2 q = {0.0, 0.0};
+  if (pdiff) {
+    const double m1 = prev1(n, yo.y), m2 = prev1(n, yo.x), m3 = prev1(n, m1);
+    const double p2 = next1(n, yo.x), p3 = next1(n, yo.y), p4 = next1(n, p2);
+    q += lds2(L.cst, 0, n.bin) * d2{m3, m2};
+    q += lds2(L.cst, 1, n.bin) * d2{m2, m1};
+    q += lds2(L.cst, 2, n.bin) * d2{m1, yo.x};
+    q += lds2(L.cst, 4, n.bin) * d2{yo.y, p2};
+    q += lds2(L.cst, 5, n.bin) * d2{p2, p3};
+    q += lds2(L.cst, 6, n.bin) * d2{p3, p4};
+  }
+  const d2 mty = TWO ? acc + s * accE : acc;
+  const bool want_s = TWO && a->adj.gdot != nullptr;
+  const int64_t nk = (int64_t)a->op.nspec * K * WAVE;
+  const int64_t ri = (step - a->adj.rec_first) * nk + oi;
+  d2 xx = {0.0, 0.0}, xa = xx, fx = xx, fa = xx, gd = xx;
+  if (want_s) {
+    xx = *reinterpret_cast<const d2*>(a->adj.rec_x + ri);
+    gd = *reinterpret_cast<const d2*>(a->adj.gdot + oi);
+    if (!s2) {
+      xa = *reinterpret_cast<const d2*>(a->adj.rec_a + ri);
+      fx = *reinterpret_cast<const d2*>(a->adj.rec_fx + ri);
+      fa = *reinterpret_cast<const d2*>(a->adj.rec_fa + ri);
+    }
+  }
+  // the step before, for u (its window may be another one: from memory)
+  double dlp = 0.0, hp = 0.0, hadp = 0.0;
+  d2 pmc = {0.0, 0.0}, pme = pmc, prc = pmc, pre = pmc;
+  if (s2 && step > 0) {
+    const int sp = step - 1;
+    const int64_t wp = cload(a->sch.win + sp);
+    dlp = cload(a->sch.dldz + sp);
+    hp = cload(a->sch.h + sp);
+    hadp = cload(a->sch.hadia + sp);
+    const int64_t dg = wp * a->op.mvals_stride + a->op.diag_off + (int64_t)ar.r * WAVE + n.bin;
+    pmc = *reinterpret_cast<const d2*>(a->op.mvals + dg);
+    prc = *reinterpret_cast<const d2*>(a->op.rpair + wp * WAVE + n.bin);
+    if (TWO) {
+      pme = *reinterpret_cast<const d2*>(a->op.mvals_e + dg);
+      pre = *reinterpret_cast<const d2*>(a->op.rpair_e + wp * WAVE + n.bin);
+    }
+  }
+  const d2 eg = lds2(L.cst, 7, n.bin), dd = lds2(L.cst, 8, n.bin);
+  const d2 rc = lds2(L.rp, 0, n.bin), mdc = lds2(L.val, ar.slot, n.bin);
+  const d2 re = TWO ? lds2(L.rp, 1, n.bin) : d2{0.0, 0.0};
+  const d2 mde = TWO ? lds2(L.val, L.slots + ar.slot, n.bin) : d2{0.0, 0.0};
+  d2 out0, out1, wv, gs;  // new lam_a and v (stage 1), lam and u (stage 2)
+#pragma unroll 1
+  for (int b = 0; b < 2; ++b) {  // one bin after the other: half the code
+    auto at = [&](const d2& v) { return b ? v.y : v.x; };
+    const BinCoef c = bin_coef<TWO>(hadia * at(eg), ar.pscale, at(rc), at(re), at(mdc), at(mde),
+                                    at(dd), s, dl, hh, pdiff);
+    const double e = exp(c.hd);
+    const double t = (at(mty) + c.kap * at(q)) * dl;
+    double o0, o1, g = 0.0, ww = 0.0;
+    if (!s2) {
+      const double p1 = phi1_of(c.hd, e), p2 = phi2_of(c.hd, e);
+      o0 = at(lp) + t;
+      ww = hh * p1 * o0;
+      o1 = ww - at(yo);
+      if (want_s) {
+        g = dl * (at(accE) + c.kapE * at(q)) * at(xa);
+        const double dJdd = o0 * (hh * e * at(xx) + hh * hh * dphi1_of(c.hd, e, p1) * at(fx)) +
+                            at(lp) * (hh * hh * dphi2_of(c.hd, p1, p2) * (at(fa) - at(fx)));
+        g += dJdd * c.dE;
+      }
+    } else {
+      o0 = e * at(lp) + t;
+      if (want_s) g = dl * (at(accE) + c.kapE * at(q)) * at(xx);
+      const BinCoef cp = bin_coef<TWO>(hadp * at(eg), ar.pscale, at(prc), at(pre), at(pmc), at(pme),
+                                       at(dd), s, dlp, hp, pdiff);
+      o1 = hp * phi2_of(cp.hd, exp(cp.hd)) * o0;
+    }
+    if (b) {
+      out0.y = o0;
+      out1.y = o1;
+      gs.y = g;
+      wv.y = ww;
+    } else {
+      out0.x = o0;
+      out1.x = o1;
+      gs.x = g;
+      wv.x = ww;
+    }
+  }
+  if (k >= kend) return;  // the odd last right-hand side's idle half
+  *reinterpret_cast<d2*>((s2 ? a->adj.lam : a->adj.lam_a) + oi) = out0;
+  if (!s2)
+    pstore<SC1>(out1, T.a, n.off, own);
+  else if (step > 0)
+    pstore<SC1>(out1, T.x, n.off, own);
+  if (want_s) *reinterpret_cast<d2*>(a->adj.gdot + oi) = gd + gs;
+  if (!s2 && ar.sslot >= 0) {
+    const double f = cload(a->sch.finj + step), lz = cload(a->adj.lnz1 + step);
+    const int J = a->op.nsrc, nc = kend - c0;
+    for (int j = 0; j < J; ++j) {
+      const double c = L.coef[(step & 1) * L.coefs + j * nc + k - c0];
+      const int64_t gi = (((int64_t)ar.sslot * J + j) * K + k) * WAVE + n.bin;
+      d2* g0 = reinterpret_cast<d2*>(a->adj.gsrc0 + gi);
+      d2* g1 = reinterpret_cast<d2*>(a->adj.gsrc1 + gi);
+      *g0 += f * c * wv;
+      *g1 += f * c * lz * wv;
+    }
+  }
+}
+
+template <bool TWO>
+__global__ void __launch_bounds__(TTHREADS) adjoint_march(AdjArgs) {
+  extern __shared__ __attribute__((aligned(16))) double lds[];
+  __shared__ int bad;
+  CAdjArgs* const A = reinterpret_cast<CAdjArgs*>(
+      reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr()));
+  const int K = A->op.K, nteam = A->tm.nteam, size = A->tm.size;
+  const int team = (int)blockIdx.x % nteam;
+  TeamPos P;
+  P.rank = (int)blockIdx.x / nteam;
+  P.n = lane_of();
+  P.wv = wave_id();
+  const int per = K / nteam, rem = K % nteam;
+  P.c0 = team * per + (team < rem ? team : rem);
+  P.cend = P.c0 + per + (team < rem ? 1 : 0);
+  if (P.c0 == P.cend) return;
+  TeamLds L;
+  L.cst = lds;
+  L.rp = L.cst + TCONST * WAVE;
+  L.red = nullptr;
+  L.coef = L.rp + (TWO ? 2 : 1) * WAVE;
+  L.coefs = A->tm.coef_slots * WAVE;
+  L.val = L.coef + 2 * L.coefs;
+  L.slots = cload(A->tm.lds_ptr + P.rank + 1) - cload(A->tm.lds_ptr + P.rank);
+  for (int i = threadIdx.x; i < WAVE; i += TTHREADS) {
+    for (int o = 0; o < 7; ++o)
+      L.cst[o * WAVE + i] = (A->op.flags & PRH_F_PARTIAL_DIFF) ? A->op.dcoef[i * 7 + o] : 0.0;
+    L.cst[7 * WAVE + i] = A->op.egrid[i];
+    L.cst[8 * WAVE + i] = A->op.ddiag[i];
+  }
+  if (threadIdx.x == 0) bad = 0;
+  P.bad = &bad;
+  P.nsub = size > 32 ? size / 32 : 1;
+  P.nsubwg = (uint32_t)size / P.nsub;
+  P.sub = A->tm.sync + SY_SUB + (team * 8 + P.rank % P.nsub) * 64;
+  P.root = A->tm.sync + SY_ROOT + team * 64;
+  P.abort_w = A->tm.sync + SY_ABORT;
+  const int k_begin = A->k_begin, k_end = A->k_end;
+  const int nc = P.cend - P.c0;
+  const bool src = A->adj.gsrc0 != nullptr && (A->op.flags & PRH_F_INJECTION) != 0;
+  if (src) coef_stage(L, k_end - 1, coef_ahead(A->op, A->sch, k_end - 1, P.c0, nc));
+  __syncthreads();
+  const int* wt = A->tm.wave_ptr + P.rank * TWAVES + P.wv;
+  const int t0 = cload(wt), t1 = cload(wt + 1);
+  uint32_t epoch = 0;
+  int wcur = -1;
+#pragma unroll 1
+  for (int p = 2 * (k_end - k_begin) - 1; p >= 0; --p) {
+    CAdjArgs* a = reread(A);
+    const int s2 = (p & 1) ^ 1;  // stage 1 of a step, then stage 2
+    const int step = k_begin + (p >> 1);
+    const bool ahead = src && s2 && step > k_begin && P.wv * WAVE < L.coefs;
+    const double cn = ahead ? coef_ahead(a->op, a->sch, step - 1, P.c0, nc) : 0.0;
+    if (!s2) {
+      const int w = cload(a->sch.win + step);
+      if (w != wcur) {
+        __syncthreads();
+        load_window<TWO>(a->op, a->tm, L, P, w);
+        wcur = w;
+        __syncthreads();
+      }
+    }
+    TeamState T;
+    T.pb = K * WAVE * 8;
+    T.x = tile_rsrc(a->adj.u, a->op.nspec * T.pb);
+    T.a = tile_rsrc(a->adj.v, a->op.nspec * T.pb);
+#pragma unroll 1
+    for (int t = t0; t < t1; ++t) {
+      const int* tk = a->tm.rows + 10 * t;
+      AdjRow ar;
+      ar.r = cload(tk);
+      ar.nd = cload(tk + 1);
+      ar.nb = cload(tk + 2);
+      ar.slot = cload(tk + 3);
+      ar.cg = cload(tk + 4);
+      ar.ncg = cload(tk + 5);
+      ar.pscale = cload(a->op.pscale + ar.r);
+      ar.sslot = src ? cload(a->op.src_slot + ar.r) : -1;
+      ar.mo = ar.sl = ar.ol = ar.ns = 0;
+      if (P.n.id < ar.nd + ar.nb) {
+        const int* q = a->tm.mothers + 4 * (cload(tk + 6) + P.n.id);
+        ar.mo = q[0];
+        ar.sl = q[1];
+        ar.ol = q[2];
+        ar.ns = q[3];
+      }
+#pragma unroll 1
+      for (int k0 = P.c0 + 2 * ar.cg; k0 < P.cend; k0 += 2 * ar.ncg)
+        adjoint_row<TWO>(a, L, T, ar, s2, step, P.c0, k0, P.cend, P.n);
+    }
+    if (ahead) coef_stage(L, step - 1, cn);
+    if (!next_phase(P, epoch)) break;
+  }
+  if (bad) {  // aborted: no silent result
+    for (int i = P.rank * TWAVES + P.wv; i < A->op.nspec; i += size * TWAVES)
+      for (int k = P.c0; k < P.cend; ++k)
+        A->adj.lam[((int64_t)i * K + k) * WAVE + P.n.id] = __builtin_nan("");
+  }
+}
+
 // Marches of one process on one device run one after the other, whatever streams
 // they are on: each waits for the event of the one before.  Two of them on the
 // chip together could each hold CUs the other's barriers need.
@@ -1289,20 +1624,16 @@ __global__ void __launch_bounds__(EMW_TILES * WAVE)
   }
 }
 
-template <int R, int KP, int KD, bool TWO, bool REC, bool SPLIT, bool EM>
-int32_t launch_team_rec(const prh_operator& op, const prh_schedule& sch, const prh_state& st,
-                        const prh_team& tm, int k_begin, int k_end, hipStream_t s) {
-  const void* fn = reinterpret_cast<const void*>(&team_march<R, KP, KD, TWO, REC, SPLIT, EM>);
-  const size_t lds =
-      8 * WAVE * (size_t)(TCONST + (TWO ? 4 : 2) + 2 * tm.coef_slots + tm.red_slots + tm.lds_slots * (TWO ? 2 : 1));
+int32_t launch_march(const void* fn, const prh_team& tm, size_t lds_rows, void* kernel_args,
+                     hipStream_t s) {
+  const size_t lds = 8 * WAVE * lds_rows;
   hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return prh_internal::check(e, "prh_team_march: dynamic LDS");
-  TeamArgs ta{op, sch, st, tm, k_begin, k_end};
-  void* args[] = {&ta};
+  if (e != hipSuccess) return prh_internal::check(e, "team march: dynamic LDS");
+  void* args[] = {kernel_args};
   int dev = -1;
   e = hipGetDevice(&dev);
   if (e != hipSuccess || dev < 0 || dev >= MAX_DEVICES)
-    return prh_internal::error("prh_team_march: no current device in [0, 64)");
+    return prh_internal::error("team march: no current device in [0, 64)");
   std::lock_guard<std::mutex> lock(g_order_mu);
   hipEvent_t& last = g_last_march[dev];
   if (!last) {
@@ -1310,16 +1641,36 @@ int32_t launch_team_rec(const prh_operator& op, const prh_schedule& sch, const p
   } else {
     e = hipStreamWaitEvent(s, last, 0);
   }
-  if (e != hipSuccess) return prh_internal::check(e, "prh_team_march: march order");
+  if (e != hipSuccess) return prh_internal::check(e, "team march: order");
   hipLaunchKernelGGL(team_reset, dim3(1), dim3(1024), 0, s, tm.sync);
   e = hipGetLastError();
   if (e == hipSuccess)
     e = hipLaunchCooperativeKernel(fn, dim3((unsigned)(tm.nteam * tm.size)), dim3(TTHREADS), args,
                                    (unsigned)lds, s);
   if (e == hipSuccess) e = hipEventRecord(last, s);
-  const int32_t rc = prh_internal::check(e, "prh_team_march launch");
+  const int32_t rc = prh_internal::check(e, "team march launch");
   // the device cannot hold the whole grid at once (or not cooperatively)
   return e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported ? 2 : rc;
+}
+
+// 0, or 2 when the stream is being captured (a cooperative launch cannot be)
+int32_t refuse_capture(hipStream_t s) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (int32_t e = prh_internal::check(hipStreamIsCapturing(s, &cs), "team march: capture status"))
+    return e;
+  if (cs == hipStreamCaptureStatusNone) return 0;
+  prh_internal::error("team march: a cooperative launch cannot be captured");
+  return 2;
+}
+
+template <int R, int KP, int KD, bool TWO, bool REC, bool SPLIT, bool EM>
+int32_t launch_team_rec(const prh_operator& op, const prh_schedule& sch, const prh_state& st,
+                        const prh_team& tm, int k_begin, int k_end, hipStream_t s) {
+  TeamArgs ta{op, sch, st, tm, k_begin, k_end};
+  return launch_march(reinterpret_cast<const void*>(&team_march<R, KP, KD, TWO, REC, SPLIT, EM>), tm,
+                      (size_t)(TCONST + (TWO ? 4 : 2) + 2 * tm.coef_slots + tm.red_slots +
+                               tm.lds_slots * (TWO ? 2 : 1)),
+                      &ta, s);
 }
 
 template <int R, int KP, int KD, bool TWO, bool SPLIT>
@@ -1383,13 +1734,7 @@ extern "C" int32_t prh_team_march(const prh_operator* op, const prh_schedule* sc
     return error("prh_team_march: more source coefficients per team than staged");
   if (k_begin == k_end) return 0;
   hipStream_t s = (hipStream_t)stream;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (int32_t e = prh_internal::check(hipStreamIsCapturing(s, &cs), "prh_team_march: capture status"))
-    return e;
-  if (cs != hipStreamCaptureStatusNone) {
-    error("prh_team_march: a cooperative launch cannot be captured; use prh_etd2_steps");
-    return 2;
-  }
+  if (int32_t e = refuse_capture(s)) return e;
   if (tm->pair_rows == 0 && ncmax > 2)
     return error("prh_team_march: single-row tasks take at most 2 right-hand sides per team");
   // one right-hand side per team: the halves of a wave share it
@@ -1433,4 +1778,47 @@ extern "C" int32_t prh_em_photon_march(const prh_operator* op, const prh_schedul
                      (hipStream_t)stream, *sch, *em, wsum, (int)w_first, (int)op->K, (int)k_begin,
                      (int)k_end);
   return prh_internal::check(hipGetLastError(), "prh_em_photon_march launch");
+}
+
+extern "C" int32_t prh_team_adjoint(const prh_operator* op, const prh_schedule* sch,
+                                    const prh_adjoint* adj, const prh_team* tm, int32_t k_begin,
+                                    int32_t k_end, void* stream) {
+  using prh_internal::error;
+  if (!op || !sch || !adj || !tm) return error("prh_team_adjoint: null argument");
+  if (op->d != WAVE) return error("prh_team_adjoint: 64 energy bins only");
+  if (op->K <= 0 || op->nspec <= 0) return error("prh_team_adjoint: empty operator");
+  if ((int64_t)op->nspec * op->K * WAVE * 8 > 0x7fffffff)
+    return error("prh_team_adjoint: a state array exceeds 2 GiB");
+  if ((op->mvals_e == nullptr) != (op->escale == nullptr) ||
+      (op->mvals_e != nullptr && op->rpair_e == nullptr))
+    return error("prh_team_adjoint: mvals_e, rpair_e and escale go together");
+  if (!adj->lam || !adj->lam_a || !adj->u || !adj->v)
+    return error("prh_team_adjoint: lam, lam_a, u and v are required");
+  if (k_begin < 0 || k_end > sch->nsteps || k_begin > k_end)
+    return error("prh_team_adjoint: step range outside the schedule");
+  if (op->mvals_e && adj->gdot) {
+    if (!adj->rec_x || !adj->rec_a || !adj->rec_fx || !adj->rec_fa)
+      return error("prh_team_adjoint: the EBL-scale gradient needs the recorded forward steps");
+    if (k_begin < adj->rec_first || k_end > adj->rec_first + adj->rec_count)
+      return error("prh_team_adjoint: steps outside the recorded chunk");
+  }
+  if (adj->gsrc0 && (!adj->gsrc1 || !adj->lnz1))
+    return error("prh_team_adjoint: source accumulators need gsrc1 and lnz1");
+  if (tm->nteam < 1 || tm->nteam > 8 || tm->size < 1 || tm->size > 256 ||
+      (tm->size > 32 && tm->size % 32 != 0))
+    return error("prh_team_adjoint: 1 to 8 teams of up to 32 workgroups, or a multiple of 32");
+  if (!tm->sync || !tm->rows || !tm->wave_ptr || !tm->mothers || !tm->lds_ptr || !tm->lds_voff)
+    return error("prh_team_adjoint: null table");
+  const int ncmax = (op->K + tm->nteam - 1) / tm->nteam;
+  if (op->nsrc * ncmax > TTHREADS || op->nsrc * ncmax > WAVE * tm->coef_slots)
+    return error("prh_team_adjoint: more source coefficients per team than staged");
+  if (k_begin == k_end) return 0;
+  hipStream_t s = (hipStream_t)stream;
+  if (int32_t e = refuse_capture(s)) return e;
+  AdjArgs ta{*op, *sch, *adj, *tm, k_begin, k_end};
+  const int nf = op->mvals_e ? 2 : 1;
+  const void* fn = op->mvals_e ? reinterpret_cast<const void*>(&adjoint_march<true>)
+                               : reinterpret_cast<const void*>(&adjoint_march<false>);
+  return launch_march(fn, *tm, (size_t)(TCONST + nf + 2 * tm->coef_slots + tm->lds_slots * nf), &ta,
+                      s);
 }

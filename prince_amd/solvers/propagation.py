@@ -834,6 +834,8 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
         self._plan["team"] = None
         if self.team_march_for(K):
             self._plan["team"] = self._team_setup(lay, dv, K, 2 if two else 1, J, self._plan)
+            if with_adjoint:
+                self._plan["team_adjoint"] = self._adjoint_team_setup(lay, dv, K, 2 if two else 1, J)
         if self._plan["team"] is None:
             self._capture_steps(self._plan)
         self.refresh_zs = zs
@@ -851,21 +853,12 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
     #: team plans (host tables on the device, read only) kept per layout
     TEAM_PLANS_KEPT = 8
 
-    def _team_setup(self, lay, dv, K, fields, nsrc, plan):
-        """Team march of this plan (``prh_team``): the layout's tables for K
-        columns, and the plan's own partials and sync words.  None when the
-        operator or the device does not fit it."""
+    def _team_tables(self, lay, key, K, dv, build):
+        """A march's tables (kept with the layout) and its own partials and sync words."""
         torch = _torch()
-        wl = lay["layout"]
-        args = getattr(self, "_tuned", {}).get(("team_args", K), {})
-        em = plan["em"]
-        if em is not None and (em.d_em % 8 or not 8 <= em.d_em <= _lib.EM_MAX):
-            return None
-        key = (K, fields, nsrc, em is not None, tuple(sorted(args.items())))
         plans = lay.setdefault("team", {})
         if key not in plans:
-            tp = team_plan.build_team(wl.blocks, wl.fwd.brow_ptr, wl.nspec, wl.d, wl.diag_off, K,
-                                      fields, nsrc, em is not None, **args)
+            tp = build()
             names = ("lds_ptr", "lds_voff", "wave_ptr", "rows", "mothers", "dense_ptr",
                      "dense_ent", "fin", "fin_blk")
             tables = None if tp is None else {
@@ -879,7 +872,7 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
             return None
         b = dict(tables)
         b["sync"] = torch.zeros(team_plan.SYNC_BYTES // 4, dtype=torch.int32, device=self.device)
-        b["dpart"] = torch.empty((2, max(1, tp.nparts), K, wl.d), dtype=torch.float64,
+        b["dpart"] = torch.empty((2, max(1, tp.nparts), K, 64), dtype=torch.float64,
                                  device=self.device)
         tm = _lib.PrhTeam(
             nteam=tp.nteam, size=tp.size, kp=tp.kp, kd=tp.kd, dgroups=tp.dgroups, ndwg=tp.ndwg,
@@ -887,7 +880,33 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
             lds_slots=tp.lds_slots, red_slots=tp.red_slots,
             pair_rows=int(tp.pair_rows), coef_slots=tp.coef_slots, pad_=0,
             **{n: t.data_ptr() for n, t in b.items()})
-        team = {"struct": tm, "bufs": b, "plan": tp, "em_steps": 0}
+        return {"struct": tm, "bufs": b, "plan": tp, "em_steps": 0}
+
+    def _adjoint_team_setup(self, lay, dv, K, fields, nsrc):
+        """Team march of the transposed operator, or None (as ``_team_setup``)."""
+        wl = lay["layout"]
+        return self._team_tables(
+            lay, ("adjoint", K, fields, nsrc), K, dv,
+            lambda: team_plan.build_adjoint_team(wl.blocks_t, wl.tr.brow_ptr, wl.nspec, wl.d,
+                                                 wl.diag_off, K, fields, nsrc))
+
+    def _team_setup(self, lay, dv, K, fields, nsrc, plan):
+        """Team march of this plan (``prh_team``): the layout's tables for K
+        columns, and the plan's own partials and sync words.  None when the
+        operator or the device does not fit it."""
+        torch = _torch()
+        wl = lay["layout"]
+        args = getattr(self, "_tuned", {}).get(("team_args", K), {})
+        em = plan["em"]
+        if em is not None and (em.d_em % 8 or not 8 <= em.d_em <= _lib.EM_MAX):
+            return None
+        team = self._team_tables(
+            lay, (K, fields, nsrc, em is not None, tuple(sorted(args.items()))), K, dv,
+            lambda: team_plan.build_team(wl.blocks, wl.fwd.brow_ptr, wl.nspec, wl.d, wl.diag_off, K,
+                                         fields, nsrc, em is not None, **args))
+        if team is None:
+            return None
+        tm, b = team["struct"], team["bufs"]
         if em is not None:
             # the march leaves the Bethe-Heitler sums of a range of steps, the
             # photons of that range follow in one launch
@@ -924,6 +943,21 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
                 _lib.check(self._lib.prh_em_photon_march(
                     ctypes.byref(plan["op"]), ctypes.byref(plan["sch"]), ctypes.byref(em),
                     team["bufs"]["em_w"].data_ptr(), k0, k0, k1, plan["stream"]), "photon march")
+        return True
+
+    def _team_adjoint_run(self, plan, k_begin, k_end):
+        """Adjoint steps [k_begin, k_end) as one cooperative launch; False when it
+        cannot run here."""
+        team = plan.get("team_adjoint")
+        if team is None or _torch().cuda.is_current_stream_capturing():
+            return False
+        rc = self._lib.prh_team_adjoint(
+            ctypes.byref(plan["opT"]), ctypes.byref(plan["sch"]), ctypes.byref(plan["adj"]),
+            ctypes.byref(team["struct"]), k_begin, k_end, plan["stream"])
+        if rc == _lib.NOT_LAUNCHABLE:
+            plan["team_adjoint"] = None
+            return False
+        _lib.check(rc, "adjoint march")
         return True
 
     def _em_setup(self, zs, K, dv):
@@ -1224,8 +1258,10 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
                 _lib.check(lib.prh_etd2_steps(ctypes.byref(plan["op"]), ctypes.byref(sch),
                                               ctypes.byref(st), k0, k1, stream), "recompute")
             adj.rec_first = k0
-            _lib.check(lib.prh_adjoint_steps(ctypes.byref(opT), ctypes.byref(sch),
-                                             ctypes.byref(adj), k0, k1, stream), "adjoint steps")
+            if not self._team_adjoint_run(plan, k0, k1):
+                _lib.check(lib.prh_adjoint_steps(ctypes.byref(opT), ctypes.byref(sch),
+                                                 ctypes.byref(adj), k0, k1, stream),
+                           "adjoint steps")
         return ab
 
     def _run_integration(self, state, z_grid, step_hook=None):

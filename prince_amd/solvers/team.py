@@ -295,3 +295,61 @@ def _bounds(slots, parts):
     """Contiguous ranges (starts, ends) of similar slot count."""
     b = _cut(slots.astype(np.float64), parts)
     return b[:-1], b[1:]
+
+
+def build_adjoint_team(blocks, brow_ptr, nspec, d, diag_off, K, fields=1, nsrc=1, size=None):
+    """Team plan of the transposed operator (``prh_team_adjoint``), or None: rows of
+    diagonal blocks and bands that end at or left of the diagonal, one per wave,
+    the team's columns shared by as many waves per row as the workgroup has."""
+    if d != 64 or nspec < 1 or nspec * K * 512 > 0x7FFFFFFF:
+        return None
+    blocks = np.asarray(blocks, dtype=np.int64).reshape(-1, 4)
+    ptr = np.asarray(brow_ptr, dtype=np.int64)
+    if np.any(blocks[:, 2] > BAND_MAX) or np.any(blocks[:, 1] + blocks[:, 2] > 1):
+        return None
+    if np.any(np.diff(ptr) > 64):
+        return None
+    for s in [1] if nspec == 1 else [size] if size is not None else [32, 64, 128, 256]:
+        nteam = min(8, CUS // s)
+        nc = -(-K // nteam)
+        if nsrc * nc > 64 * WAVES:
+            continue
+        coef = -(-nsrc * nc // 64)
+        budget = (LDS_BYTES // 512 - CONST_SLOTS - fields - 2 * coef) // fields
+        slots = np.array([1 + int(blocks[ptr[r]:ptr[r + 1], 2].sum()) for r in range(nspec)])
+        bounds = _cut(slots + 8.0, s)
+        lds_ptr, voff, wave_ptr, rows, ents = [0], [], [0], [], []
+        for i in range(s):
+            mine = list(range(bounds[i], bounds[i + 1]))
+            ncg = max(1, min(WAVES // max(1, len(mine)), -(-nc // 2)))
+            base = len(voff)
+            per_wave = [[] for _ in range(WAVES)]
+            for q, r in enumerate(mine):
+                b = blocks[ptr[r]:ptr[r + 1]]
+                diag = (b[:, 2] == 1) & (b[:, 1] == 0)
+                head = len(voff) - base
+                voff.append((diag_off + r * 64, 0))
+                first = len(ents)
+                for mo, ol, ns, vo in np.concatenate([b[diag], b[~diag]]).tolist():
+                    ents.append([mo, len(voff) - base, ol, ns])
+                    voff += [(vo + 64 * x, 0) for x in range(ns)]
+                for cg in range(ncg):
+                    per_wave[(q * ncg + cg) % WAVES].append(
+                        [r, int(diag.sum()), int((~diag).sum()), head, cg, ncg, first, 0, 0, 0])
+            for w in per_wave:
+                rows += w
+                wave_ptr.append(len(rows))
+            lds_ptr.append(len(voff))
+        n = int(np.diff(lds_ptr).max())
+        if n <= budget:
+            return TeamPlan(
+                nteam=nteam, size=s, kp=1, kd=1, dgroups=1, ndwg=0, nfwg=0, pair_rows=False, nparts=0,
+                dense_rows=[], lds_slots=n, red_slots=0, coef_slots=coef,
+                lds_ptr=np.asarray(lds_ptr, dtype=np.int32),
+                lds_voff=np.asarray(voff, dtype=np.int32).reshape(-1, 2),
+                wave_ptr=np.asarray(wave_ptr, dtype=np.int32),
+                rows=np.asarray(rows, dtype=np.int32).reshape(-1, 10),
+                mothers=np.asarray(ents, dtype=np.int32).reshape(-1, 4),
+                dense_ptr=np.zeros(1, dtype=np.int32), dense_ent=np.zeros((0, 5), dtype=np.int32),
+                fin=np.zeros((0, 8), dtype=np.int32), fin_blk=np.zeros((0, 4), dtype=np.int32))
+    return None

@@ -177,3 +177,32 @@ def test_em_march_equals_the_stage_kernels(K, z):
     dg = np.linalg.norm(out[0][1] - out[1][1]) / np.linalg.norm(out[1][1])
     print(f"K={K}: nuclei {dx:.2e}, photons {dg:.2e}")
     assert dx <= TOL and dg <= TOL
+
+
+@pytest.mark.parametrize("K,two", [(1, True), (3, False), (8, True), (13, True), (40, False),
+                                   (70, True)])
+def test_adjoint_march_equals_the_transposed_stages(K, two):
+    """The adjoint sweep by marches against the per-step kernels, more than one
+    checkpoint chunk, ragged columns."""
+    import torch
+
+    run = workloads.nuclear_run()
+    out = []
+    for team in (True, False):
+        g = _solver(run, 0.07, K, 7, team, np.linspace(0.6, 1.4, K) if two else None)
+        p = g.prepare(1e-3, with_adjoint=True)
+        assert ((p.get("team_adjoint") is not None) == team)
+        lam = torch.randn(tuple(p["x"].shape), dtype=torch.float64,
+                          generator=torch.Generator().manual_seed(2)).to(p["x"].device)
+        res = []
+        for _ in range(2):
+            g.forward_checkpointed(p)
+            ab = g.adjoint_sweep(p, lam)
+            res.append({k: ab[k].clone() for k in ("lam", "gsrc0", "gsrc1", "gdot")})
+        assert all(torch.equal(res[0][k], res[1][k]) for k in res[0])
+        out.append(res[0])
+        g.close()
+    for k in ("lam", "gsrc0", "gsrc1") + (("gdot",) if two else ()):
+        d = _norm_dev(out[0][k], out[1][k])
+        print(f"K={K} {k}: {d:.2e}")
+        assert d <= TOL, k

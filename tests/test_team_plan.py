@@ -140,3 +140,45 @@ def test_operators_outside_the_march_are_refused():
     assert team.build_team(diag, ptr, 1, 64, 0, 5_000_000) is None  # state beyond 2 GiB
     assert team.build_team(diag, ptr, 1, 64, 0, 64, nsrc=128) is not None
     assert team.build_team(diag, ptr, 1, 64, 0, 64, nsrc=129) is None  # coefficients per team
+
+
+@pytest.mark.parametrize("name,K,fields,size", [
+    ("proton", 3, 2, None), ("nuclear", 1, 1, None), ("nuclear", 64, 2, None),
+    ("nuclear", 37, 2, 128), ("nuclear", 300, 1, None)])
+def test_adjoint_plan_reproduces_the_transposed_operator(layouts, name, K, fields, size):
+    from prince_amd.solvers.layout import transposed_layout
+
+    lay, M, m0 = layouts[name]
+    nspec, n = lay.nspec, lay.n
+    tr = transposed_layout(M.indptr, M.indices, m0, nspec, 64)
+    blocks = tr.blocks.copy()
+    blocks[:, 3] += n
+    pick = np.where(tr.sel < 0, 0.0, m0[np.maximum(tr.sel, 0)])
+    vals = np.concatenate([pick[tr.zslots:], pick[:tr.zslots]])
+    p = team.build_adjoint_team(blocks, tr.brow_ptr, nspec, 64, 0, K, fields, size=size)
+    nc = -(-K // p.nteam)
+    assert np.all((p.lds_voff[:, 0] >= 0) & (p.lds_voff[:, 0] + 64 <= vals.size))
+    x = np.random.default_rng(4).standard_normal((nspec, 64))
+    got = {}
+    for rank in range(p.size):
+        lds = [vals[v:v + 64] for v, _ in p.lds_voff[p.lds_ptr[rank]:p.lds_ptr[rank + 1]]]
+        assert len(lds) <= p.lds_slots
+        for t in range(p.wave_ptr[rank * 16], p.wave_ptr[(rank + 1) * 16]):
+            r, nd, nb, head, cg, ncg, first = (int(v) for v in p.rows[t][:7])
+            assert nd + nb <= 64 and np.array_equal(lds[head], vals[64 * r:64 * r + 64])
+            y = np.zeros(64)
+            for e, (mo, sl, ol, ns) in enumerate(p.mothers[first:first + nd + nb].tolist()):
+                assert (ns == 1 and ol == 0) if e < nd else (ns <= 8 and ol + ns <= 1)
+                for i in range(ns):
+                    sh = np.zeros(64)
+                    o = -(ol + i)
+                    sh[o:] = x[mo][:64 - o]
+                    y += lds[sl + i] * sh
+            got.setdefault(r, []).append((cg, ncg, y))
+    full = M.copy()
+    full.data = m0.copy()
+    want = (full.T @ x.ravel() - full.diagonal() * x.ravel()).reshape(nspec, 64)
+    for r in range(nspec):  # every pair of columns by exactly one wave
+        pairs = sorted(q for cg, ncg, _ in got[r] for q in range(cg, -(-nc // 2), ncg))
+        assert pairs == list(range(-(-nc // 2)))
+        assert np.allclose(got[r][0][2], want[r], rtol=1e-12, atol=1e-12 * np.abs(want).max())
