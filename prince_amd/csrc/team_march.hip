@@ -125,7 +125,6 @@ struct Lane {
   int bin;          // first of its two bins
   int off;          // byte offset of its bins in the pair's [2][64] panel
   bool first, last; // bins 0, 1 / 62, 63
-  bool edge0, edge1;  // bins below 4 / above 59
 };
 __device__ __forceinline__ Lane lane_of() {
   Lane n;
@@ -135,8 +134,6 @@ __device__ __forceinline__ Lane lane_of() {
   n.off = n.id * 16;
   n.first = n.bin == 0;
   n.last = n.bin == 62;
-  n.edge0 = n.bin < 4;
-  n.edge1 = n.bin > 59;
   return n;
 }
 
@@ -320,13 +317,23 @@ __device__ __forceinline__ void team_epilogue(COp& op, CSt& st,
     d2 out = acc[p];
     if (pdiff) {
       const d2 kx = f.kap * xo[p];
-      // stencil neighbours of bins 2 l and 2 l + 1, added in the order -3 .. 3
-      const double m1 = prev1(n, kx.y);  // bin 2 l - 1
-      const double m2 = prev1(n, kx.x);  // bin 2 l - 2
-      const double m3 = prev1(n, m1);    // bin 2 l - 3
-      const double q2 = next1(n, kx.x);  // bin 2 l + 2
-      const double q3 = next1(n, kx.y);  // bin 2 l + 3
-      const double q4 = next1(n, q2);    // bin 2 l + 4
+      // stencil neighbours of bins 2 l and 2 l + 1, added in the order -3 .. 3.
+      // Past the ends of a half the shifts bring the other column's bins, which
+      // meet coefficients that are exactly zero; masked unless all are finite.
+      double m1 = lane_prev(kx.y);  // bin 2 l - 1
+      double m2 = lane_prev(kx.x);  // bin 2 l - 2
+      double m3 = lane_prev(m1);    // bin 2 l - 3
+      double q2 = lane_next(kx.x);  // bin 2 l + 2
+      double q3 = lane_next(kx.y);  // bin 2 l + 3
+      double q4 = lane_next(q2);    // bin 2 l + 4
+      if (__builtin_expect(!__all(isfinite(kx.x) && isfinite(kx.y)), 0)) {
+        m1 = n.first ? 0.0 : m1;
+        m2 = n.first ? 0.0 : m2;
+        m3 = n.bin < 4 ? 0.0 : m3;
+        q2 = n.last ? 0.0 : q2;
+        q3 = n.last ? 0.0 : q3;
+        q4 = n.bin > 59 ? 0.0 : q4;
+      }
       d2 dx = {0.0, 0.0};
       dx += lds2(L.cst, 0, n.bin) * d2{m3, m2};
       dx += lds2(L.cst, 1, n.bin) * d2{m2, m1};
