@@ -537,8 +537,8 @@ typedef struct prh_cascade {
   const double* kern_b;    /* [n][d][nb] Bethe-Heitler kernel */
 } prh_cascade;
 
-/* Kinetic single-scatter cascade transfer of nwin windows (one 16-wave
- * workgroup each).  contr [nwin][cstride]: the window's target densities
+/* Kinetic single-scatter cascade transfer of nwin windows (16 columns of a
+ * window to a workgroup).  contr [nwin][cstride]: the window's target densities
  * contracted with the field-free tensors (prh_fold_gemm): IC emission
  * [n][n], pair injection [n][n], IC power [n], IC rate [n], sum w n,
  * sum w eps n; dtau [nwin][n] the opacity per unit length, dl [nwin] the

@@ -2226,29 +2226,46 @@ void launch_adjoint_two(const prh_operator& op, const prh_schedule& sch, const p
 // cascade/cascade.py:284-407 and 425-589, cascade/bethe_heitler.py:219-351).
 //
 // For every window w (redshift z_w, field scale s_w) the field-free tensors
-// are contracted with the target-photon densities by prh_fold_gemm (MFMA);
-// cascade_transfer_kernel then builds, per window in one 16-wave workgroup,
-// the pair matrix P, the IC emission shape Sg, the degraded-electron map De,
-// the IC cooling map Mic and the kinetic single-scatter iteration
+// are contracted with the target-photon densities by prh_fold_gemm (MFMA).
+// From these come, per window, the pair matrix P, the IC emission shape Sg, the
+// degraded-electron map De and the IC cooling map Mic, then the kinetic
+// single-scatter iteration
 //   esc += pesc G;  e += P ((G - pesc G) dE);
 //   G_c = Mic (e_cold dE);  G_h = Sg (e_hot dE);  e = De (e_hot dE);
 //   esc += pesc G_c;  G = G_h + G_c - pesc G_c
-// until the energy left in G and e is below tol of each column's input; the
-// outputs are T_gamma = esc and T_electron = esc (Mic dE).  The three
-// products of a step share their right operand and run as one pass of
-// v_mfma_f64_16x16x4 tiles over the 144 x 144 padded matrices held in a
-// per-window workspace in HBM (L2-resident while the workgroup runs).
+// until the energy left in G and e is below tol of each column's input, and
+// T_gamma = esc, T_electron = esc (Mic dE).
+//
+// The columns of the iterates are independent, so a workgroup takes 16 columns
+// of a window (9 per window: 288 windows are 2592 workgroups on 256 CUs), keeps
+// its tiles of G, e and esc in registers in the layout the MFMA returns, and
+// passes the right operands through two 18 KB LDS panels.  No scatter raises an
+// energy, so the four matrices are upper triangular and a block of columns holds
+// zeros below its diagonal tile: rows and contraction indices of zero tiles are
+// left out (165 of 729 tile products of a full 144), and of the three products
+// after a scatter only those whose electrons (cold or hot) a tile holds.  This
+// is read from the matrices, not assumed: any nonzero below the diagonal tiles
+// or any non-finite value sends the window through all tiles.  A wave takes row
+// tiles v and last - v, which together have the same number of k steps.
+//
+// Bound by the serial chain of an iteration (34 to 42 iterations of three
+// barriers and up to 9 tiles of k).  288 windows of 136 bins: 17.45 ms with a
+// workgroup a window and full matrices, 4.42 ms so (1.38 ms the first launch,
+// 0.83 the second, 0.41 the columns, 1.2 the contraction before).
 // ---------------------------------------------------------------------------
 constexpr int CNP = 144;              // padded EM dimension (n <= 144)
 constexpr int CTL = CNP / 16;         // 9 tiles per matrix side
-constexpr int CWAVES = 8;
+constexpr int CWAVES = 5;             // row tiles v and last - v
 constexpr int CTHREADS = CWAVES * WAVE;
-constexpr int CTILES = CTL * CTL;     // 81 output tiles
-constexpr int CTPW = (CTILES + CWAVES - 1) / CWAVES;  // tiles per wave (11)
+constexpr int CPREP = 256;            // threads of the preparing kernels
+constexpr int CPIT = 17;              // LDS pitch of a 16-column tile column
 constexpr int64_t CMAT = (int64_t)CNP * CNP;
-constexpr int CKU = 4;                // k-steps whose loads are issued together (36 = 9 x 4)
-constexpr int CKU2 = 2;               // the same for the 3 x 3-tile products (register budget)
-enum CascadeMat { CM_P = 0, CM_SG, CM_DE, CM_MIC, CM_G, CM_E, CM_E1, CM_ESC, CM_T, CM_COUNT };
+// per-window workspace; P .. Mic are stored transposed (k-major): an operand
+// fragment (16 rows x 4 k) is four 128-byte row segments
+enum CascadeMat { CM_P = 0, CM_SG, CM_DE, CM_MIC, CM_G, CM_E, CM_INFO, CM_ESC, CM_SPARE, CM_COUNT };
+// doubles of the CM_INFO matrix: cold flags, then per column block the
+// iterations done, converged or not, and triangular and finite or not
+constexpr int CI_COLD = 0, CI_ITS = CNP, CI_DONE = CI_ITS + 16, CI_TRI = CI_DONE + 16;
 
 // rows of the contraction output per window (prh_cascade layout)
 __device__ __forceinline__ int64_t crow_emis(int) { return 0; }
@@ -2258,302 +2275,466 @@ __device__ __forceinline__ int64_t crow_rate(int n) { return 2 * (int64_t)n * n 
 __device__ __forceinline__ int64_t crow_den(int n) { return 2 * (int64_t)n * n + 2 * n; }
 __device__ __forceinline__ int64_t crow_num(int n) { return 2 * (int64_t)n * n + 2 * n + 1; }
 
-// trapezoid of E * M[:, j] over E (column j, rows 0..n-1), sequential
-__device__ __forceinline__ double column_energy(const double* M, int j, int n,
-                                                const double* E) {
+// trapezoid of E * M[:, c] over E (column c of an LDS tile), sequential
+__device__ __forceinline__ double column_energy(const double* M, int c, int n, const double* E) {
   double acc = 0.0;
   for (int i = 0; i + 1 < n; ++i) {
     const double dx = E[i + 1] - E[i];
-    acc += dx * (E[i + 1] * M[(int64_t)(i + 1) * CNP + j] + E[i] * M[(int64_t)i * CNP + j]) / 2.0;
+    acc += dx * (E[i + 1] * M[(i + 1) * CPIT + c] + E[i] * M[i * CPIT + c]) / 2.0;
   }
   return acc;
 }
 
-__global__ void __launch_bounds__(CTHREADS) cascade_transfer_kernel(
-    prh_cascade cs, const double* __restrict__ contr, int64_t cstride,
-    const double* __restrict__ dtau, const double* __restrict__ dl, double* __restrict__ work,
-    double* __restrict__ tg, double* __restrict__ te, int32_t* __restrict__ iters) {
-  __shared__ double sE[CNP], sdE[CNP], sR[CNP], sloss[CNP], spesc[CNP], scold[CNP], sEin[CNP];
-  __shared__ double sred[CNP];
-  __shared__ int sdone;
-  const int n = cs.n;
-  const int w = blockIdx.x;
-  const int tid = threadIdx.x;
-  const int lane = tid & (WAVE - 1);
-  const int wv = wave_id();
+// IC cooling map before its normalisation, 16 rows of a window: row i cumulates
+// emis / loss along j, relative to column i.
+__global__ void __launch_bounds__(CPREP) cascade_cool_kernel(prh_cascade cs,
+                                                             const double* __restrict__ contr,
+                                                             int64_t cstride,
+                                                             double* __restrict__ work) {
+  __shared__ double sE[CNP], sloss[CNP], tile[CNP * CPIT];
+  const int n = cs.n, tid = threadIdx.x;
+  const int w = blockIdx.x / CTL, i0 = (blockIdx.x % CTL) * 16;
   const double* cw = contr + (int64_t)w * cstride;
-  double* M = work + (int64_t)w * CM_COUNT * CMAT;
-  double* P = M + CM_P * CMAT;
-  double* Sg = M + CM_SG * CMAT;
-  double* De = M + CM_DE * CMAT;
-  double* Mic = M + CM_MIC * CMAT;
-  double* G = M + CM_G * CMAT;
-  double* Ev = M + CM_E * CMAT;
-  double* E1 = M + CM_E1 * CMAT;
-  double* Esc = M + CM_ESC * CMAT;
-  double* Tc = M + CM_T * CMAT;  // G_c of the iteration, until it is added into G
-
-  for (int i = tid; i < CNP; i += CTHREADS) {
-    sE[i] = i < n ? cs.E[i] : 0.0;
-    sdE[i] = i < n ? cs.dE[i] : 0.0;
-  }
-  // emission into E1, pair spectrum into P, every other matrix zeroed: the
-  // padded rows and columns (n <= i, j < 144) take part in the tile products
-  // and must hold zeros, never stale workspace contents
-  for (int64_t t = tid; t < CMAT; t += CTHREADS) {
-    const int i = (int)(t / CNP), j = (int)(t % CNP);
-    const bool in = i < n && j < n;
-    E1[t] = in ? cs.pref_emis[j] * cw[crow_emis(n) + (int64_t)i * n + j] : 0.0;
-    P[t] = in ? cs.pref_pair[j] * cw[crow_pair(n) + (int64_t)i * n + j] : 0.0;
-    Sg[t] = 0.0;
-    De[t] = 0.0;
-    Mic[t] = 0.0;
-    G[t] = (in && i == j) ? 1.0 : 0.0;
-    Ev[t] = 0.0;
-    Esc[t] = 0.0;
-    Tc[t] = 0.0;
-  }
-  __syncthreads();
-  // per column j: pair-matrix energy normalisation, IC emission rate R_j
-  for (int j = tid; j < n; j += CTHREADS) {
-    const double oe = column_energy(P, j, n, sE);
-    if (oe > 0.0)
-      for (int i = 0; i < n; ++i) P[(int64_t)i * CNP + j] = (P[(int64_t)i * CNP + j] / oe) * sE[j];
-    double r = 0.0;
-    for (int i = 0; i < n; ++i) r += E1[(int64_t)i * CNP + j] * sdE[i];
-    sR[j] = r;
-  }
-  if (tid == 0) {
-    const double den = cw[crow_den(n)];
-    const double eps_mean = den > 0.0 ? cw[crow_num(n)] / den : 0.0;
-    sred[0] = eps_mean;
-  }
-  __syncthreads();
-  const double eps_mean = sred[0];
-  for (int j = tid; j < n; j += CTHREADS) {
-    const double pw = cs.pref_emis[j] * cw[crow_power(n) + j];
-    const double rt = cs.pref_emis[j] * cw[crow_rate(n) + j];
-    sloss[j] = pw - rt * eps_mean;
-  }
-  __syncthreads();
-  // Sg, cold flag and the degraded-electron map (column j by one thread, rows
-  // in order as the host's scatter-add)
-  for (int j = tid; j < n; j += CTHREADS) {
-    const double r = sR[j];
-    double eg = 0.0;
-    for (int i = 0; i < n; ++i) {
-      const double s = r > 0.0 ? E1[(int64_t)i * CNP + j] / r : 0.0;
-      Sg[(int64_t)i * CNP + j] = s;
-      eg += (sE[i] * s) * sdE[i];
-    }
-    scold[j] = ((eg < cs.cool_floor * sE[j]) || (r <= 0.0)) ? 1.0 : 0.0;
-    if (r > 0.0) {
-      for (int k = 0; k < n; ++k) {
-        const int b = cs.cic_b[(int64_t)k * n + j];
-        const double wk = Sg[(int64_t)k * CNP + j] * sdE[k];
-        if (b < 0 || !(wk > 0.0)) continue;
-        const double f = cs.cic_f[(int64_t)k * n + j];
-        De[(int64_t)b * CNP + j] += wk * f / sdE[b];
-        De[(int64_t)(b + 1) * CNP + j] += wk * (1.0 - f) / sdE[b + 1];
-      }
+  double* Mic = work + ((int64_t)w * CM_COUNT + CM_MIC) * CMAT;
+  const double den = cw[crow_den(n)];
+  const double eps_mean = den > 0.0 ? cw[crow_num(n)] / den : 0.0;
+  for (int j = tid; j < CNP; j += CPREP) {
+    sE[j] = j < n ? cs.E[j] : 0.0;
+    sloss[j] = 0.0;
+    if (j < n) {
+      const double pw = cs.pref_emis[j] * cw[crow_power(n) + j];
+      const double rt = cs.pref_emis[j] * cw[crow_rate(n) + j];
+      sloss[j] = pw - rt * eps_mean;
     }
   }
-  // IC cooling map: row i cumulates emis/loss along j, relative to column i
-  for (int i = tid; i < n; i += CTHREADS) {
+  __syncthreads();
+  for (int t = tid; t < 16 * CNP; t += CPREP) {
+    const int r = t / CNP, j = t % CNP, i = i0 + r;
+    const double l = sloss[j];
+    const double e = i < n && j < n ? cs.pref_emis[j] * cw[crow_emis(n) + (int64_t)i * n + j] : 0.0;
+    tile[j * CPIT + r] = l > 0.0 ? e / l : 0.0;
+  }
+  __syncthreads();
+  if (tid < 16 && i0 + tid < n) {
+    const int i = i0 + tid;
     double cum = 0.0, prev = 0.0, at_i = 0.0;
     for (int j = 0; j < n; ++j) {
-      const double l = sloss[j];
-      const double g = l > 0.0 ? E1[(int64_t)i * CNP + j] / l : 0.0;
+      const double g = tile[j * CPIT + tid];
       if (j > 0) cum = cum + (sE[j] - sE[j - 1]) * (g + prev) / 2.0;
       prev = g;
       if (j == i) at_i = cum;
-      Mic[(int64_t)i * CNP + j] = j >= i ? cum - at_i : 0.0;
+      tile[j * CPIT + tid] = j >= i ? cum - at_i : 0.0;
     }
-    spesc[i] = exp(-dtau[(int64_t)w * n + i] * dl[w]);
-    sEin[i] = sE[i] * sdE[i];
-  }
-  for (int i = n + tid; i < CNP; i += CTHREADS) {
-    spesc[i] = 0.0;
-    sEin[i] = 0.0;
-    scold[i] = 0.0;
   }
   __syncthreads();
-  for (int j = tid; j < n; j += CTHREADS) {
-    const double oe = column_energy(Mic, j, n, sE);
-    if (oe > 0.0)
-      for (int i = 0; i < n; ++i) Mic[(int64_t)i * CNP + j] = (Mic[(int64_t)i * CNP + j] / oe) * sE[j];
+  for (int t = tid; t < 16 * CNP; t += CPREP) {
+    const int j = t / 16, r = t % 16;
+    Mic[(int64_t)j * CNP + i0 + r] = j < n && i0 + r < n ? tile[j * CPIT + r] : 0.0;
   }
-  __syncthreads();
-  // the four fixed left operands of the iteration stored transposed (k-major):
-  // an operand fragment (16 rows x 4 k) is then four 128-byte row segments
-  double* fixed[4] = {P, Sg, De, Mic};
-  for (int m = 0; m < 4; ++m) {
-    double* X = fixed[m];
-    for (int64_t t = tid; t < CMAT; t += CTHREADS) Tc[t] = X[t];
-    __syncthreads();
-    for (int64_t t = tid; t < CMAT; t += CTHREADS) {
-      const int i = (int)(t / CNP), j = (int)(t % CNP);
-      X[t] = Tc[(int64_t)j * CNP + i];
-    }
-    __syncthreads();
-  }
+}
 
-  const int col = lane & 15;
-  const int kq = lane >> 4;
-  int it = 0;
-  for (it = 1; it <= cs.max_scatter; ++it) {
-    // e1 = e + P ((G - pesc G) dE);  esc += pesc G
-    // unit = 3 row tiles x 1 column tile (27 units): per k-step 3 + 1 operand
-    // loads for 3 products, the loads of CKU k-steps issued together
-#pragma unroll 1
-    for (int u = wv; u < 3 * CTL; u += CWAVES) {
-      const int r0 = (u / CTL) * 48, c0 = (u % CTL) * 16;
-      double4_t acc[3];
-#pragma unroll
-      for (int r = 0; r < 3; ++r) acc[r] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 1
-      for (int k0 = 0; k0 < CNP; k0 += 4 * CKU) {
-        double a[CKU][3], g[CKU];
-#pragma unroll
-        for (int v = 0; v < CKU; ++v) {
-          const int k = k0 + 4 * v + kq;
-#pragma unroll
-          for (int r = 0; r < 3; ++r) a[v][r] = P[(int64_t)k * CNP + r0 + 16 * r + col];
-          g[v] = G[(int64_t)k * CNP + c0 + col];
-        }
-#pragma unroll
-        for (int v = 0; v < CKU; ++v) {
-          const int k = k0 + 4 * v + kq;
-          const double b = (g[v] - spesc[k] * g[v]) * sdE[k];
-#pragma unroll
-          for (int r = 0; r < 3; ++r)
-            acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[v][r], b, acc[r], 0, 0, 0);
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < 3; ++r) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int i = r0 + 16 * r + kq + 4 * v, j = c0 + col;
-          const int64_t o = (int64_t)i * CNP + j;
-          E1[o] = Ev[o] + acc[r][v];
-          Esc[o] += spesc[i] * G[o];
-        }
-      }
-    }
-    __syncthreads();
-    // G_c = Mic (e1 cold dE) -> Tc, G_h = Sg (e1 hot dE) -> G, e = De (e1 hot dE)
-    // -> Ev; unit = one product on 3 x 3 tiles (27 units): per k-step 3 + 3
-    // operand loads for 9 products
-#pragma unroll 1
-    for (int u = wv; u < 27; u += CWAVES) {
-      const int pr = u / 9, st = u % 9;
-      const int r0 = (st / 3) * 48, c0 = (st % 3) * 48;
-      const double* A = pr == 0 ? Mic : (pr == 1 ? Sg : De);
-      const bool cold = pr == 0;
-      double4_t acc[3][3];
-#pragma unroll
-      for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) acc[r][c] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 1
-      for (int k0 = 0; k0 < CNP; k0 += 4 * CKU2) {
-        double a[CKU2][3], e[CKU2][3];
-#pragma unroll
-        for (int v = 0; v < CKU2; ++v) {
-          const int k = k0 + 4 * v + kq;
-#pragma unroll
-          for (int r = 0; r < 3; ++r) a[v][r] = A[(int64_t)k * CNP + r0 + 16 * r + col];
-#pragma unroll
-          for (int c = 0; c < 3; ++c) e[v][c] = E1[(int64_t)k * CNP + c0 + 16 * c + col];
-        }
-#pragma unroll
-        for (int v = 0; v < CKU2; ++v) {
-          const int k = k0 + 4 * v + kq;
-          const bool take = (scold[k] != 0.0) == cold;
-#pragma unroll
-          for (int c = 0; c < 3; ++c) {
-            const double y = take ? e[v][c] * sdE[k] : 0.0;
-#pragma unroll
-            for (int r = 0; r < 3; ++r)
-              acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[v][r], y, acc[r][c], 0, 0, 0);
-          }
-        }
-      }
-      double* out = pr == 0 ? Tc : (pr == 1 ? G : Ev);
-#pragma unroll
-      for (int r = 0; r < 3; ++r) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int i = r0 + 16 * r + kq + 4 * v, j = c0 + 16 * c + col;
-            const int64_t o = (int64_t)i * CNP + j;
-            out[o] = acc[r][c][v];
-            if (cold) Esc[o] += spesc[i] * acc[r][c][v];
-          }
-        }
-      }
-    }
-    __syncthreads();
-    // G = (G_h + G_c) - pesc G_c
-    for (int64_t t = tid; t < CMAT; t += CTHREADS) {
-      const int i = (int)(t / CNP);
-      G[t] = (G[t] + Tc[t]) - spesc[i] * Tc[t];
-    }
-    __syncthreads();
-    // energy still in G and e per input column, relative to the column's input
-    double worst = -1.0;
-    for (int j = tid; j < n; j += CTHREADS) {
-      double eg = 0.0, ee = 0.0;
+// P, Sg, De and the normalised Mic of 16 columns of a window.  The sums of a
+// column run in row order (as the host's), one thread each: wave 0 the IC
+// emission with its degraded electrons, wave 1 the pairs, wave 2 the cooling.
+__global__ void __launch_bounds__(CPREP) cascade_columns_kernel(
+    prh_cascade cs, const double* __restrict__ contr, int64_t cstride,
+    const double* __restrict__ dtau, const double* __restrict__ dl, double* __restrict__ work) {
+  __shared__ double sE[CNP], sdE[CNP], snorm[3][16];
+  __shared__ double ts[CNP * CPIT], td[CNP * CPIT], tp[CNP * CPIT], tm[CNP * CPIT];
+  const int n = cs.n, tid = threadIdx.x;
+  const int w = blockIdx.x / CTL, cb = blockIdx.x % CTL, j0 = cb * 16;
+  const double* cw = contr + (int64_t)w * cstride;
+  double* M = work + (int64_t)w * CM_COUNT * CMAT;
+  double* info = M + CM_INFO * CMAT;
+  for (int i = tid; i < CNP; i += CPREP) {
+    sE[i] = i < n ? cs.E[i] : 0.0;
+    sdE[i] = i < n ? cs.dE[i] : 0.0;
+  }
+  for (int t = tid; t < 16 * CNP; t += CPREP) {
+    const int i = t / 16, c = t % 16, j = j0 + c;
+    const bool in = i < n && j < n;
+    const int64_t q = (int64_t)i * n + j;
+    ts[i * CPIT + c] = in ? cs.pref_emis[j] * cw[crow_emis(n) + q] : 0.0;
+    tp[i * CPIT + c] = in ? cs.pref_pair[j] * cw[crow_pair(n) + q] : 0.0;
+    td[i * CPIT + c] = 0.0;
+    tm[(t % CNP) * CPIT + t / CNP] = M[CM_MIC * CMAT + (int64_t)(j0 + t / CNP) * CNP + t % CNP];
+  }
+  if (tid < 48) snorm[tid / 16][tid % 16] = 0.0;
+  __syncthreads();
+  const int wv = wave_id(), c = tid & (WAVE - 1), j = j0 + c;
+  if (c < 16 && j < n) {
+    if (wv == 0) {
+      double r = 0.0;
+      for (int i = 0; i < n; ++i) r += ts[i * CPIT + c] * sdE[i];
+      double eg = 0.0;
       for (int i = 0; i < n; ++i) {
-        eg += sEin[i] * G[(int64_t)i * CNP + j];
-        ee += sEin[i] * Ev[(int64_t)i * CNP + j];
+        const double v = r > 0.0 ? ts[i * CPIT + c] / r : 0.0;
+        ts[i * CPIT + c] = v;
+        eg += (sE[i] * v) * sdE[i];
       }
-      worst = fmax(worst, (eg + ee) / sEin[j]);
-    }
-    if (tid < CNP) sred[tid] = worst;
-    __syncthreads();
-    if (tid == 0) {
-      double m = sred[0];
-      for (int j = 1; j < CNP; ++j) m = fmax(m, sred[j]);
-      sdone = m < cs.tol ? 1 : 0;
-    }
-    __syncthreads();
-    if (sdone) {
-      for (int64_t t = tid; t < CMAT; t += CTHREADS) {
-        const int i = (int)(t / CNP);
-        Esc[t] += spesc[i] * G[t];
+      info[CI_COLD + j] = ((eg < cs.cool_floor * sE[j]) || (r <= 0.0)) ? 1.0 : 0.0;
+      if (r > 0.0) {
+        for (int k = 0; k < n; ++k) {
+          const int b = cs.cic_b[(int64_t)k * n + j];
+          const double f = cs.cic_f[(int64_t)k * n + j];
+          const double wk = ts[k * CPIT + c] * sdE[k];
+          if (b < 0 || !(wk > 0.0)) continue;
+          td[b * CPIT + c] += wk * f / sdE[b];
+          td[(b + 1) * CPIT + c] += wk * (1.0 - f) / sdE[b + 1];
+        }
       }
-      __syncthreads();
-      break;
+    } else if (wv == 1) {
+      snorm[1][c] = column_energy(tp, c, n, sE);
+    } else if (wv == 2) {
+      snorm[2][c] = column_energy(tm, c, n, sE);
     }
   }
-  if (tid == 0) iters[w] = it > cs.max_scatter ? cs.max_scatter : it;
-  // outputs: T_gamma = esc, T_electron = esc (Mic dE)
-  double* tgw = tg + (int64_t)w * n * n;
-  double* tew = te + (int64_t)w * n * n;
-  for (int64_t t = tid; t < (int64_t)n * n; t += CTHREADS) {
-    const int i = (int)(t / n), j = (int)(t % n);
-    tgw[t] = Esc[(int64_t)i * CNP + j];
+  if (tid < 16 && j0 + tid >= n) info[CI_COLD + j0 + tid] = 0.0;
+  __syncthreads();
+  bool odd = false;  // a nonzero below the diagonal tile, or not finite
+  for (int t = tid; t < 16 * CNP; t += CPREP) {
+    const int cc = t / CNP, i = t % CNP, jj = j0 + cc, o = i * CPIT + cc;
+    double p = tp[o], m = tm[o];
+    if (snorm[1][cc] > 0.0) p = (p / snorm[1][cc]) * sE[jj];
+    if (snorm[2][cc] > 0.0) m = (m / snorm[2][cc]) * sE[jj];
+    const int64_t q = (int64_t)jj * CNP + i;
+    M[CM_P * CMAT + q] = p;
+    M[CM_SG * CMAT + q] = ts[o];
+    M[CM_DE * CMAT + q] = td[o];
+    M[CM_MIC * CMAT + q] = m;
+    odd = odd || !isfinite(p) || !isfinite(ts[o]) || !isfinite(td[o]) || !isfinite(m);
+    if (i >= j0 + 16) odd = odd || p != 0.0 || ts[o] != 0.0 || td[o] != 0.0 || m != 0.0;
   }
-#pragma unroll 1
-  for (int q = 0; q < CTPW; ++q) {
-    const int t = wv + CWAVES * q;
-    if (t >= CTILES) break;
-    const int r0 = (t / CTL) * 16, c0 = (t % CTL) * 16;
+  if (tid < 16 && j0 + tid < n)
+    odd = odd || !isfinite(exp(-dtau[(int64_t)w * n + j0 + tid] * dl[w])) || !isfinite(sdE[j0 + tid]);
+  if (__syncthreads_or(odd ? 1 : 0)) {
+    if (tid == 0) info[CI_TRI + cb] = 0.0;
+  } else if (tid == 0) {
+    info[CI_TRI + cb] = 1.0;
+  }
+}
+
+struct CascadeLds {
+  double dE[CNP], pesc[CNP], cold[CNP], Ein[CNP];
+  double y[CNP * 16], e[CNP * 16];  // right operands of the pairs and of the scatter
+  double red[CWAVES][16];
+};
+struct CascadeTiles {  // this wave's two row tiles of one column block
+  double4_t G[2], E[2], X[2];  // X: escaped
+};
+// Which tiles of a window take part, the same for all its column blocks.
+struct CascadeForm {
+  bool tri;
+  uint32_t cold, hot;  // 16-energy tiles that hold cold, hot electrons
+};
+
+__device__ __forceinline__ CascadeForm cascade_setup(const prh_cascade& cs, CascadeLds& L, int w,
+                                                     const double* dtau, const double* dl,
+                                                     const double* info) {
+  const int n = cs.n;
+  for (int i = threadIdx.x; i < CNP; i += CTHREADS) {
+    L.dE[i] = i < n ? cs.dE[i] : 0.0;
+    L.pesc[i] = i < n ? exp(-dtau[(int64_t)w * n + i] * dl[w]) : 0.0;
+    L.cold[i] = info[CI_COLD + i];
+    L.Ein[i] = i < n ? cs.E[i] * cs.dE[i] : 0.0;
+  }
+  __syncthreads();
+  CascadeForm f{true, 0, 0};
+  for (int b = 0; b < CTL; ++b) f.tri = f.tri && info[CI_TRI + b] != 0.0;
+  for (int i = 0; i < CNP; ++i) (L.cold[i] != 0.0 ? f.cold : f.hot) |= 1u << (i / 16);
+  if (!f.tri) f.cold = f.hot = (1u << CTL) - 1;
+  f.tri = __builtin_amdgcn_readfirstlane(f.tri);
+  f.cold = __builtin_amdgcn_readfirstlane(f.cold);
+  f.hot = __builtin_amdgcn_readfirstlane(f.hot);
+  return f;
+}
+
+// Row tile of slot t of this wave, or -1.
+__device__ __forceinline__ int cascade_tile(const CascadeForm& f, int cb, int t) {
+  const int last = f.tri ? cb : CTL - 1, v = wave_id();
+  if (t == 0) return v <= last - v ? v : -1;
+  return v < last - v ? last - v : -1;
+}
+
+// One iteration of column block cb; true when every column is below tol.
+__device__ __forceinline__ bool cascade_iterate(const prh_cascade& cs, CascadeLds& L,
+                                                const CascadeForm& f, const double* M, int cb,
+                                                CascadeTiles& T) {
+  const int lane = threadIdx.x & (WAVE - 1), col = lane & 15, kq = lane >> 4;
+  const int kend = f.tri ? cb + 1 : CTL;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int r = cascade_tile(f, cb, t);
+    if (r < 0) continue;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = 16 * r + kq + 4 * v;
+      const double g = T.G[t][v];
+      L.y[i * 16 + col] = (g - L.pesc[i] * g) * L.dE[i];
+      T.X[t][v] += L.pesc[i] * g;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int r = cascade_tile(f, cb, t);
+    if (r < 0) continue;
     double4_t acc = {0.0, 0.0, 0.0, 0.0};
-    for (int k0 = 0; k0 < CNP; k0 += 4) {
-      const int k = k0 + kq;
-      const int j = c0 + col;
-      const double a = Esc[(int64_t)(r0 + col) * CNP + k];
-      const double b = Mic[(int64_t)j * CNP + k] * sdE[j];  // Mic is stored transposed
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
+#pragma unroll 1
+    for (int kt = f.tri ? r : 0; kt < kend; ++kt) {
+      double a[4], b[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int k = 16 * kt + 4 * u + kq;
+        a[u] = M[CM_P * CMAT + k * CNP + 16 * r + col];
+        b[u] = L.y[k * 16 + col];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b[u], acc, 0, 0, 0);
     }
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int i = r0 + kq + 4 * v, j = c0 + col;
-      if (i < n && j < n) tew[(int64_t)i * n + j] = acc[v];
+      const int i = 16 * r + kq + 4 * v;
+      L.e[i * 16 + col] = (T.E[t][v] + acc[v]) * L.dE[i];
+    }
+  }
+  __syncthreads();
+  double eg = 0.0, ee = 0.0;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int r = cascade_tile(f, cb, t);
+    if (r < 0) continue;
+    double4_t gc = {0.0, 0.0, 0.0, 0.0}, gh = gc, en = gc;
+#pragma unroll 1
+    for (int kt = f.tri ? r : 0; kt < kend; ++kt) {
+      double y[4];
+      bool cold[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int k = 16 * kt + 4 * u + kq;
+        y[u] = L.e[k * 16 + col];
+        cold[u] = L.cold[k] != 0.0;
+      }
+      const double* A = M + (16 * kt + kq) * CNP + 16 * r + col;
+      if (f.cold >> kt & 1) {
+        double a[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) a[u] = A[CM_MIC * CMAT + 4 * u * CNP];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          gc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], cold[u] ? y[u] : 0.0, gc, 0, 0, 0);
+      }
+      if (f.hot >> kt & 1) {
+        double a[4], b[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          a[u] = A[CM_SG * CMAT + 4 * u * CNP];
+          b[u] = A[CM_DE * CMAT + 4 * u * CNP];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const double yh = cold[u] ? 0.0 : y[u];
+          gh = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], yh, gh, 0, 0, 0);
+          en = __builtin_amdgcn_mfma_f64_16x16x4f64(b[u], yh, en, 0, 0, 0);
+        }
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = 16 * r + kq + 4 * v;
+      T.X[t][v] += L.pesc[i] * gc[v];
+      T.G[t][v] = (gh[v] + gc[v]) - L.pesc[i] * gc[v];
+      eg += L.Ein[i] * T.G[t][v];
+      ee += L.Ein[i] * en[v];
+    }
+    T.E[t] = en;
+  }
+  // energy still in G and e per input column, relative to the column's input
+  double left = eg + ee;
+  left += __shfl_xor(left, 16);
+  left += __shfl_xor(left, 32);
+  if (lane < 16) L.red[wave_id()][lane] = left;
+  __syncthreads();  // also: L.e is consumed before the next iteration writes it
+  double tot = 0.0;
+#pragma unroll
+  for (int v = 0; v < CWAVES; ++v) tot += L.red[v][col];
+  const int j = cb * 16 + col;
+  // a NaN column does not hold the others up (fmax over the columns)
+  return __all(fmax(-1.0, j < cs.n ? tot / L.Ein[j] : -1.0) < cs.tol);
+}
+
+__device__ __forceinline__ void cascade_load(const CascadeForm& f, const double* M, int cb,
+                                             CascadeTiles& T) {
+  const int lane = threadIdx.x & (WAVE - 1), col = lane & 15, kq = lane >> 4;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int r = cascade_tile(f, cb, t);
+    if (r < 0) continue;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int o = (16 * r + kq + 4 * v) * CNP + cb * 16 + col;
+      T.G[t][v] = M[CM_G * CMAT + o];
+      T.E[t][v] = M[CM_E * CMAT + o];
+      T.X[t][v] = M[CM_ESC * CMAT + o];
+    }
+  }
+}
+__device__ __forceinline__ void cascade_store(const CascadeForm& f, double* M, int cb,
+                                              const CascadeTiles& T) {
+  const int lane = threadIdx.x & (WAVE - 1), col = lane & 15, kq = lane >> 4;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int r = cascade_tile(f, cb, t);
+    if (r < 0) continue;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int o = (16 * r + kq + 4 * v) * CNP + cb * 16 + col;
+      M[CM_G * CMAT + o] = T.G[t][v];
+      M[CM_E * CMAT + o] = T.E[t][v];
+      M[CM_ESC * CMAT + o] = T.X[t][v];
+    }
+  }
+}
+__device__ __forceinline__ int cascade_most(const double* info) {
+  double m = info[CI_ITS];
+  for (int b = 1; b < CTL; ++b) m = fmax(m, info[CI_ITS + b]);
+  return (int)m;
+}
+__device__ __forceinline__ bool cascade_done(const double* info) {
+  bool done = true;
+  for (int b = 0; b < CTL; ++b) done = done && info[CI_DONE + b] != 0.0;
+  return done;
+}
+
+// First launch: every column block to its own convergence.  The wide blocks
+// (last columns) start first.
+__global__ void __launch_bounds__(CTHREADS, 4) cascade_first_kernel(
+    prh_cascade cs, const double* __restrict__ dtau, const double* __restrict__ dl, double* work,
+    int nwin) {
+  __shared__ CascadeLds L;
+  const int cb = CTL - 1 - (int)(blockIdx.x / nwin), w = blockIdx.x % nwin;
+  double* M = work + (int64_t)w * CM_COUNT * CMAT;
+  double* info = M + CM_INFO * CMAT;
+  const CascadeForm f = cascade_setup(cs, L, w, dtau, dl, info);
+  const int lane = threadIdx.x & (WAVE - 1), col = lane & 15, kq = lane >> 4;
+  CascadeTiles T;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int r = cascade_tile(f, cb, t);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = 16 * r + kq + 4 * v;
+      T.G[t][v] = r >= 0 && i == cb * 16 + col && i < cs.n ? 1.0 : 0.0;
+      T.E[t][v] = 0.0;
+      T.X[t][v] = 0.0;
+    }
+  }
+  int it = 0;
+  bool done = false;
+  while (!done && it < cs.max_scatter) {
+    done = cascade_iterate(cs, L, f, M, cb, T);
+    ++it;
+  }
+  cascade_store(f, M, cb, T);
+  if (f.tri) {  // the zero tiles below the diagonal
+    for (int t = threadIdx.x; t < (CNP - 16 * (cb + 1)) * 16; t += CTHREADS) {
+      const int o = (16 * (cb + 1) + t / 16) * CNP + cb * 16 + t % 16;
+      M[CM_G * CMAT + o] = 0.0;
+      M[CM_E * CMAT + o] = 0.0;
+      M[CM_ESC * CMAT + o] = 0.0;
+    }
+  }
+  if (threadIdx.x == 0) {
+    info[CI_ITS + cb] = it;
+    info[CI_DONE + cb] = done ? 1.0 : 0.0;
+  }
+}
+
+// Second launch: every block on to the window's largest count.  The counts stay
+// as the first launch left them: other blocks of the window still read them.
+__global__ void __launch_bounds__(CTHREADS, 4) cascade_level_kernel(
+    prh_cascade cs, const double* __restrict__ dtau, const double* __restrict__ dl, double* work,
+    int nwin) {
+  __shared__ CascadeLds L;
+  const int cb = CTL - 1 - (int)(blockIdx.x / nwin), w = blockIdx.x % nwin;
+  double* M = work + (int64_t)w * CM_COUNT * CMAT;
+  double* info = M + CM_INFO * CMAT;
+  const int from = (int)info[CI_ITS + cb], most = cascade_most(info);
+  if (from == most) return;
+  const CascadeForm f = cascade_setup(cs, L, w, dtau, dl, info);
+  CascadeTiles T;
+  cascade_load(f, M, cb, T);
+  bool done = false;
+#pragma unroll 1
+  for (int it = from; it < most; ++it) done = cascade_iterate(cs, L, f, M, cb, T);
+  cascade_store(f, M, cb, T);
+  if (threadIdx.x == 0) info[CI_DONE + cb] = done ? 1.0 : 0.0;
+}
+
+// Third launch: a window with a block that rose above tol again goes on, all its
+// columns an iteration at a time (no window has been seen to).
+__global__ void __launch_bounds__(CTHREADS, 4) cascade_rest_kernel(
+    prh_cascade cs, const double* __restrict__ dtau, const double* __restrict__ dl, double* work,
+    int32_t* __restrict__ iters) {
+  __shared__ CascadeLds L;
+  const int w = blockIdx.x;
+  double* M = work + (int64_t)w * CM_COUNT * CMAT;
+  double* info = M + CM_INFO * CMAT;
+  int it = cascade_most(info);
+  bool done = cascade_done(info);
+  if (!done && it < cs.max_scatter) {
+    const CascadeForm f = cascade_setup(cs, L, w, dtau, dl, info);
+    while (!done && it < cs.max_scatter) {
+      done = true;
+#pragma unroll 1
+      for (int cb = 0; cb < CTL; ++cb) {
+        CascadeTiles T;
+        cascade_load(f, M, cb, T);
+        done = cascade_iterate(cs, L, f, M, cb, T) && done;
+        cascade_store(f, M, cb, T);
+        __syncthreads();  // L.red is consumed
+      }
+      ++it;
+    }
+    if (threadIdx.x == 0)
+      for (int b = 0; b < CTL; ++b) info[CI_DONE + b] = done ? 1.0 : 0.0;
+  }
+  if (threadIdx.x == 0) iters[w] = it;
+}
+
+// T_gamma = esc (what is left in G escapes once converged) and T_electron =
+// esc (Mic dE), 16 rows of a window.
+__global__ void __launch_bounds__(CTHREADS) cascade_output_kernel(
+    prh_cascade cs, const double* __restrict__ dtau, const double* __restrict__ dl,
+    const double* __restrict__ work, double* __restrict__ tg, double* __restrict__ te) {
+  __shared__ double x[16 * (CNP + 1)];
+  const int n = cs.n, lane = threadIdx.x & (WAVE - 1), col = lane & 15, kq = lane >> 4;
+  const int w = blockIdx.x / CTL, r0 = (blockIdx.x % CTL) * 16;
+  const double* M = work + (int64_t)w * CM_COUNT * CMAT;
+  const double* info = M + CM_INFO * CMAT;
+  const bool done = cascade_done(info);
+  for (int t = threadIdx.x; t < 16 * CNP; t += CTHREADS) {
+    const int r = t / CNP, j = t % CNP, i = r0 + r;
+    double v = M[CM_ESC * CMAT + (int64_t)i * CNP + j];
+    if (done && i < n)
+      v += exp(-dtau[(int64_t)w * n + i] * dl[w]) * M[CM_G * CMAT + (int64_t)i * CNP + j];
+    x[r * (CNP + 1) + j] = v;
+    if (i < n && j < n) tg[((int64_t)w * n + i) * n + j] = v;
+  }
+  __syncthreads();
+  for (int ct = wave_id(); ct < CTL; ct += CWAVES) {
+    const int j = ct * 16 + col;
+    const double de = j < n ? cs.dE[j] : 0.0;
+    double4_t acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int k0 = 0; k0 < CNP; k0 += 4) {
+      const double b = M[CM_MIC * CMAT + (int64_t)j * CNP + k0 + kq] * de;  // stored transposed
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[col * (CNP + 1) + k0 + kq], b, acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = r0 + kq + 4 * v;
+      if (i < n && j < n) te[((int64_t)w * n + i) * n + j] = acc[v];
     }
   }
 }
@@ -2945,8 +3126,17 @@ int32_t prh_cascade_transfer(const prh_cascade* cs, const double* contr, int64_t
   if (cstride < rows) return set_error("prh_cascade_transfer: cstride below the contraction rows");
   if (work_bytes < (int64_t)nwin * CM_COUNT * CMAT * 8)
     return set_error("prh_cascade_transfer: workspace below 9 * 144 * 144 doubles per window");
-  hipLaunchKernelGGL(cascade_transfer_kernel, dim3((unsigned)nwin), dim3(CTHREADS), 0,
-                     (hipStream_t)stream, *cs, contr, cstride, dtau, dl, work, tg, te, iters);
+  const hipStream_t st = (hipStream_t)stream;
+  const dim3 blocks((unsigned)nwin * CTL);
+  hipLaunchKernelGGL(cascade_cool_kernel, blocks, dim3(CPREP), 0, st, *cs, contr, cstride, work);
+  hipLaunchKernelGGL(cascade_columns_kernel, blocks, dim3(CPREP), 0, st, *cs, contr, cstride, dtau,
+                     dl, work);
+  hipLaunchKernelGGL(cascade_first_kernel, blocks, dim3(CTHREADS), 0, st, *cs, dtau, dl, work, nwin);
+  hipLaunchKernelGGL(cascade_level_kernel, blocks, dim3(CTHREADS), 0, st, *cs, dtau, dl, work, nwin);
+  hipLaunchKernelGGL(cascade_rest_kernel, dim3((unsigned)nwin), dim3(CTHREADS), 0, st, *cs, dtau, dl,
+                     work, iters);
+  hipLaunchKernelGGL(cascade_output_kernel, blocks, dim3(CTHREADS), 0, st, *cs, dtau, dl, work, tg,
+                     te);
   return check_hip(hipGetLastError(), "prh_cascade_transfer launch");
 }
 
