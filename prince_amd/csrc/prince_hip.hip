@@ -122,40 +122,61 @@ __global__ void __launch_bounds__(FOLD_THREADS) fold_gemm_mfma(const double* __r
 }
 
 // Same product for a contraction length above 128 (the cascade tensors: 400
-// and 256 target-photon points): the kernel rows are re-read from cache per
-// 16-window tile instead of held in registers.
+// and 256 target-photon points).  A wave takes 16 kernel rows and CONTR_TILES
+// tiles of 16 windows at once: one load of a kernel value serves 3 products, and
+// groups of windows are workgroups of their own (neighbours in the grid, so that
+// they meet the same kernel rows in cache).  288 windows of 37266 x 400 values:
+// 1.20 ms with a tile at a time in 2600 waves, 0.64 ms so.
+constexpr int CONTR_TILES = 3;
 __global__ void __launch_bounds__(THREADS) contract_rows_mfma(const double* __restrict__ kern,
                                                               int64_t nrows, int kdim,
                                                               const double* __restrict__ vec,
-                                                              int nvec, double* __restrict__ out,
+                                                              int nvec, int groups,
+                                                              double* __restrict__ out,
                                                               int64_t out_stride) {
+  constexpr int CT = CONTR_TILES;
   const int lane = threadIdx.x & (WAVE - 1);
-  const int64_t wave = (int64_t)blockIdx.x * WAVES_PER_BLOCK + wave_id();
+  const int64_t wave = (int64_t)(blockIdx.x / groups) * WAVES_PER_BLOCK + wave_id();
+  const int w0 = (int)(blockIdx.x % groups) * (16 * CT);
   const int64_t r0 = wave * 16;
   if (r0 >= nrows) return;
   const int col = lane & 15;
   const int kq = lane >> 4;
   const int64_t r = r0 + col;
   const double* kr = kern + (r < nrows ? r : nrows - 1) * (int64_t)kdim;
-  for (int w0 = 0; w0 < nvec; w0 += 16) {
-    double4_t acc = {0.0, 0.0, 0.0, 0.0};
-    const int wa = w0 + col;
-    const double* va = vec + (int64_t)(wa < nvec ? wa : nvec - 1) * kdim;
-    for (int k0 = 0; k0 < kdim; k0 += 16) {
-      double a[4], b[4];
+  const int tiles = (nvec - w0 + 15) / 16 < CT ? (nvec - w0 + 15) / 16 : CT;
+  const double* va[CT];
+  double4_t acc[CT];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int k = k0 + 4 * u + kq;
-        a[u] = (wa < nvec && k < kdim) ? va[k] : 0.0;
-        b[u] = (r < nrows && k < kdim) ? kr[k] : 0.0;
-      }
+  for (int c = 0; c < CT; ++c) {
+    const int wa = w0 + 16 * c + col;
+    va[c] = vec + (int64_t)(wa < nvec ? wa : nvec - 1) * kdim;
+    acc[c] = {0.0, 0.0, 0.0, 0.0};
+  }
+  for (int k0 = 0; k0 < kdim; k0 += 16) {
+    double a[CT][4], b[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b[u], acc, 0, 0, 0);
+    for (int u = 0; u < 4; ++u) {
+      const int k = k0 + 4 * u + kq;
+      b[u] = (r < nrows && k < kdim) ? kr[k] : 0.0;
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+        a[c][u] = (c < tiles && w0 + 16 * c + col < nvec && k < kdim) ? va[c][k] : 0.0;
     }
 #pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      if (c >= tiles) break;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[c][u], b[u], acc[c], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < CT; ++c) {
+#pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int w = w0 + kq + 4 * v;
-      if (w < nvec && r < nrows) out[(int64_t)w * out_stride + r] = acc[v];
+      const int w = w0 + 16 * c + kq + 4 * v;
+      if (w < nvec && r < nrows) out[(int64_t)w * out_stride + r] = acc[c][v];
     }
   }
 }
@@ -2250,8 +2271,9 @@ void launch_adjoint_two(const prh_operator& op, const prh_schedule& sch, const p
 //
 // Bound by the serial chain of an iteration (34 to 42 iterations of three
 // barriers and up to 9 tiles of k).  288 windows of 136 bins: 17.45 ms with a
-// workgroup a window and full matrices, 4.42 ms so (1.38 ms the first launch,
-// 0.83 the second, 0.41 the columns, 1.2 the contraction before).
+// workgroup a window and full matrices, 4.42 ms so, 3.60 with the
+// contraction of three window tiles a wave (1.37 ms the first launch, 0.82 the second, 0.41 the
+// columns, 0.64 the contraction).
 // ---------------------------------------------------------------------------
 constexpr int CNP = 144;              // padded EM dimension (n <= 144)
 constexpr int CTL = CNP / 16;         // 9 tiles per matrix side
@@ -2860,9 +2882,14 @@ int32_t prh_fold_gemm(const double* kern, int64_t nrows, int32_t dph, const doub
     hipLaunchKernelGGL(fold_gemm_mfma, dim3((unsigned)((waves + FOLD_WAVES - 1) / FOLD_WAVES)),
                        dim3(FOLD_THREADS), 0, (hipStream_t)stream, kern, nrows, (int)dph, phot,
                        (int)nwin, out, out_stride);
-  else
-    hipLaunchKernelGGL(contract_rows_mfma, dim3((unsigned)blocks), dim3(THREADS), 0,
-                       (hipStream_t)stream, kern, nrows, (int)dph, phot, (int)nwin, out, out_stride);
+  else {
+    const int groups = (nwin + 16 * CONTR_TILES - 1) / (16 * CONTR_TILES);
+    // beyond a grid's 2^32 threads the output alone exceeds the card's memory
+    if (blocks * groups * THREADS > 0xffffffffLL) return set_error("prh_fold_gemm: too many rows");
+    hipLaunchKernelGGL(contract_rows_mfma, dim3((unsigned)(blocks * groups)), dim3(THREADS), 0,
+                       (hipStream_t)stream, kern, nrows, (int)dph, phot, (int)nwin, groups, out,
+                       out_stride);
+  }
   return check_hip(hipGetLastError(), "prh_fold_gemm launch");
 }
 
