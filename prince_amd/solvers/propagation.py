@@ -1078,12 +1078,13 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
 
     # ---------------------------------------------------------------- autotuner
     def tuning_candidates(self, K):
-        """Stage configurations the autotuner times for K right-hand sides:
-        right-hand sides per wave (kt), part budget (block cost per wave part,
-        i.e. rows per wave), waves per workgroup, the dense-row mode and, with
-        dense rows as split rows, row-pair tasks on or off."""
+        """Configurations the autotuner times for K right-hand sides: the march
+        as one launch, then the stage kernels over right-hand sides per wave
+        (kt), part budget (block cost per wave part, i.e. rows per wave), waves
+        per workgroup, the dense-row mode and, with dense rows as split rows,
+        row-pair tasks on or off."""
         kts = [kt for kt in (8, 4, 2, 1) if kt <= K][:2]
-        out = []
+        out = [{("team", K): True}]
         for kt in kts:
             for pc in (48, 96) if K >= 8 else (12, 24):
                 for wgw in (8, 16):
