@@ -15,9 +15,9 @@
 // invalidation is needed, and a team barrier costs 1.5 us (32 workgroups of
 // one XCD) to 2.6 us (256).  A full agent-scope release / acquire pair instead
 // measured 37 us per stage: it writes back and invalidates the whole L2.
-// Measured per stage of the A <= 56 run, stage kernels -> march: K = 1 11.6 ->
-// 6.3 us, K = 7 19.9 -> 6.6, K = 64 33 -> 17, K = 300 129 -> 45, K = 512 92 -> 82;
-// two fields, K = 48: 48 -> 21.
+// Measured per stage of the A <= 56 run, stage kernels -> march: K = 1 11.5 ->
+// 6.3 us, K = 7 20 -> 6.8, K = 64 33 -> 16.5, K = 300 129 -> 45, K = 512 92 -> 75;
+// two fields, K = 48: 48 -> 21.6.
 //
 // Teams are workgroups blockIdx % nteam, which the dispatcher places on one
 // XCD (nteam = 8) or on a pair of XCDs (nteam = 4); only speed depends on that
@@ -319,7 +319,8 @@ __device__ __forceinline__ void team_epilogue(COp& op, CSt& st,
       const d2 kx = f.kap * xo[p];
       // stencil neighbours of bins 2 l and 2 l + 1, added in the order -3 .. 3.
       // Past the ends of a half the shifts bring the other column's bins, which
-      // meet coefficients that are exactly zero; masked unless all are finite.
+      // meet coefficients that are exactly zero; masked unless all are finite
+      // (K = 64 33.3 -> 32.7 ms per 2000 stages with the masks off).
       double m1 = lane_prev(kx.y);  // bin 2 l - 1
       double m2 = lane_prev(kx.x);  // bin 2 l - 2
       double m3 = lane_prev(m1);    // bin 2 l - 3
