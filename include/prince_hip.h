@@ -362,7 +362,7 @@ typedef struct prh_team {
   int32_t red_slots; /* LDS rows of the mother groups' partial sums */
   int32_t pair_rows; /* tasks hold row pairs */
   int32_t coef_slots; /* LDS rows of staged source coefficients: >= J x columns of a team / 64 */
-  int32_t pad_;
+  int32_t spin_limit; /* polls after which a wait between workgroups gives up; 0: 2^25 */
   const int32_t* lds_ptr;
   const int32_t* lds_voff;
   const int32_t* wave_ptr;
@@ -389,7 +389,11 @@ typedef struct prh_team {
  * op->blocks are not used.  The launch needs nteam * size CUs with
  * 8 * 64 * (11 + 2 coef_slots + red_slots + lds_slots) bytes of LDS each (two fields: 13 and
  * twice lds_slots).  Returns 2 (nothing launched) when the device cannot hold
- * that grid or the stream is capturing. */
+ * that grid or the stream is capturing.
+ * The workgroups wait for each other; marches of one process on one device run one
+ * after the other.  A wait that gives up ends the march; x, the record arrays and
+ * em_w of the range are then NaN (the status is still 0: the launch is
+ * asynchronous). */
 int32_t prh_team_march(const prh_operator* op, const prh_schedule* sch, const prh_state* st,
                        const prh_team* tm, int32_t k_begin, int32_t k_end, void* stream);
 
@@ -400,7 +404,8 @@ int32_t prh_team_march(const prh_operator* op, const prh_schedule* sch, const pr
  * diagonal (0, or negative), diagonals (<= 8, none right of the main one)}, the
  * diagonal blocks first, at most 64 entries a row; a wave takes every
  * `column groups`-th pair of its team's columns.  Dense and tail fields are not
- * used.  Returns 2 (nothing launched) as prh_team_march. */
+ * used.  Returns 2 (nothing launched) as prh_team_march; a sweep whose wait gave up
+ * leaves NaN in lam, gdot and the source accumulators. */
 int32_t prh_team_adjoint(const prh_operator* opT, const prh_schedule* sch, const prh_adjoint* adj,
                          const prh_team* tm, int32_t k_begin, int32_t k_end, void* stream);
 

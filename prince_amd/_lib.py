@@ -259,7 +259,7 @@ class PrhTeam(ctypes.Structure):
         ("red_slots", _i32),
         ("pair_rows", _i32),
         ("coef_slots", _i32),
-        ("pad_", _i32),
+        ("spin_limit", _i32),
         ("lds_ptr", _p),
         ("lds_voff", _p),
         ("wave_ptr", _p),

@@ -41,9 +41,12 @@
 // 16-byte ones reach 32 TB/s, with or without sc1; a shift by one bin also
 // moves half as many registers.
 //
-// Every wait is bounded: a workgroup that polls SPIN_LIMIT times without
-// progress raises the abort word, all workgroups leave, and the state is
-// filled with NaN.
+// Every wait is bounded: a workgroup that polls SPIN_LIMIT times (prh_team.spin_limit)
+// without progress raises the abort word and leaves, and the others do when they
+// next wait.  Which of them still stored results is then a matter of timing, so a
+// launch behind the march reads the word and, where it is raised, fills with NaN
+// everything that march writes for its caller: no result of an aborted march, nor
+// of what follows from it, is finite.
 
 #include <hip/hip_runtime.h>
 
@@ -794,11 +797,12 @@ __device__ __forceinline__ void dense_partial(COp& op, __amdgpu_buffer_rsrc_t y,
 // Arrive at and wait for a team barrier.  Stores of every wave have reached the
 // coherence point before the arrival (vmcnt(0) of sc1 stores).  Returns false
 // when the march is aborted.
-__device__ __forceinline__ bool wait_count(const uint32_t* c, uint32_t target, uint32_t* abort_w) {
+__device__ __forceinline__ bool wait_count(const uint32_t* c, uint32_t target, uint32_t* abort_w,
+                                           int limit) {
   int spins = 0;
   while (__hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-    if ((++spins & 1023) == 0 &&
-        (spins >= SPIN_LIMIT ||
+    if (++spins >= limit ||
+        ((spins & 1023) == 0 &&
          __hip_atomic_load(abort_w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
       __hip_atomic_store(abort_w, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       return false;
@@ -808,7 +812,7 @@ __device__ __forceinline__ bool wait_count(const uint32_t* c, uint32_t target, u
 }
 __device__ __forceinline__ bool team_barrier(uint32_t* sub, uint32_t nsubwg, uint32_t* root,
                                              uint32_t nsub, uint32_t epoch, uint32_t* abort_w,
-                                             int* bad) {
+                                             int limit, int* bad) {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
@@ -820,10 +824,10 @@ __device__ __forceinline__ bool team_barrier(uint32_t* sub, uint32_t nsubwg, uin
           __hip_atomic_fetch_add(sub, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (old + 1 == epoch * nsubwg)
         __hip_atomic_fetch_add(root, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      ok = wait_count(root, epoch * nsub, abort_w);
+      ok = wait_count(root, epoch * nsub, abort_w, limit);
     } else {
       __hip_atomic_fetch_add(sub, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      ok = wait_count(sub, epoch * nsubwg, abort_w);
+      ok = wait_count(sub, epoch * nsubwg, abort_w, limit);
     }
     if (!ok) *bad = 1;
   }
@@ -845,11 +849,13 @@ struct TeamPos {
   Lane n;
   uint32_t *sub, *root, *abort_w;
   uint32_t nsub, nsubwg;
+  int limit;  // polls of a wait
   int* bad;
 };
 
 __device__ __forceinline__ bool next_phase(const TeamPos& P, uint32_t& epoch) {
-  return team_barrier(P.sub, P.nsubwg, P.root, P.nsub, ++epoch, P.abort_w, P.bad);
+  return team_barrier(P.sub, P.nsubwg, P.root, P.nsub, ++epoch, P.abort_w, P.limit,
+                      P.bad);
 }
 
 template <bool REC>
@@ -1181,6 +1187,7 @@ __global__ void __launch_bounds__(TTHREADS) team_march(TeamArgs) {
   P.sub = A->tm.sync + SY_SUB + (team * 8 + P.rank % P.nsub) * 64;
   P.root = A->tm.sync + SY_ROOT + team * 64;
   P.abort_w = A->tm.sync + SY_ABORT;
+  P.limit = A->tm.spin_limit > 0 ? A->tm.spin_limit : SPIN_LIMIT;
   __syncthreads();
 
   const int ndwg = A->tm.ndwg, nfwg = A->tm.nfwg;
@@ -1190,11 +1197,27 @@ __global__ void __launch_bounds__(TTHREADS) team_march(TeamArgs) {
     march_finish<TWO, REC, EM>(A, L, P);
   else
     march_rows<R, KP, TWO, REC, SPLIT, EM>(A, L, P);
-  if (bad) {  // aborted: no silent result
-    for (int i = P.rank * TWAVES + P.wv; i < A->op.nspec; i += size * TWAVES)
-      for (int k = P.c0; k < P.cend; ++k)
-        A->st.x[((int64_t)i * K + k) * WAVE + P.n.id] = __builtin_nan("");
+}
+
+// Behind a march: NaN for the state, the recorded stage vectors and the EM weights
+// of an aborted one.
+__device__ __forceinline__ void fill_nan(double* p, int64_t n) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
+    p[i] = __builtin_nan("");
+}
+__global__ void team_void(TeamArgs a) {
+  if (a.tm.sync[SY_ABORT] == 0) return;
+  const int64_t panel = (int64_t)a.op.K * WAVE, nk = a.op.nspec * panel;
+  fill_nan(a.st.x, nk);
+  if (a.st.rec_x) {
+    fill_nan(a.st.rec_x, a.st.rec_count * nk);
+    fill_nan(a.st.rec_a, a.st.rec_count * nk);
+    fill_nan(a.st.rec_fx, a.st.rec_count * nk);
+    fill_nan(a.st.rec_fa, a.st.rec_count * nk);
   }
+  if (a.tm.em_w)
+    fill_nan(a.tm.em_w + (a.k_begin - a.tm.em_first) * panel, (a.k_end - a.k_begin) * panel);
 }
 
 // ---------------------------------------------------------------------------
@@ -1469,6 +1492,7 @@ __global__ void __launch_bounds__(TTHREADS) adjoint_march(AdjArgs) {
   P.sub = A->tm.sync + SY_SUB + (team * 8 + P.rank % P.nsub) * 64;
   P.root = A->tm.sync + SY_ROOT + team * 64;
   P.abort_w = A->tm.sync + SY_ABORT;
+  P.limit = A->tm.spin_limit > 0 ? A->tm.spin_limit : SPIN_LIMIT;
   const int k_begin = A->k_begin, k_end = A->k_end;
   const int nc = P.cend - P.c0;
   const bool src = A->adj.gsrc0 != nullptr && (A->op.flags & PRH_F_INJECTION) != 0;
@@ -1523,12 +1547,22 @@ __global__ void __launch_bounds__(TTHREADS) adjoint_march(AdjArgs) {
         adjoint_row<TWO>(a, L, T, ar, s2, step, P.c0, k0, P.cend, P.n);
     }
     if (ahead) coef_stage(L, step - 1, cn);
-    if (!next_phase(P, epoch)) break;
+    if (!next_phase(P, epoch)) return;
   }
-  if (bad) {  // aborted: no silent result
-    for (int i = P.rank * TWAVES + P.wv; i < A->op.nspec; i += size * TWAVES)
-      for (int k = P.c0; k < P.cend; ++k)
-        A->adj.lam[((int64_t)i * K + k) * WAVE + P.n.id] = __builtin_nan("");
+}
+
+// Behind it: NaN for lam and the accumulators of an aborted sweep.
+__global__ void adjoint_void(AdjArgs a) {
+  if (a.tm.sync[SY_ABORT] == 0) return;
+  const int64_t panel = (int64_t)a.op.K * WAVE, nk = a.op.nspec * panel;
+  fill_nan(a.adj.lam, nk);
+  if (a.adj.gdot) fill_nan(a.adj.gdot, nk);
+  if (!a.adj.gsrc0 || !(a.op.flags & PRH_F_INJECTION)) return;
+  for (int i = 0; i < a.op.nspec; ++i) {
+    const int s = a.op.src_slot[i];
+    if (s < 0) continue;
+    fill_nan(a.adj.gsrc0 + s * (a.op.nsrc * panel), a.op.nsrc * panel);
+    fill_nan(a.adj.gsrc1 + s * (a.op.nsrc * panel), a.op.nsrc * panel);
   }
 }
 
@@ -1632,8 +1666,9 @@ __global__ void __launch_bounds__(EMW_TILES * WAVE)
   }
 }
 
-int32_t launch_march(const void* fn, const prh_team& tm, size_t lds_rows, void* kernel_args,
-                     hipStream_t s) {
+// fn: the march; behind: the launch that voids an aborted one's results (same arguments)
+int32_t launch_march(const void* fn, const void* behind, const prh_team& tm, size_t lds_rows,
+                     void* kernel_args, hipStream_t s) {
   const size_t lds = 8 * WAVE * lds_rows;
   hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return prh_internal::check(e, "team march: dynamic LDS");
@@ -1655,6 +1690,7 @@ int32_t launch_march(const void* fn, const prh_team& tm, size_t lds_rows, void* 
   if (e == hipSuccess)
     e = hipLaunchCooperativeKernel(fn, dim3((unsigned)(tm.nteam * tm.size)), dim3(TTHREADS), args,
                                    (unsigned)lds, s);
+  if (e == hipSuccess) e = hipLaunchKernel(behind, dim3(256), dim3(256), args, 0, s);
   if (e == hipSuccess) e = hipEventRecord(last, s);
   const int32_t rc = prh_internal::check(e, "team march launch");
   // the device cannot hold the whole grid at once (or not cooperatively)
@@ -1675,7 +1711,8 @@ template <int R, int KP, int KD, bool TWO, bool REC, bool SPLIT, bool EM>
 int32_t launch_team_rec(const prh_operator& op, const prh_schedule& sch, const prh_state& st,
                         const prh_team& tm, int k_begin, int k_end, hipStream_t s) {
   TeamArgs ta{op, sch, st, tm, k_begin, k_end};
-  return launch_march(reinterpret_cast<const void*>(&team_march<R, KP, KD, TWO, REC, SPLIT, EM>), tm,
+  return launch_march(reinterpret_cast<const void*>(&team_march<R, KP, KD, TWO, REC, SPLIT, EM>),
+                      reinterpret_cast<const void*>(&team_void), tm,
                       (size_t)(TCONST + (TWO ? 4 : 2) + 2 * tm.coef_slots + tm.red_slots +
                                tm.lds_slots * (TWO ? 2 : 1)),
                       &ta, s);
@@ -1827,6 +1864,7 @@ extern "C" int32_t prh_team_adjoint(const prh_operator* op, const prh_schedule* 
   const int nf = op->mvals_e ? 2 : 1;
   const void* fn = op->mvals_e ? reinterpret_cast<const void*>(&adjoint_march<true>)
                                : reinterpret_cast<const void*>(&adjoint_march<false>);
-  return launch_march(fn, *tm, (size_t)(TCONST + nf + 2 * tm->coef_slots + tm->lds_slots * nf), &ta,
-                      s);
+  return launch_march(fn, reinterpret_cast<const void*>(&adjoint_void), *tm,
+                      (size_t)(TCONST + nf + 2 * tm->coef_slots + tm->lds_slots * nf),
+                      &ta, s);
 }

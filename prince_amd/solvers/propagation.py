@@ -878,7 +878,7 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
             nteam=tp.nteam, size=tp.size, kp=tp.kp, kd=tp.kd, dgroups=tp.dgroups, ndwg=tp.ndwg,
             nfwg=tp.nfwg, nfin=tp.fin.shape[0], nparts=tp.nparts,
             lds_slots=tp.lds_slots, red_slots=tp.red_slots,
-            pair_rows=int(tp.pair_rows), coef_slots=tp.coef_slots, pad_=0,
+            pair_rows=int(tp.pair_rows), coef_slots=tp.coef_slots, spin_limit=0,
             **{n: t.data_ptr() for n, t in b.items()})
         return {"struct": tm, "bufs": b, "plan": tp, "em_steps": 0}
 
