@@ -1,0 +1,75 @@
+// march_launch.h -- host side of a march: one cooperative launch, in order with the
+// other marches of its device.  Host code only (HIP runtime calls).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <cstdint>
+#include <mutex>
+
+#include "internal.h"
+
+namespace prh_internal {
+
+// Marches of one process on one device run one after the other, whatever streams
+// they are on: each waits for the event of the one before.  Two of them on the
+// chip together could each hold CUs the other's barriers need.
+constexpr int MAX_DEVICES = 64;
+inline std::mutex g_order_mu;
+inline hipEvent_t g_last_march[MAX_DEVICES] = {};
+
+// A march belongs to its stream's device: the event that orders it and the dynamic
+// LDS limit of its kernel are that device's, whichever one the caller has current.
+struct StreamDevice {
+  int id = -1, before = -1;
+  hipError_t error;
+  explicit StreamDevice(hipStream_t s) {
+    error = hipStreamGetDevice(s, &id);
+    if (error == hipSuccess) error = hipGetDevice(&before);
+    if (error == hipSuccess && id != before) error = hipSetDevice(id);
+  }
+  ~StreamDevice() {
+    if (before >= 0 && id != before) (void)hipSetDevice(before);
+  }
+  StreamDevice(const StreamDevice&) = delete;
+  StreamDevice& operator=(const StreamDevice&) = delete;
+};
+
+struct MarchLaunch {
+  const void* reset;   // one workgroup, argument sync: clears the sync words
+  const void* march;   // the cooperative kernel
+  const void* behind;  // voids an aborted march's results (same arguments)
+  unsigned blocks, threads;
+  size_t lds;
+  uint32_t* sync;
+  void* args;
+};
+
+inline int32_t launch_march(const MarchLaunch& m, hipStream_t s) {
+  const StreamDevice dev(s);
+  if (dev.error != hipSuccess) return check(dev.error, "team march: device of the stream");
+  if (dev.id < 0 || dev.id >= MAX_DEVICES) return error("team march: no device in [0, 64)");
+  hipError_t e =
+      hipFuncSetAttribute(m.march, hipFuncAttributeMaxDynamicSharedMemorySize, (int)m.lds);
+  if (e != hipSuccess) return check(e, "team march: dynamic LDS");
+  std::lock_guard<std::mutex> lock(g_order_mu);
+  hipEvent_t& last = g_last_march[dev.id];
+  e = last ? hipStreamWaitEvent(s, last, 0)
+           : hipEventCreateWithFlags(&last, hipEventDisableTiming);
+  if (e != hipSuccess) return check(e, "team march: order");
+  uint32_t* sync = m.sync;
+  void* reset_args[] = {&sync};
+  void* args[] = {m.args};
+  e = hipLaunchKernel(m.reset, dim3(1), dim3(1024), reset_args, 0, s);
+  if (e == hipSuccess)
+    e = hipLaunchCooperativeKernel(m.march, dim3(m.blocks), dim3(m.threads), args,
+                                   (unsigned)m.lds, s);
+  if (e == hipSuccess) e = hipLaunchKernel(m.behind, dim3(256), dim3(256), args, 0, s);
+  if (e == hipSuccess) e = hipEventRecord(last, s);
+  const int32_t rc = check(e, "team march launch");
+  // the device cannot hold the whole grid at once (or not cooperatively)
+  return e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported ? 2 : rc;
+}
+
+}  // namespace prh_internal

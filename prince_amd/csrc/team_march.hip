@@ -51,12 +51,11 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
-#include <mutex>
-#include <string>
 #include <type_traits>
 
 #include "../../include/prince_hip.h"
 #include "internal.h"
+#include "march_launch.h"
 
 namespace {
 
@@ -1566,13 +1565,6 @@ __global__ void adjoint_void(AdjArgs a) {
   }
 }
 
-// Marches of one process on one device run one after the other, whatever streams
-// they are on: each waits for the event of the one before.  Two of them on the
-// chip together could each hold CUs the other's barriers need.
-constexpr int MAX_DEVICES = 64;
-std::mutex g_order_mu;
-hipEvent_t g_last_march[MAX_DEVICES] = {};
-
 // ---------------------------------------------------------------------------
 // Photons of the co-evolved EM cascade over a range of steps.  The nuclei do not
 // see the photons, so the march leaves only the Bethe-Heitler sums of each step
@@ -1669,32 +1661,10 @@ __global__ void __launch_bounds__(EMW_TILES * WAVE)
 // fn: the march; behind: the launch that voids an aborted one's results (same arguments)
 int32_t launch_march(const void* fn, const void* behind, const prh_team& tm, size_t lds_rows,
                      void* kernel_args, hipStream_t s) {
-  const size_t lds = 8 * WAVE * lds_rows;
-  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return prh_internal::check(e, "team march: dynamic LDS");
-  void* args[] = {kernel_args};
-  int dev = -1;
-  e = hipGetDevice(&dev);
-  if (e != hipSuccess || dev < 0 || dev >= MAX_DEVICES)
-    return prh_internal::error("team march: no current device in [0, 64)");
-  std::lock_guard<std::mutex> lock(g_order_mu);
-  hipEvent_t& last = g_last_march[dev];
-  if (!last) {
-    e = hipEventCreateWithFlags(&last, hipEventDisableTiming);
-  } else {
-    e = hipStreamWaitEvent(s, last, 0);
-  }
-  if (e != hipSuccess) return prh_internal::check(e, "team march: order");
-  hipLaunchKernelGGL(team_reset, dim3(1), dim3(1024), 0, s, tm.sync);
-  e = hipGetLastError();
-  if (e == hipSuccess)
-    e = hipLaunchCooperativeKernel(fn, dim3((unsigned)(tm.nteam * tm.size)), dim3(TTHREADS), args,
-                                   (unsigned)lds, s);
-  if (e == hipSuccess) e = hipLaunchKernel(behind, dim3(256), dim3(256), args, 0, s);
-  if (e == hipSuccess) e = hipEventRecord(last, s);
-  const int32_t rc = prh_internal::check(e, "team march launch");
-  // the device cannot hold the whole grid at once (or not cooperatively)
-  return e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported ? 2 : rc;
+  return prh_internal::launch_march(
+      {reinterpret_cast<const void*>(&team_reset), fn, behind, (unsigned)(tm.nteam * tm.size),
+       TTHREADS, 8 * WAVE * lds_rows, tm.sync, kernel_args},
+      s);
 }
 
 // 0, or 2 when the stream is being captured (a cooperative launch cannot be)
