@@ -46,13 +46,37 @@ struct MarchLaunch {
   void* args;
 };
 
+// status: nothing was launched, the stage kernels can run instead
+constexpr int32_t NOT_LAUNCHABLE = 2;
+
+// Whether the device can hold the whole grid at once; asked before the launch, so that
+// stepping aside leaves no runtime error behind for the next call to report.
+inline hipError_t march_fits(const MarchLaunch& m, int dev, bool& fits) {
+  int coop = 0, lds = 0, cus = 0, per_cu = 0;
+  fits = false;
+  hipError_t e = hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev);
+  if (e == hipSuccess)
+    e = hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  if (e != hipSuccess || !coop || m.lds > (size_t)lds) return e;
+  e = hipFuncSetAttribute(m.march, hipFuncAttributeMaxDynamicSharedMemorySize, (int)m.lds);
+  if (e == hipSuccess)
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, m.march, (int)m.threads, m.lds);
+  fits = e == hipSuccess && (int64_t)per_cu * cus >= m.blocks;
+  return e;
+}
+
 inline int32_t launch_march(const MarchLaunch& m, hipStream_t s) {
   const StreamDevice dev(s);
   if (dev.error != hipSuccess) return check(dev.error, "team march: device of the stream");
   if (dev.id < 0 || dev.id >= MAX_DEVICES) return error("team march: no device in [0, 64)");
-  hipError_t e =
-      hipFuncSetAttribute(m.march, hipFuncAttributeMaxDynamicSharedMemorySize, (int)m.lds);
-  if (e != hipSuccess) return check(e, "team march: dynamic LDS");
+  bool fits;
+  hipError_t e = march_fits(m, dev.id, fits);
+  if (e != hipSuccess) return check(e, "team march: what the device holds");
+  if (!fits) {
+    error("team march: the device cannot hold the grid");
+    return NOT_LAUNCHABLE;
+  }
   std::lock_guard<std::mutex> lock(g_order_mu);
   hipEvent_t& last = g_last_march[dev.id];
   e = last ? hipStreamWaitEvent(s, last, 0)
@@ -68,8 +92,9 @@ inline int32_t launch_march(const MarchLaunch& m, hipStream_t s) {
   if (e == hipSuccess) e = hipLaunchKernel(m.behind, dim3(256), dim3(256), args, 0, s);
   if (e == hipSuccess) e = hipEventRecord(last, s);
   const int32_t rc = check(e, "team march launch");
-  // the device cannot hold the whole grid at once (or not cooperatively)
-  return e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported ? 2 : rc;
+  if (e != hipErrorCooperativeLaunchTooLarge && e != hipErrorNotSupported) return rc;
+  (void)hipGetLastError();  // refused after all: no error is left for the stage kernels' checks
+  return NOT_LAUNCHABLE;
 }
 
 }  // namespace prh_internal

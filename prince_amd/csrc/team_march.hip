@@ -1667,14 +1667,14 @@ int32_t launch_march(const void* fn, const void* behind, const prh_team& tm, siz
       s);
 }
 
-// 0, or 2 when the stream is being captured (a cooperative launch cannot be)
+// 0, or NOT_LAUNCHABLE when the stream is being captured (a cooperative launch cannot be)
 int32_t refuse_capture(hipStream_t s) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (int32_t e = prh_internal::check(hipStreamIsCapturing(s, &cs), "team march: capture status"))
     return e;
   if (cs == hipStreamCaptureStatusNone) return 0;
   prh_internal::error("team march: a cooperative launch cannot be captured");
-  return 2;
+  return prh_internal::NOT_LAUNCHABLE;
 }
 
 template <int R, int KP, int KD, bool TWO, bool REC, bool SPLIT, bool EM>

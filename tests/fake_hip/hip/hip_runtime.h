@@ -29,13 +29,19 @@ struct dim3 {
   dim3(unsigned a = 1, unsigned b = 1, unsigned c = 1) : x(a), y(b), z(c) {}
 };
 enum { hipFuncAttributeMaxDynamicSharedMemorySize = 8, hipEventDisableTiming = 2 };
+enum hipDeviceAttribute_t {
+  hipDeviceAttributeCooperativeLaunch,
+  hipDeviceAttributeMaxSharedMemoryPerBlock,
+  hipDeviceAttributeMultiprocessorCount
+};
 
 namespace fake {
 inline int current = 0;
 inline hipError_t last = hipSuccess;  // the latest error, until it is read
 inline std::string log;
 inline std::map<std::pair<int, const void*>, int> lds;  // limit set per device and kernel
-inline unsigned max_blocks = 256;
+inline unsigned max_blocks = 256;  // a cooperative launch may have
+inline int lds_max = 163840, per_cu = 1, coop = 1;  // what the device says of itself
 inline int device_of(hipStream_t s) { return s ? s->device : current; }
 inline hipError_t ret(hipError_t e) {
   if (e != hipSuccess) last = e;
@@ -64,7 +70,18 @@ inline hipError_t hipGetLastError() {
   fake::last = hipSuccess;
   return e;
 }
+inline hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t a, int) {
+  *v = a == hipDeviceAttributeCooperativeLaunch         ? fake::coop
+       : a == hipDeviceAttributeMaxSharedMemoryPerBlock ? fake::lds_max
+                                                        : 256;
+  return hipSuccess;
+}
+inline hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t) {
+  *n = fake::per_cu;
+  return hipSuccess;
+}
 inline hipError_t hipFuncSetAttribute(const void* fn, int, int bytes) {
+  if (bytes > fake::lds_max) return fake::ret(hipErrorInvalidValue);
   fake::lds[{fake::current, fn}] = bytes;
   return hipSuccess;
 }

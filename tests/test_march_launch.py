@@ -1,6 +1,6 @@
 """Host side of a march (``csrc/march_launch.h``) compiled against a model of the HIP
-runtime with two devices (``fake_hip/``): the device a march belongs to and the
-order of marches."""
+runtime with two devices (``fake_hip/``): the device a march belongs to, the order of
+marches, and the status when the device cannot hold one."""
 
 import ctypes
 import os
@@ -29,6 +29,12 @@ extern "C" int launch(int stream, unsigned blocks, unsigned lds) {
 extern "C" void set_current(int d) { fake::current = d; }
 extern "C" int current() { return fake::current; }
 extern "C" int pending() { return fake::last; }
+extern "C" void device(unsigned max_blocks, int lds_max, int per_cu, int coop) {
+  fake::max_blocks = max_blocks;
+  fake::lds_max = lds_max;
+  fake::per_cu = per_cu;
+  fake::coop = coop;
+}
 extern "C" const char* calls() {
   static std::string s;
   s = fake::log;
@@ -74,3 +80,19 @@ def test_marches_of_one_device_follow_each_other(lib):
     got = [c for c in lib.calls().decode().split() if not c.startswith("kernel")]
     assert got == ["march0", "record0", "march1", "record1", "wait0", "march0", "record0",
                    "wait1", "march1", "record1"]
+
+
+@pytest.mark.parametrize("blocks,device", [
+    (257, (256, 163840, 1, 1)),   # more workgroups than the chip holds
+    (256, (256, 163840, 0, 1)),   # none fits a CU
+    (256, (256, 65536, 1, 1)),    # less LDS
+    (256, (256, 163840, 1, 0)),   # no cooperative launches
+    (256, (128, 163840, 1, 1)),   # refused by the launch itself
+])
+def test_a_march_that_does_not_fit_steps_aside_without_an_error(lib, blocks, device):
+    lib.device(*device)
+    assert lib.launch(0, blocks, LDS) == 2
+    assert lib.pending() == 0
+    assert "march" not in lib.calls().decode()
+    lib.device(256, 163840, 1, 1)
+    assert lib.launch(0, 256, LDS) == 0
