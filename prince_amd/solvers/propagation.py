@@ -402,12 +402,26 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
                 return kt
         return 1
 
-    def team_march_for(self, K):
-        """Whether the march may run as one cooperative launch (``prh_team_march``):
-        unless a stage configuration was forced or tuned for K."""
+    #: settings of the forward and of the transposed stage kernels: one of them forced
+    #: or tuned for K means that those kernels are wanted
+    STAGE_KEYS = ("kt", "part_cost", "wg_waves", "dense", "dense_chunk", "dense_chunk_cost",
+                  "dense_place", "pairs")
+    ADJOINT_STAGE_KEYS = ("kt_adjoint", "part_cost_adjoint")
+
+    def _march_wanted(self, K, stage_keys):
         tuned = getattr(self, "_tuned", {})
         on = tuned.get(("team", K))
-        return bool(on) if on is not None else not any(key[1] == K for key in tuned)
+        return bool(on) if on is not None else not any((key, K) in tuned for key in stage_keys)
+
+    def team_march_for(self, K):
+        """Whether the march may run as one cooperative launch (``prh_team_march``):
+        unless a forward stage configuration was forced or tuned for K."""
+        return self._march_wanted(K, self.STAGE_KEYS)
+
+    def adjoint_march_for(self, K):
+        """The same for the adjoint sweep (``prh_team_adjoint``) and the transposed
+        stages' settings; the forward ones were never timed against it."""
+        return self._march_wanted(K, self.ADJOINT_STAGE_KEYS)
 
     def __init__(self, *args, **kwargs):
         super().__init__(*args, **kwargs)
@@ -834,8 +848,8 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
         self._plan["team"] = None
         if self.team_march_for(K):
             self._plan["team"] = self._team_setup(lay, dv, K, 2 if two else 1, J, self._plan)
-            if with_adjoint:
-                self._plan["team_adjoint"] = self._adjoint_team_setup(lay, dv, K, 2 if two else 1, J)
+        if with_adjoint and self.adjoint_march_for(K):
+            self._plan["team_adjoint"] = self._adjoint_team_setup(lay, dv, K, 2 if two else 1, J)
         if self._plan["team"] is None:
             self._capture_steps(self._plan)
         self.refresh_zs = zs
