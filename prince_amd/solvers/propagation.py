@@ -910,14 +910,13 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
         operator or the device does not fit it."""
         torch = _torch()
         wl = lay["layout"]
-        args = getattr(self, "_tuned", {}).get(("team_args", K), {})
         em = plan["em"]
         if em is not None and (em.d_em % 8 or not 8 <= em.d_em <= _lib.EM_MAX):
             return None
         team = self._team_tables(
-            lay, (K, fields, nsrc, em is not None, tuple(sorted(args.items()))), K, dv,
+            lay, (K, fields, nsrc, em is not None), K, dv,
             lambda: team_plan.build_team(wl.blocks, wl.fwd.brow_ptr, wl.nspec, wl.d, wl.diag_off, K,
-                                         fields, nsrc, em is not None, **args))
+                                         fields, nsrc, em is not None))
         if team is None:
             return None
         tm, b = team["struct"], team["bufs"]

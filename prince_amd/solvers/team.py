@@ -103,8 +103,7 @@ def tail_rows(blocks, ptr, nspec):
     return dense, sorted(tail)
 
 
-def build_team(blocks, brow_ptr, nspec, d, diag_off, K, fields=1, nsrc=1, em=False, size=None,
-               ndwg=None, nfwg=None):
+def build_team(blocks, brow_ptr, nspec, d, diag_off, K, fields=1, nsrc=1, em=False, size=None):
     """Team plan of an operator for K right-hand sides, or None when its rows do
     not fit the march (d != 64, more than two dense rows, bands left of the
     diagonal or wider than 8, a long tail, values beyond the LDS, more source
@@ -129,13 +128,13 @@ def build_team(blocks, brow_ptr, nspec, d, diag_off, K, fields=1, nsrc=1, em=Fal
             return None
     sizes = [1] if len(tail) == nspec else [size] if size is not None else [32, 64, 128, 256]
     for s in sizes:
-        plan = _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, em, s, ndwg, nfwg)
+        plan = _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, em, s)
         if plan is not None:
             return plan
     return None
 
 
-def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, em, size, ndwg, nfwg):
+def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, em, size):
     nteam = min(8, CUS // size)
     nc = -(-K // nteam)
     kd, dgroups = dense_tiling(nc)
@@ -160,9 +159,8 @@ def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, em, size,
     nsum = DENSE_MAX + int(em)
     red = WAVES * nsum * 2 if (mothers and dgroups > 1) else 0
     budget = (LDS_BYTES // 512 - CONST_SLOTS - 2 * fields - 2 * coef - red) // fields
-    if not mothers:
-        ndwg = 0
-    elif ndwg is None:
+    ndwg = 0
+    if mothers:
         # the least number of workgroups whose LDS holds the dense values
         ndwg = max(1, -(-int(eslots.sum()) // max(1, budget)))
         while ndwg < size and max(eslots[a:b].sum() for a, b in zip(*_bounds(eslots, ndwg))) > budget:
@@ -170,7 +168,7 @@ def _build(blocks, ptr, nspec, dense, tail, diag_off, K, fields, nsrc, em, size,
     heavy = [da for da in range(nspec) if da not in tset]
     # tail rows that are not dense sum their heavy mothers among the heavy rows
     light = [da for da in tail if da not in dense]
-    nfwg = 0 if not tail else 1 if size == 1 or nfwg is None and len(tail) * nc <= WAVES else (nfwg or 2)
+    nfwg = 0 if not tail else 1 if size == 1 or len(tail) * nc <= WAVES else 2
     nrow_wg = size - ndwg - nfwg
     if nrow_wg < (1 if heavy else 0):
         return None
