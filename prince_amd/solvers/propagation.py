@@ -408,20 +408,25 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
                   "dense_place", "pairs")
     ADJOINT_STAGE_KEYS = ("kt_adjoint", "part_cost_adjoint")
 
-    def _march_wanted(self, K, stage_keys):
+    def _march_wanted(self, K, stage_keys, pays):
         tuned = getattr(self, "_tuned", {})
         on = tuned.get(("team", K))
-        return bool(on) if on is not None else not any((key, K) in tuned for key in stage_keys)
+        if on is not None:
+            return bool(on)
+        return pays and not any((key, K) in tuned for key in stage_keys)
 
-    def team_march_for(self, K):
+    def team_march_for(self, K, nspec=None, fields=1, gradient=False):
         """Whether the march may run as one cooperative launch (``prh_team_march``):
-        unless a forward stage configuration was forced or tuned for K."""
-        return self._march_wanted(K, self.STAGE_KEYS)
+        unless a forward stage configuration was forced or tuned for K, or (nspec
+        given) the stage kernels are faster for that many rows and columns."""
+        return self._march_wanted(K, self.STAGE_KEYS,
+                                  nspec is None or team_plan.march_pays(nspec, K, fields, gradient))
 
-    def adjoint_march_for(self, K):
+    def adjoint_march_for(self, K, nspec=None, fields=1):
         """The same for the adjoint sweep (``prh_team_adjoint``) and the transposed
         stages' settings; the forward ones were never timed against it."""
-        return self._march_wanted(K, self.ADJOINT_STAGE_KEYS)
+        return self._march_wanted(K, self.ADJOINT_STAGE_KEYS,
+                                  nspec is None or team_plan.adjoint_march_pays(nspec, K, fields))
 
     def __init__(self, *args, **kwargs):
         super().__init__(*args, **kwargs)
@@ -846,10 +851,11 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
             "em": em_struct, "em_bufs": em_bufs,
         }
         self._plan["team"] = None
-        if self.team_march_for(K):
-            self._plan["team"] = self._team_setup(lay, dv, K, 2 if two else 1, J, self._plan)
-        if with_adjoint and self.adjoint_march_for(K):
-            self._plan["team_adjoint"] = self._adjoint_team_setup(lay, dv, K, 2 if two else 1, J)
+        fields = 2 if two else 1
+        if self.team_march_for(K, nspec, fields, with_adjoint):
+            self._plan["team"] = self._team_setup(lay, dv, K, fields, J, self._plan)
+        if with_adjoint and self.adjoint_march_for(K, nspec, fields):
+            self._plan["team_adjoint"] = self._adjoint_team_setup(lay, dv, K, fields, J)
         if self._plan["team"] is None:
             self._capture_steps(self._plan)
         self.refresh_zs = zs

@@ -31,6 +31,65 @@ TAIL_MAX = 32
 SYNC_BYTES = 18688
 
 
+# Right-hand sides up to which a march beats the stage kernels, by species rows: (rows
+# from, K below 256, K from 256 on, where the stage kernels take 8 right-hand sides per
+# wave).  A march has at most 8 teams; few rows leave most of a team's workgroups idle,
+# so its columns queue up where the stage kernels fill the chip.  Stage kernels over
+# march, time per step, at K inside a line | beyond it:
+#   one field   1 row     255 1.22, 448 1.05 | 512 0.94, 4096 0.15
+#               2         192 1.10, 256 - 320 1.21 - 1.04 | 224 0.92, 384 0.92
+#               4 - 41    128 0.99 - 1.33 | 192 0.67 - 1.06, 256 0.74 - 1.04, 512 0.54
+#               53 - 77   128 1.21 - 1.47, 288 1.06 - 1.20 | 160 0.85 - 1.04, 384 0.87 - 1.01
+#               89, 113   384 1.01, 1.11 | 512 0.84
+#               137       448 1.05 | 512 0.95
+#               209       768 1.04 | 896 0.97
+#               257, 305  512 1.32, 1.18 | 640 1.11, 0.93; 1024 1.00, 0.95
+#   two fields  1 row     160 1.01, 512 1.06 | 192 0.98
+#               2 - 41    64 1.16 - 1.40 | 80 0.77 - 0.95, 256 0.86 - 1.00
+#               53 - 77   96 0.99 - 1.11, 256 1.15 - 1.32 | 160 0.73, 384 0.85 - 0.92
+#               89, 113   320 1.10, 1.25 | 384 0.93, 1.06
+#               137, 173  384 1.11, 1.30; 448 1.21 | 512 0.95, 1.15
+#               209       768 1.21
+#               257, 305  384 0.93, 1.04 | 512 0.85, 0.97
+# With the EM cascade as one field (305 rows 512 1.20 | 640 0.99; 7 rows 128 1.24 | 512 0.63).
+MARCH_PAYS = {
+    1: ((1, 255, 448), (2, 192, 320), (3, 128, 0), (48, 128, 288), (85, 255, 384), (120, 255, 448),
+        (200, 255, 768), (250, 255, 512)),
+    2: ((1, 160, 512), (2, 64, 0), (48, 96, 288), (85, 255, 320), (120, 255, 448), (200, 255, 768),
+        (250, 255, 384)),
+}
+# A gradient's forward stages (16 waves, no row pairs) lose to the march for longer: one
+# field, 305 rows, 1024 1.25.
+GRADIENT_ROWS, GRADIENT_K = 200, 2048
+# The adjoint march, by the time of a sweep:
+#   one field   1, 2 rows  512 1.13, 1.00 | 768 0.85;  7 512 1.11;  17 2048 1.03;  53 - 305 1.09 - 1.40
+#   two fields  1 row      128 1.00 | 160 0.95;  2 64 1.12 | 80 0.92;  7 80 1.07 | 128 0.93
+#               17         255 1.04, 448 1.12;  35 128 1.00 | 192 0.88;  53 80 1.14 | 128 0.92
+#               89, 137    128 1.07, 1.06 | 255 0.91, 0.96
+#               209, 305   128 0.98, 1.01 | 192 0.89, 0.96
+ADJOINT_PAYS = {
+    1: ((1, 255, 512), (8, 255, 2048)),
+    2: ((1, 128, 0), (2, 64, 0), (3, 80, 0), (8, 255, 448), (29, 128, 0), (48, 80, 0), (85, 128, 0)),
+}
+
+
+def _within(lines, nspec, K):
+    _, below, above = [ln for ln in lines if ln[0] <= nspec][-1]
+    return K <= (below if K < 256 else above)
+
+
+def march_pays(nspec, K, fields, gradient=False):
+    """Whether the march beats the stage kernels for K right-hand sides."""
+    if gradient and fields == 1 and nspec >= GRADIENT_ROWS:
+        return K <= GRADIENT_K
+    return _within(MARCH_PAYS[fields], nspec, K)
+
+
+def adjoint_march_pays(nspec, K, fields):
+    """The same for the adjoint sweep."""
+    return _within(ADJOINT_PAYS[fields], nspec, K)
+
+
 @dataclass
 class TeamPlan:
     nteam: int
