@@ -876,17 +876,15 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
     def _team_tables(self, lay, key, K, dv, build):
         """A march's tables (kept with the layout) and its own partials and sync words."""
         torch = _torch()
-        plans = lay.setdefault("team", {})
-        if key not in plans:
+        names = ("lds_ptr", "lds_voff", "wave_ptr", "rows", "mothers", "dense_ptr", "dense_ent",
+                 "fin", "fin_blk")
+
+        def make():
             tp = build()
-            names = ("lds_ptr", "lds_voff", "wave_ptr", "rows", "mothers", "dense_ptr",
-                     "dense_ent", "fin", "fin_blk")
-            tables = None if tp is None else {
+            return tp, None if tp is None else {
                 n: dv(np.append(getattr(tp, n).ravel(), 0), np.int32) for n in names}
-            while len(plans) >= self.TEAM_PLANS_KEPT:
-                plans.pop(next(iter(plans)))
-            plans[key] = (tp, tables)
-        tp, tables = plans[key]
+
+        tp, tables = team_plan.kept(lay, key, make, self.TEAM_PLANS_KEPT)
         props = torch.cuda.get_device_properties(self.device)
         if tp is None or props.multi_processor_count < tp.nteam * tp.size:
             return None

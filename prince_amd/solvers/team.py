@@ -15,6 +15,7 @@ workgroups finish the tail rows.  Pure numpy.
 
 from __future__ import annotations
 
+import threading
 from dataclasses import dataclass
 
 import numpy as np
@@ -88,6 +89,24 @@ def march_pays(nspec, K, fields, gradient=False):
 def adjoint_march_pays(nspec, K, fields):
     """The same for the adjoint sweep."""
     return _within(ADJOINT_PAYS[fields], nspec, K)
+
+
+_KEPT_LOCK = threading.Lock()
+
+
+def kept(lay, key, make, most):
+    """``make()`` of a key, kept with the layout ``lay``; at most ``most`` of them, the
+    oldest goes first.  Solvers of several threads share a layout."""
+    with _KEPT_LOCK:
+        value = lay.setdefault("team", {}).get(key)
+    if value is None:
+        value = make()
+        with _KEPT_LOCK:
+            plans = lay["team"]
+            value = plans.setdefault(key, value)
+            while len(plans) > most:
+                plans.pop(next(k for k in plans if k != key))
+    return value
 
 
 @dataclass

@@ -182,3 +182,33 @@ def test_adjoint_plan_reproduces_the_transposed_operator(layouts, name, K, field
         pairs = sorted(q for cg, ncg, _ in got[r] for q in range(cg, -(-nc // 2), ncg))
         assert pairs == list(range(-(-nc // 2)))
         assert np.allclose(got[r][0][2], want[r], rtol=1e-12, atol=1e-12 * np.abs(want).max())
+
+
+def test_kept_plans_are_shared_by_threads():
+    """Threads that prepare solves on one run at once: each gets the plan of its own
+    size while the others' displace it."""
+    import sys
+    import threading
+
+    lay, wrong = {}, []
+
+    def work(seed):
+        rng = np.random.default_rng(seed)
+        try:
+            for k in rng.integers(0, 12, size=4000).tolist():
+                if team.kept(lay, k, lambda: ("plan", k), 3) != ("plan", k):
+                    wrong.append(k)
+        except Exception as e:  # noqa: BLE001
+            wrong.append(repr(e))
+
+    old = sys.getswitchinterval()
+    sys.setswitchinterval(1e-6)
+    try:
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(8)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        sys.setswitchinterval(old)
+    assert not wrong and 0 < len(lay["team"]) <= 3
