@@ -888,6 +888,11 @@ class ETD2SolverHIP(UHECRPropagationSolverETD2):
         props = torch.cuda.get_device_properties(self.device)
         if tp is None or props.multi_processor_count < tp.nteam * tp.size:
             return None
+        # the tables may have been made on another stream, whose allocations must not
+        # take their memory over while this plan's stream still reads it
+        stream = torch.cuda.current_stream(self.device)
+        for t in tables.values():
+            t.record_stream(stream)
         b = dict(tables)
         b["sync"] = torch.zeros(team_plan.SYNC_BYTES // 4, dtype=torch.int32, device=self.device)
         b["dpart"] = torch.empty((2, max(1, tp.nparts), K, 64), dtype=torch.float64,

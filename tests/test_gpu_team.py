@@ -206,3 +206,40 @@ def test_adjoint_march_equals_the_transposed_stages(K, two):
         d = _norm_dev(out[0][k], out[1][k])
         print(f"K={K} {k}: {d:.2e}")
         assert d <= TOL, k
+
+
+def test_displaced_tables_outlive_their_use_on_another_stream():
+    """Two plans on two streams share a layout's tables.  Displaced and dropped while
+    the second stream still marches, their memory is not given to new tensors of the
+    stream that made them."""
+    import torch
+
+    run = workloads.nuclear_run()
+    K = 65  # no other test's plan
+    g = _solver(run, 2.0, K, 11, True)
+    p = g.prepare(1e-3)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        g2 = _solver(run, 2.0, K, 11, True)
+        p2 = g2.prepare(1e-3)
+    shared = ("rows", "mothers", "lds_voff", "dense_ent")
+    ptrs = {n: p2["team"]["bufs"][n].data_ptr() for n in shared}
+    sizes = {n: p2["team"]["bufs"][n].numel() for n in shared}
+    assert all(p["team"]["bufs"][n].data_ptr() == q for n, q in ptrs.items())
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        want = g2.execute(p2).clone()
+        torch.cuda.synchronize()
+        x = g2.execute(p2)  # about 70 ms on the side stream
+    for lay in g._device_cache().layouts.values():
+        for key in [k for k in lay.get("team", {}) if k[0] == K]:
+            del lay["team"][key]
+    g.close()
+    g2.close()
+    del p, p2
+    new = [torch.empty(n, dtype=torch.int32, device=x.device) for n in sizes.values() for _ in range(8)]
+    assert not side.query(), "the march ended too early for this test"
+    assert not {t.data_ptr() for t in new} & set(ptrs.values())
+    torch.cuda.synchronize()
+    assert torch.equal(x, want)
