@@ -58,7 +58,8 @@ typedef struct prh_operator {
   int64_t diag_off;     /* offset of the diagonal inside a window */
   const double* mvals;
   const double* egrid;  /* [d] bin-centre energies (adiabatic loss) */
-  const double* dcoef;  /* [d][7] FD coefficients for offsets -3..3 */
+  const double* dcoef;  /* [d][7] FD coefficients for offsets -3..3; not used where the
+                           neighbour lies outside the grid */
   const double* ddiag;  /* [d] FD diagonal */
   const double* pscale; /* [nspec] pair-production scale per species */
   const double* rpair;  /* [nwin][d] pair-production rate per window */

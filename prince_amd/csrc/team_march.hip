@@ -1173,8 +1173,10 @@ __global__ void __launch_bounds__(TTHREADS) team_march(TeamArgs) {
   L.val = L.coef + 2 * L.coefs;
   L.slots = cload(A->tm.lds_ptr + P.rank + 1) - cload(A->tm.lds_ptr + P.rank);
   for (int i = threadIdx.x; i < WAVE; i += TTHREADS) {
-    for (int o = 0; o < 7; ++o)
-      L.cst[o * WAVE + i] = (A->op.flags & PRH_F_PARTIAL_DIFF) ? A->op.dcoef[i * 7 + o] : 0.0;
+    for (int o = 0; o < 7; ++o)  // zero where the neighbour lies outside the grid (team_epilogue)
+      L.cst[o * WAVE + i] = (A->op.flags & PRH_F_PARTIAL_DIFF) && (unsigned)(i + o - 3) < WAVE
+                                ? A->op.dcoef[i * 7 + o]
+                                : 0.0;
     L.cst[7 * WAVE + i] = A->op.egrid[i];
     L.cst[8 * WAVE + i] = A->op.ddiag[i];
   }
@@ -1479,8 +1481,10 @@ __global__ void __launch_bounds__(TTHREADS) adjoint_march(AdjArgs) {
   L.val = L.coef + 2 * L.coefs;
   L.slots = cload(A->tm.lds_ptr + P.rank + 1) - cload(A->tm.lds_ptr + P.rank);
   for (int i = threadIdx.x; i < WAVE; i += TTHREADS) {
-    for (int o = 0; o < 7; ++o)
-      L.cst[o * WAVE + i] = (A->op.flags & PRH_F_PARTIAL_DIFF) ? A->op.dcoef[i * 7 + o] : 0.0;
+    for (int o = 0; o < 7; ++o)  // zero where the neighbour lies outside the grid (team_epilogue)
+      L.cst[o * WAVE + i] = (A->op.flags & PRH_F_PARTIAL_DIFF) && (unsigned)(i + o - 3) < WAVE
+                                ? A->op.dcoef[i * 7 + o]
+                                : 0.0;
     L.cst[7 * WAVE + i] = A->op.egrid[i];
     L.cst[8 * WAVE + i] = A->op.ddiag[i];
   }

@@ -243,3 +243,20 @@ def test_displaced_tables_outlive_their_use_on_another_stream():
     assert not {t.data_ptr() for t in new} & set(ptrs.values())
     torch.cuda.synchronize()
     assert torch.equal(x, want)
+
+
+@pytest.mark.parametrize("K", [1, 2, 40])
+def test_stencil_coefficients_outside_the_grid_are_not_used(K):
+    """An operator whose table holds numbers there: as the stage kernels, the march
+    gives what it gives for zeros."""
+    import torch
+
+    g = _solver(workloads.nuclear_run(), 0.02, K, 12, True)
+    p = g.prepare(1e-3)
+    want = g.execute(p).clone()
+    t = p["bufs"]["dcoef"].view(64, 7)
+    bins = torch.arange(64, device=t.device)[:, None] + torch.arange(-3, 4, device=t.device)[None, :]
+    outside = (bins < 0) | (bins > 63)
+    assert int(outside.sum()) == 12 and not bool(t[outside].any())
+    t[outside] = 3.0
+    assert torch.equal(g.execute(p), want)
