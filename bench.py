@@ -67,6 +67,8 @@ def parse():
                    help="initial redshift (3.0 is the benchmark; smaller values shorten profiler runs)")
     p.add_argument("--traffic", default=os.path.join(ROOT, "profiles", "etd2_stage_K512_traffic.json"),
                    help="rocprofv3 FETCH_SIZE / WRITE_SIZE summary of the stage kernels (JSON)")
+    p.add_argument("--march-traffic", default=os.path.join(ROOT, "profiles", "team_march_traffic.json"),
+                   help="the same of the march")
     return p.parse_args()
 
 
@@ -91,6 +93,36 @@ def measured_traffic(path, stage_groups):
                              + v["WRITE_SIZE_KiB"] / rec["write_factor"])
         per.append(tot)
     return float(np.mean(per))
+
+
+def march_traffic(path, kp, kd):
+    """HBM bytes per stage of the one-field march, from its own counter summary
+    (as ``measured_traffic``; a dispatch covers ``stages_per_dispatch`` stages)."""
+    name = f"team_march<2, {kp}, {kd}, false, false, false, false>"
+    if not os.path.exists(path):
+        return None
+    with open(path) as f:
+        rec = json.load(f)
+    ks = [v for k, v in rec["kernels"].items() if name in k]
+    if len(ks) != 1:
+        return None
+    v = ks[0]
+    return 1024.0 / rec["stages_per_dispatch"] * (v["FETCH_SIZE_KiB"] / rec["fetch_factor"]
+                                                  + v["WRITE_SIZE_KiB"] / rec["write_factor"])
+
+
+def march_stage_time(solver, plan, torch):
+    """Seconds per stage of the march (one launch over the whole solve), HIP events;
+    the second of two."""
+    solver.execute(plan)
+    plan["x"].zero_()
+    solver.fold_windows(plan)
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    ev[0].record()
+    solver._launch_steps(plan, 0, plan["nsteps"])
+    ev[1].record()
+    torch.cuda.synchronize()
+    return ev[0].elapsed_time(ev[1]) * 1e-3 / (2 * plan["nsteps"])
 
 
 def timed(fn, torch, reps):
@@ -637,6 +669,27 @@ def main():
             "implementation_bytes_per_launch": own,
             "implementation_frac": round(own / avg / 1e9 / HBM_PEAK_GBS, 4),
         }
+        if bplan["team"] is not None:
+            # the timed solves ran the march: the roofline is its launch over 2 nsteps
+            # stages, the stage kernels' stands beside it
+            tm = march_stage_time(multi, bplan, torch)
+            mp = bplan["team"]["plan"]
+            traffic = march_traffic(args.march_traffic, mp.kp, mp.kd)
+            march = {
+                "bound": "hbm",
+                "achieved": round(nbytes / tm / 1e9, 1),
+                "peak": HBM_PEAK_GBS,
+                "unit": "GB/s",
+                "frac": round(nbytes / tm / 1e9 / HBM_PEAK_GBS, 4),
+                "traffic": None if traffic is None else traffic * 2 * nsteps,
+                "kernel": "team_march (one launch per solve, batched K=%d)" % K,
+                "bytes_per_launch": nbytes * 2 * nsteps,
+                "avg_launch_us": round(tm * 2e6 * nsteps, 2),
+                "us_per_stage": round(tm * 1e6, 2),
+                "stage_kernels": roof,
+            }
+            roof = march
+            kernels["team_march_stage_us"] = round(tm * 1e6, 2)
         kernels["etd2_stage1_us"] = round(t1s * 1e6, 2)
         kernels["etd2_stage2_us"] = round(t2s * 1e6, 2)
         # fold GEMM (MFMA) timing
