@@ -2283,7 +2283,8 @@ constexpr int CPREP = 256;            // threads of the preparing kernels
 constexpr int CPIT = 17;              // LDS pitch of a 16-column tile column
 constexpr int64_t CMAT = (int64_t)CNP * CNP;
 // per-window workspace; P .. Mic are stored transposed (k-major): an operand
-// fragment (16 rows x 4 k) is four 128-byte row segments
+// fragment (16 rows x 4 k) is four 128-byte row segments.  CM_SPARE is not used: the
+// workspace of 9 matrices a window is part of the interface
 enum CascadeMat { CM_P = 0, CM_SG, CM_DE, CM_MIC, CM_G, CM_E, CM_INFO, CM_ESC, CM_SPARE, CM_COUNT };
 // doubles of the CM_INFO matrix: cold flags, then per column block the
 // iterations done, converged or not, and triangular and finite or not

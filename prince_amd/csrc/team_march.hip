@@ -16,8 +16,14 @@
 // one XCD) to 2.6 us (256).  A full agent-scope release / acquire pair instead
 // measured 37 us per stage: it writes back and invalidates the whole L2.
 // Measured per stage of the A <= 56 run, stage kernels -> march: K = 1 11.5 ->
-// 6.3 us, K = 7 20 -> 6.8, K = 64 33 -> 16.5, K = 300 129 -> 45, K = 512 92 -> 75;
-// two fields, K = 48: 48 -> 21.6.
+// 6.3 us, K = 7 20 -> 6.8, K = 64 33 -> 16.5, K = 300 129 -> 45, K = 512 92 -> 79;
+// two fields, K = 48: 48 -> 21.6.  What bounds it, by counters: K = 1 a serial chain
+// (the SIMDs issue 0.6 of 6.2 us, waves wait 70 % of their time: barrier, load
+// latency, one row's instructions); K = 64 the same at 8 us of issue per SIMD, 77 %
+// of the L2 requests hit and 33 MB go past the L2 per stage; K = 512 traffic: a team's
+// state is 10 MB per array against 4 MB of L2, 40 % of the requests miss and 373 MB
+// per stage pass at 4.7 TB/s, the rate of a large copy.  With few rows or beyond
+// those columns the stage kernels are faster (solvers/team.py, march_pays).
 //
 // Teams are workgroups blockIdx % nteam, which the dispatcher places on one
 // XCD (nteam = 8) or on a pair of XCDs (nteam = 4); only speed depends on that
@@ -38,15 +44,17 @@
 // Lanes: a wave holds two right-hand sides, 32 lanes each, two energy bins per
 // lane, so every state and value access is 16 bytes per lane.  8-byte loads of
 // the same panels stop at 18.8 TB/s over the chip (half of a CU's load path),
-// 16-byte ones reach 32 TB/s, with or without sc1; a shift by one bin also
-// moves half as many registers.
+// 16-byte ones reach 28 - 32 TB/s with sc1 and 31 - 36 without, where the panels
+// fit an L2; a shift by one bin also moves half as many registers.
 //
 // Every wait is bounded: a workgroup that polls SPIN_LIMIT times (prh_team.spin_limit)
 // without progress raises the abort word and leaves, and the others do when they
 // next wait.  Which of them still stored results is then a matter of timing, so a
 // launch behind the march reads the word and, where it is raised, fills with NaN
 // everything that march writes for its caller: no result of an aborted march, nor
-// of what follows from it, is finite.
+// of what follows from it, is finite.  Within a process marches of one device run one
+// after the other (march_launch.h).  Those of two processes on one card meet only in
+// the driver's scheduling of cooperative launches, which was not measured.
 
 #include <hip/hip_runtime.h>
 
@@ -453,7 +461,10 @@ __device__ __forceinline__ void couple_run(const TeamState& T, const TeamLds& L,
 }
 
 // One stage of a row task for the KP pairs of right-hand sides from k0.  Pairs
-// past kend read other panels (or zeros past the array) and are not stored.
+// past kend read other panels, or zeros past the array, and are not stored: on gfx950
+// the range check of a buffer load takes the scalar offset in, also one beyond the
+// range (checked with a descriptor shorter than its allocation).  Clamping the
+// columns instead cost 3.7 % at K = 64.
 template <int KP, bool TWO, bool REC>
 __device__ __forceinline__ void team_rows(COp& op, CSch& sch,
                                           CSt& st, const TeamState& T,
