@@ -205,8 +205,8 @@ struct TeamState {
 // the step's work, so that no stage waits for memory it never touched before (about
 // 2 us; 5 us per stage on the rows with sources at K = 64).
 __device__ __forceinline__ double coef_ahead(COp& op, CSch& sch, int step, int c0, int nc) {
-  if (!(op.flags & PRH_F_INJECTION)) return 0.0;  // uniform
   const int J = op.nsrc;
+  if (!(op.flags & PRH_F_INJECTION) || J < 1) return 0.0;  // uniform
   const int i = (int)threadIdx.x < J * nc ? threadIdx.x : J * nc - 1;
   const int j = i / nc;
   return sch.src_coef[((int64_t)step * J + j) * op.K + c0 + (i - j * nc)];

@@ -260,3 +260,25 @@ def test_stencil_coefficients_outside_the_grid_are_not_used(K):
     assert int(outside.sum()) == 12 and not bool(t[outside].any())
     t[outside] = 3.0
     assert torch.equal(g.execute(p), want)
+
+
+@pytest.mark.parametrize("K", [1, 9, 40])
+def test_injection_without_sources_adds_nothing(K):
+    """The flag set and no sources (nsrc 0): no coefficient is read, and the steps are
+    those without the flag, as in the stage kernels."""
+    import torch
+
+    from prince_amd import _lib
+
+    g = _solver(workloads.nuclear_run(), 0.02, K, 13, True)
+    p = g.prepare(1e-3)
+    x0 = torch.rand(tuple(p["x"].shape), dtype=torch.float64,
+                    generator=torch.Generator().manual_seed(1)).to(p["x"].device)
+    g.fold_windows(p)
+    out = []
+    for nsrc, flags in ((0, p["op"].flags), (p["op"].nsrc, p["op"].flags & ~_lib.PRH_F_INJECTION)):
+        p["op"].nsrc, p["op"].flags = nsrc, flags
+        p["x"].copy_(x0)
+        g._launch_steps(p, 0, p["nsteps"])
+        out.append(p["x"].clone())
+    assert torch.equal(*out) and not torch.equal(out[0], x0)
